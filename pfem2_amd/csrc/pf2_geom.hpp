@@ -284,6 +284,116 @@ PF2_HD bool inverse_quadratic(const double (*P)[2], const double* p, double* out
     return false;
 }
 
+// ---------------------------------------------------------------------------
+// Quotients and square roots without range scaling (device).  The compiler's
+// FP64 division refines v_rcp_f64 by two Newton steps, forms n y and corrects
+// it by the remainder, between steps that scale operands of extreme
+// exponents and fix up special values; its square root does the same with
+// v_rsq_f64.  Operands in the middle of the exponent range pass the scaling
+// and the fix-up unchanged, so the steps below give the same bits there, and
+// quotients of one divisor share its reciprocal.  Callers check the range.
+__device__ __forceinline__ double rcp_refined(double d) {
+    double y = __builtin_amdgcn_rcp(d);
+    y = fma(y, fma(-d, y, 1.0), y);
+    return fma(y, fma(-d, y, 1.0), y);
+}
+
+__device__ __forceinline__ double div_refined(double n, double d, double y) {
+    const double q = n * y;
+    return fma(fma(-d, q, n), y, q);
+}
+
+__device__ __forceinline__ double sqrt_refined(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = y * 0.5;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, x), h, g);
+    return fma(fma(-g, g, x), h, g);
+}
+
+// What inverse_quadratic computes from a cell's vertices alone, kept across
+// the points of one cell: the leading coefficient, its double and the
+// refined reciprocal of that, the bounds of the divisors of xi_0.  A
+// cell out of the middle exponent range gets NaN for the reciprocal or
+// infinite bounds, so that closed_form answers 2 for it.
+struct QuadCell {
+    double a, a2, ya, tx, ty;
+    __device__ __forceinline__ void init(const double (*P)[2]) {
+        const double x0 = P[0][0], x1 = P[1][0], x2 = P[2][0], x3 = P[3][0];
+        const double y0 = P[0][1], y1 = P[1][1], y2 = P[2][1], y3 = P[3][1];
+        a = (x1 - x3) * (y0 - y2) - (x0 - x2) * (y1 - y3);
+        a2 = 2 * a;
+        ya = fabs(a2) > 0x1p-300 && fabs(a2) < 0x1p300 ? rcp_refined(a2) : __builtin_nan("");
+        const double mx = dmax(dmax(fabs(x0), fabs(x1)), dmax(fabs(x2), fabs(x3)));
+        const double my = dmax(dmax(fabs(y0), fabs(y1)), dmax(fabs(y2), fabs(y3)));
+        const bool mid = mx > 0x1p-300 && mx < 0x1p300 && my > 0x1p-300 && my < 0x1p300;
+        tx = mid ? 1e-10 * mx : __builtin_inf();
+        ty = mid ? 1e-10 * my : __builtin_inf();
+    }
+};
+
+// inverse_map<2>'s closed form at p.  0: the point lies in the unit square,
+// out holds inverse_quadratic's bits; 1: within 1e-15 of the square but not
+// in it (inverse_map accepts it, the unit-cell test does not); 2: anything
+// else (outside, a degenerate quadratic, or operands out of the middle
+// exponent range), where the caller runs inverse_map or a test that implies
+// its answer.  Straight-line but for the choice of the root's quotient: a
+// value out of range or NaN fails a comparison at the end.  About 105 instead
+// of 150 instructions per point (one reciprocal per cell for the two roots,
+// no scaling steps): k_move, bound by them, 134 -> 118 us per step on 101,785
+// cells with 2.4M particles, 759 -> 670 us on 407,140 with 11M; early exits
+// instead of the straight line took most of that back (707 us).
+__device__ __forceinline__ int closed_form(const double (*P)[2], const QuadCell& q, const double* p, double* out) {
+    const double x = p[0], y = p[1];
+    const double x0 = P[0][0], x1 = P[1][0], x2 = P[2][0], x3 = P[3][0];
+    const double y0 = P[0][1], y1 = P[1][1], y2 = P[2][1], y3 = P[3][1];
+    const double b = -(x0 - x1 - x2 + x3) * y + (x - 2 * x1 + x3) * y0 - (x - 2 * x0 + x2) * y1
+                     - (x - x1) * y2 + (x - x0) * y3;
+    const double c = (x0 - x1) * y - (x - x1) * y0 + (x - x0) * y1;
+    const double disc = b * b - 4 * q.a * c;
+    bool ok = (disc > 0x1p-600) & (disc < 0x1p600);
+    const double sq = sqrt_refined(disc);
+    double eta;
+    if (fabs(b) == sq) {   // (b != 0: sq is positive)
+        eta = div_refined(-c, b, rcp_refined(b));
+        ok = ok & (fabs(c) > 0x1p-600) & (fabs(c) < 0x1p600);
+    } else {
+        // neither -b - sq nor -b + sq is zero here, and one below 2^-360
+        // would need |b| and sq to agree beyond their 53 bits
+        const double bm = -b - sq, bp = -b + sq;
+        double eta1, eta2;
+        if (fabs(q.a) < 1e-8 * fabs(b)) {
+            eta1 = div_refined(2 * c, bm, rcp_refined(bm));
+            eta2 = div_refined(2 * c, bp, rcp_refined(bp));
+            ok = ok & (fabs(b) < 0x1p400) & (fabs(c) > 0x1p-500) & (fabs(c) < 0x1p400);
+        } else {
+            eta1 = div_refined(bm, q.a2, q.ya);
+            eta2 = div_refined(bp, q.a2, q.ya);
+        }
+        eta = (fabs(eta1 - 0.5) < fabs(eta2 - 0.5)) ? eta1 : eta2;
+    }
+    const double sub0 = -eta * x2 + x0 * (eta - 1);
+    double den = eta * x3 - x1 * (eta - 1) + sub0;
+    double num = x + sub0;
+    if (!(fabs(den) > q.tx)) {
+        const double sub1 = -eta * y2 + y0 * (eta - 1);
+        den = eta * y3 - y1 * (eta - 1) + sub1;
+        num = sub1 + y;
+        ok = ok & (fabs(den) > q.ty);
+    }
+    // (with eta in the unit interval the divisor is in range; a numerator
+    // above the range gives a value far outside or NaN)
+    const double xi = div_refined(num, den, rcp_refined(den));
+    const double eps = 1e-15;
+    ok = ok & (fabs(num) > 0x1p-600) & (eta >= -eps) & (eta <= 1 + eps) & (xi >= -eps) & (xi <= 1 + eps);
+    out[0] = xi;
+    out[1] = eta;
+    if (!ok) return 2;
+    return (xi >= 0.0) & (xi <= 1.0) & (eta >= 0.0) & (eta <= 1.0) ? 0 : 1;
+}
+
 // Newton iteration with step-halving line search, started from the affine
 // least-squares fit of the cell (deal.II MappingQGeneric's inverse).
 template <int DIM>

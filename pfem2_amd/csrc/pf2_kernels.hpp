@@ -287,8 +287,10 @@ __device__ __forceinline__ int part_key(const DevParams& pp, const double* xi) {
     bool in = true;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) {
+        // xi_d / h truncated: h is 1/q (middle exponents), and a xi_d below
+        // them truncates to 0 either way
         const double h = pp.hq[d];
-        const unsigned num = (unsigned)(xi[d] / h);
+        const unsigned num = (unsigned)div_refined(xi[d], h, rcp_refined(h));
         key += (int)num * stride;
         stride *= pp.q[d] + 1;
         in = in && (int)num < pp.q[d];
@@ -324,84 +326,72 @@ __device__ __forceinline__ void lattice_point(const DevParams& pp, int ordinal, 
 // that is the containing cell with the largest key, earliest star position on
 // ties, which is what the loop below selects.  Returns -1 if no star cell
 // contains the point.
-struct NoPrefetch {
-    __device__ void load(int) {}
-};
-
-// nodal velocities of a candidate cell (FP64 path)
+// nodal velocities of cell c (FP64 path)
 template <int DIM, int DEG = 1>
-struct PrefetchV64 {
-    static constexpr int ND = QF<DIM, DEG>::ND;
-    const double* cellV;
-    double Vc[ND][DIM];
-    __device__ void load(int cc) {
-        const double* cf = cellV + (size_t)cc * ND * DIM;
+__device__ __forceinline__ void load_nodes(const double* __restrict__ cellV, int c, double (*Vc)[DIM]) {
+    constexpr int ND = QF<DIM, DEG>::ND;
+    const double* cf = cellV + (size_t)c * ND * DIM;
 #pragma unroll
-        for (int k = 0; k < ND; ++k)
+    for (int k = 0; k < ND; ++k)
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) Vc[k][d] = cf[k * DIM + d];
-    }
-};
+        for (int d = 0; d < DIM; ++d) Vc[k][d] = cf[k * DIM + d];
+}
 
-// `Q` returns the vertices of the cell found; `pre.load(cell)` is called for
-// each candidate before its containment test, so that a caller can have the
-// candidate's other data loaded alongside its vertices (the data of the
-// last candidate loaded is the found cell's).
 // Face through which the step from xold to x most likely left the cell: the
 // linearised reference displacement J(xi_old)^-1 (x - xold) added to xi_old,
 // the component furthest outside [0, 1] (face 2a + s is xi_a = s), -1 if
-// none.  Only a guess: the caller verifies it.
+// none.  Only a guess, which the caller verifies: it rounds as it likes
+// (fused multiply-adds) and scales by det J instead of dividing (a cell with
+// det <= 0 gets an arbitrary face).
 template <int DIM>
 __device__ __forceinline__ int exit_face(const double (*P)[DIM], const double* xi_old, const double* xold,
                                          const double* x) {
-    constexpr int NV = Q1<DIM>::NV;
-    double J[DIM][DIM], Ji[DIM][DIM], dx[DIM], dxi[DIM];
+    double J[DIM][DIM], Ji[DIM][DIM], dx[DIM];   // J[i][j] = d x_i / d xi_j
 #pragma unroll
-    for (int i = 0; i < DIM; ++i)
-#pragma unroll
-        for (int j = 0; j < DIM; ++j) J[i][j] = 0.0;
-#pragma unroll
-    for (int k = 0; k < NV; ++k)
-#pragma unroll
-        for (int j = 0; j < DIM; ++j) {
-            double w = ((k >> j) & 1) ? 1.0 : -1.0;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d)
-                if (d != j) w *= ((k >> d) & 1) ? xi_old[d] : 1.0 - xi_old[d];
-#pragma unroll
-            for (int i = 0; i < DIM; ++i) J[i][j] += w * P[k][i];
+    for (int i = 0; i < DIM; ++i) {
+        if constexpr (DIM == 2) {
+            const double e0 = P[1][i] - P[0][i], e1 = P[2][i] - P[0][i], w = (P[3][i] - P[2][i]) - e0;
+            J[i][0] = fma(w, xi_old[1], e0);
+            J[i][1] = fma(w, xi_old[0], e1);
+        } else {
+            const double a = xi_old[0], b = xi_old[1], c = xi_old[2];
+            // edge differences interpolated over the opposite directions
+            auto lin = [&](double t, double lo, double hi) { return fma(t, hi - lo, lo); };
+            J[i][0] = lin(c, lin(b, P[1][i] - P[0][i], P[3][i] - P[2][i]), lin(b, P[5][i] - P[4][i], P[7][i] - P[6][i]));
+            J[i][1] = lin(c, lin(a, P[2][i] - P[0][i], P[3][i] - P[1][i]), lin(a, P[6][i] - P[4][i], P[7][i] - P[5][i]));
+            J[i][2] = lin(b, lin(a, P[4][i] - P[0][i], P[5][i] - P[1][i]), lin(a, P[6][i] - P[2][i], P[7][i] - P[3][i]));
         }
-    // J^-1 = adj(J) / det: the face is chosen from values scaled by det, so
-    // no division (the choice is only a guess; a cell with det <= 0 gets an
-    // arbitrary one, which the caller's containment test rejects)
+    }
+    auto cof = [](double a, double b, double c, double d) { return fma(a, d, -(b * c)); };
     if constexpr (DIM == 2) {
         Ji[0][0] = J[1][1];
         Ji[0][1] = -J[0][1];
         Ji[1][0] = -J[1][0];
         Ji[1][1] = J[0][0];
     } else {
-        Ji[0][0] = J[1][1] * J[2][2] - J[1][2] * J[2][1];
-        Ji[0][1] = J[0][2] * J[2][1] - J[0][1] * J[2][2];
-        Ji[0][2] = J[0][1] * J[1][2] - J[0][2] * J[1][1];
-        Ji[1][0] = J[1][2] * J[2][0] - J[1][0] * J[2][2];
-        Ji[1][1] = J[0][0] * J[2][2] - J[0][2] * J[2][0];
-        Ji[1][2] = J[0][2] * J[1][0] - J[0][0] * J[1][2];
-        Ji[2][0] = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-        Ji[2][1] = J[0][1] * J[2][0] - J[0][0] * J[2][1];
-        Ji[2][2] = J[0][0] * J[1][1] - J[0][1] * J[1][0];
+        Ji[0][0] = cof(J[1][1], J[1][2], J[2][1], J[2][2]);
+        Ji[0][1] = cof(J[0][2], J[0][1], J[2][2], J[2][1]);
+        Ji[0][2] = cof(J[0][1], J[0][2], J[1][1], J[1][2]);
+        Ji[1][0] = cof(J[1][2], J[1][0], J[2][2], J[2][0]);
+        Ji[1][1] = cof(J[0][0], J[0][2], J[2][0], J[2][2]);
+        Ji[1][2] = cof(J[0][2], J[0][0], J[1][2], J[1][0]);
+        Ji[2][0] = cof(J[1][0], J[1][1], J[2][0], J[2][1]);
+        Ji[2][1] = cof(J[0][1], J[0][0], J[2][1], J[2][0]);
+        Ji[2][2] = cof(J[0][0], J[0][1], J[1][0], J[1][1]);
     }
-    double dt = 0.0;
+    double det = J[0][0] * Ji[0][0];
 #pragma unroll
-    for (int j = 0; j < DIM; ++j) dt += J[0][j] * Ji[j][0];
+    for (int j = 1; j < DIM; ++j) det = fma(J[0][j], Ji[j][0], det);
 #pragma unroll
     for (int d = 0; d < DIM; ++d) dx[d] = x[d] - xold[d];
-    matvec<DIM>(Ji, dx, dxi);
     int f = -1;
     double worst = 0.0;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) {
-        const double e = xi_old[d] * dt + dxi[d];   // det * (reference coordinate after the move)
-        const double o = e < 0.0 ? -e : e - dt;
+        double e = xi_old[d] * det;   // det * (reference coordinate after the move)
+#pragma unroll
+        for (int j = 0; j < DIM; ++j) e = fma(Ji[d][j], dx[j], e);
+        const double o = e < 0.0 ? -e : e - det;
         if (o > worst) {
             worst = o;
             f = 2 * d + (e < 0.0 ? 0 : 1);
@@ -410,100 +400,192 @@ __device__ __forceinline__ int exit_face(const double (*P)[DIM], const double* x
     return f;
 }
 
+// The vertex of cell c that the velocity points at most from xold: the
+// largest product of the normalised velocity and the normalised direction to
+// the vertex, the first on ties (cylinder2D/pfem2particle.cpp:283-300).  Only
+// the choice matters, so it is made with v_rsq_f64 estimates (relative error
+// below 2^-20) of |velocity| times the products wherever the largest leads
+// the next by more than 2^-14 |velocity| and the squares are in the middle of
+// the exponent range; the definition's square roots and divisions decide the
+// rest (about one in ten thousand).  9 instead of ~45 instructions a vertex.
+template <int DIM>
+__device__ __forceinline__ int star_vertex(const DevMesh<DIM>& m, int c, const double (*P)[DIM], const double* xold,
+                                           const double* vext) {
+    constexpr int NV = Q1<DIM>::NV;
+    double best = -1e300, next = -1e300, lo = 1e300, sum = 0.0;
+    int cvk = 0;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        double t = P[k][0] - xold[0];
+        double s2 = t * t, dot = vext[0] * t;
+#pragma unroll
+        for (int d = 1; d < DIM; ++d) {
+            t = P[k][d] - xold[d];
+            s2 = fma(t, t, s2);
+            dot = fma(vext[d], t, dot);
+        }
+        const double a = dot * __builtin_amdgcn_rsq(s2);
+        const bool g = a > best;
+        next = g ? best : (a > next ? a : next);
+        best = g ? a : best;
+        cvk = g ? k : cvk;
+        lo = s2 < lo ? s2 : lo;
+        sum += s2;
+    }
+    double v2 = vext[0] * vext[0];
+#pragma unroll
+    for (int d = 1; d < DIM; ++d) v2 = fma(vext[d], vext[d], v2);
+    const double lead = best - next;
+    if ((lead > 0.0) & (lead * lead > 0x1p-28 * v2) & (v2 > 0x1p-900) & (v2 < 0x1p900) & (lo > 0x1p-900) &
+        (sum < 0x1p900))
+        return cvk;
+    double vn[DIM], a0 = 0.0;
+    const double rv = 1.0 / vnorm<DIM>(vext);
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) vn[d] = vext[d] * rv;
+    cvk = 0;
+#pragma unroll 1
+    for (int k = 0; k < NV; ++k) {
+        const double* p = m.cellX + ((size_t)c * NV + k) * DIM;
+        double t[DIM];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) t[d] = p[d] - xold[d];
+        const double rn = 1.0 / vnorm<DIM>(t);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) t[d] *= rn;
+        const double a = vdot<DIM>(vn, t);
+        if (k == 0 || a > a0) {
+            cvk = k;
+            a0 = a;
+        }
+    }
+    return cvk;
+}
+
 // margin in reference coordinates beyond which a point inside one cell is
 // inside no other cell under the containment test (the Newton acceptance
 // radius is 1e-10 of a cell diameter)
 constexpr double NBR_MARGIN = 1e-6;
 
-template <int DIM, class Pre, bool SHORTCUT = true>
+template <int DIM>
+__device__ __forceinline__ bool inside_margin(const double* r) {
+    bool in = true;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) in = in & (r[d] >= NBR_MARGIN) & (r[d] <= 1.0 - NBR_MARGIN);
+    return in;
+}
+
+// inverse_map and the unit-cell test of a candidate cell.  CLOSED (2-D): the
+// closed form first, the clearly-outside test only where it does not decide
+// (both orders give the same answer).
+template <int DIM, bool CLOSED>
+__device__ __forceinline__ bool contains(const double (*Q)[DIM], const double* x, double* r, double tol) {
+    if constexpr (CLOSED && DIM == 2) {
+        QuadCell qc;
+        qc.init(Q);
+        const int st = closed_form(Q, qc, x, r);
+        if (st != 2) return st == 0;
+    }
+    return inverse_map<DIM>(Q, x, r, tol, true) && inside_unit<DIM>(r);
+}
+
+// `Q` returns the vertices of the cell found.  (A caller's other data of the
+// cell, loaded with each candidate's vertices to overlap the two loads, cost
+// more in registers than it saved: FP64 search 167 -> 147 us, FP32 round 0
+// 77 -> 71 us per step on 101,785 cells without it.)
+//
+// OWN and own (2-D): the own-cell test's clearly-outside test said no and the
+// rest of it is pending; only that test runs: c is returned if it places x in
+// cell c, else RELOC_AGAIN, and the caller comes back for the search.
+//
+// The own cell and the star cells go through one inlined inverse map: the
+// code of its Newton iteration is large, and with four copies of it the
+// search kernels missed the instruction cache.
+constexpr int RELOC_AGAIN = -2;
+
+template <int DIM, bool SHORTCUT, bool OWN>
 __device__ __forceinline__ int relocate(const DevMesh<DIM>& m, int c, const double (*P)[DIM], const double* xi_old,
-                        const double* vext, const double* x, double* xi_out, double (*Q)[DIM], Pre& pre) {
+                                        const double* vext, const double* x, double* xi_out, double (*Q)[DIM],
+                                        int& searches, bool own) {
     constexpr int NV = Q1<DIM>::NV;
     constexpr int CH = 4;   // star entries read together
-    int nb[2 * DIM];
-    if constexpr (SHORTCUT) {
+    int s0 = 0, n = 0, last = -1;
+    double dir[DIM], lastkey = 0.0;
+    // the selected vertex and its star; the face-neighbour shortcut (its cell, or -1)
+    auto select = [&]() -> int {
+        ++searches;
+        int nb[2 * DIM];
+        if constexpr (SHORTCUT) {
 #pragma unroll
-        for (int h = 0; h < DIM - 1; ++h) {
-            const int4 q = m.cell_nbr[(size_t)c * (DIM - 1) + h];
-            nb[4 * h] = q.x;
-            nb[4 * h + 1] = q.y;
-            if (4 * h + 2 < 2 * DIM) nb[4 * h + 2] = q.z;
-            if (4 * h + 3 < 2 * DIM) nb[4 * h + 3] = q.w;
+            for (int h = 0; h < DIM - 1; ++h) {
+                const int4 q = m.cell_nbr[(size_t)c * (DIM - 1) + h];
+                nb[4 * h] = q.x;
+                nb[4 * h + 1] = q.y;
+                if (4 * h + 2 < 2 * DIM) nb[4 * h + 2] = q.z;
+                if (4 * h + 3 < 2 * DIM) nb[4 * h + 3] = q.w;
+            }
         }
-    }
-    double xold[DIM], vn[DIM], t[DIM];
-    forward<DIM>(P, xi_old, xold);
-    const double rv = 1.0 / vnorm<DIM>(vext);
+        double xold[DIM];
+        forward<DIM>(P, xi_old, xold);
+        const int cvk = star_vertex<DIM>(m, c, P, xold, vext);
+        if constexpr (SHORTCUT) {
+            // Face-neighbour shortcut.  The neighbour g across the exit face
+            // is in the selected vertex's star when that vertex lies on the
+            // face; if g contains x at least NBR_MARGIN inside, no other cell
+            // contains x, so g is the first containing cell of the star in
+            // any order: the star loop's result, with the same inverse map
+            // (2-D: its closed form, which alone places a point there but
+            // for a few that the star loop then finds).
+            const int f = exit_face<DIM>(P, xi_old, xold, x);
+            int g = -1;
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) vn[d] = vext[d] * rv;
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) t[d] = P[0][d] - xold[d];
-    double rn = 1.0 / vnorm<DIM>(t);
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) t[d] *= rn;
-    double best = vdot<DIM>(vn, t);
-    int cvk = 0;
-    double dir[DIM];
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) dir[d] = P[0][d];
-#pragma unroll
-    for (int k = 1; k < NV; ++k) {
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) t[d] = P[k][d] - xold[d];
-        rn = 1.0 / vnorm<DIM>(t);
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) t[d] *= rn;
-        const double a = vdot<DIM>(vn, t);
-        if (a > best) {
-            cvk = k;
-            best = a;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) dir[d] = P[k][d];
-        }
-    }
-    // the selected vertex's star range, loaded alongside the shortcut's cell
-    const int2 se = m.cell_star[(size_t)c * NV + cvk];
-    if constexpr (SHORTCUT) {
-        // Face-neighbour shortcut.  The neighbour g across the exit face is in
-        // the selected vertex's star when that vertex lies on the face; if g
-        // contains x at least NBR_MARGIN inside, no other cell contains x,
-        // so g is the first containing cell of the star in any order: the
-        // result of the loop below, with the same inverse map.
-        const int f = exit_face<DIM>(P, xi_old, xold, x);
-        if (f >= 0 && ((cvk >> (f >> 1)) & 1) == (f & 1)) {
-            int g = nb[0];
-#pragma unroll
-            for (int q = 1; q < 2 * DIM; ++q)
-                if (f == q) g = nb[q];
+            for (int q = 0; q < 2 * DIM; ++q)
+                if (f == q && ((cvk >> (q >> 1)) & 1) == (q & 1)) g = nb[q];
             if (g >= 0) {
-                double r[DIM];
                 load_vertices<DIM>(m, g, Q);
-                pre.load(g);
-                bool in = inverse_map<DIM>(Q, x, r, m.ftol[g], true);
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) in = in && r[d] >= NBR_MARGIN && r[d] <= 1.0 - NBR_MARGIN;
-                if (in) {
+                double r[DIM];
+                bool in;
+                if constexpr (DIM == 2) {
+                    QuadCell qc;
+                    qc.init(Q);
+                    in = closed_form(Q, qc, x, r) == 0;
+                } else {
+                    in = inverse_map<DIM>(Q, x, r, m.ftol[g], true);
+                }
+                if (in && inside_margin<DIM>(r)) {
 #pragma unroll
                     for (int d = 0; d < DIM; ++d) xi_out[d] = r[d];
                     return g;
                 }
             }
         }
+        const int2 se = m.cell_star[(size_t)c * NV + cvk];
+        s0 = se.x;
+        n = se.y - se.x;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) dir[d] = x[d] - m.cellX[((size_t)c * NV + cvk) * DIM + d];
+        const double rn = 1.0 / vnorm<DIM>(dir);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) dir[d] *= rn;
+        return -1;
+    };
+    const bool one = OWN && own;
+    if (!one) {
+        const int g = select();
+        if (g >= 0) return g;
     }
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) dir[d] = x[d] - dir[d];
-    rn = 1.0 / vnorm<DIM>(dir);
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) dir[d] *= rn;
-    const int s0 = se.x, n = se.y - se.x;
-    if (n <= 32) {
-        // candidates in decreasing key order (ties: star order), first
-        // containing cell wins -- the reference's sorted loop, stopping early.
-        // Each pass re-reads the star (cache hits, CH entries at a time)
-        // instead of holding the keys in registers.
-        unsigned tried = 0;
-        for (int it = 0; it < n; ++it) {
-            int best_e = -1, cc = -1;
+    for (int it = 0;; ++it) {
+        int cc = c;
+        if (one) {
+            if (it > 0) return RELOC_AGAIN;
+        } else {
+            // star candidates in decreasing key order (ties: star order),
+            // first containing cell wins -- the reference's sorted loop,
+            // stopping early.  Each pass re-reads the star (cache hits, CH
+            // entries at a time) for the first entry after the last one
+            // tried.  (x on the selected vertex: keys are NaN, star order.)
+            if (it >= n) return -1;
+            int be = -1;
             double bk = 0.0;
             for (int e0 = 0; e0 < n; e0 += CH) {
                 double key[CH];
@@ -515,54 +597,31 @@ __device__ __forceinline__ int relocate(const DevMesh<DIM>& m, int c, const doub
 #pragma unroll
                     for (int d = 0; d < DIM; ++d) sd[d] = m.star_dir[(size_t)(s0 + e) * DIM + d];
                     key[u] = vdot<DIM>(sd, dir);
+                    if (!(key[u] == key[u])) key[u] = 0.0;
                     cell[u] = m.star_cell[s0 + e];
                 }
 #pragma unroll
                 for (int u = 0; u < CH; ++u) {
                     const int e = e0 + u;
-                    if (e < n && !((tried >> e) & 1u) && (best_e < 0 || key[u] > bk)) {
-                        best_e = e;
+                    const bool left = it == 0 || key[u] < lastkey || (key[u] == lastkey && e > last);
+                    if (e < n && left && (be < 0 || key[u] > bk)) {
+                        be = e;
                         bk = key[u];
                         cc = cell[u];
                     }
                 }
             }
-            tried |= 1u << best_e;
-            double r[DIM];
-            load_vertices<DIM>(m, cc, Q);
-            pre.load(cc);
-            if (inverse_map<DIM>(Q, x, r, m.ftol[cc], true) && inside_unit<DIM>(r)) {
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) xi_out[d] = r[d];
-                return cc;
-            }
+            last = be;
+            lastkey = bk;
         }
-        return -1;
-    }
-    // stars of more than 32 cells: the containing cell with the largest key
-    int bestc = -1;
-    double bestkey = 0.0;
-    for (int e = s0; e < s0 + n; ++e) {
-        double sd[DIM];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) sd[d] = m.star_dir[(size_t)e * DIM + d];
-        const double key = vdot<DIM>(sd, dir);
-        if (bestc >= 0 && !(key > bestkey)) continue;
-        const int cc = m.star_cell[e];
         double r[DIM];
         load_vertices<DIM>(m, cc, Q);
-        if (inverse_map<DIM>(Q, x, r, m.ftol[cc], true) && inside_unit<DIM>(r)) {
-            bestc = cc;
-            bestkey = key;
+        if (contains<DIM, !SHORTCUT>(Q, x, r, m.ftol[cc])) {
 #pragma unroll
             for (int d = 0; d < DIM; ++d) xi_out[d] = r[d];
+            return cc;
         }
     }
-    if (bestc >= 0) {
-        load_vertices<DIM>(m, bestc, Q);
-        pre.load(bestc);
-    }
-    return bestc;
 }
 
 // ---------------------------------------------------------------------------
@@ -752,48 +811,37 @@ constexpr int PARK_NEWTON = 1 << 30;
 constexpr int DEST_KEPT = 1 << 30;
 
 // Runs substeps until done (returns 0) or the own-cell test fails (returns
-// 1; s is the substep whose test failed).  pending: the test of substep s at
-// the current x comes first, before any new substep.
-// CLOSED (2-D, k_move): the own-cell test takes only inverse_map's closed
-// form and returns 2 where inverse_map would go on to its clearly-outside
-// test and Newton iteration (the point is outside the closed form's unit
-// square, or the closed form is degenerate); the search kernel finishes that
-// test (pending).  This keeps the Newton code, and its registers, out of
+// 1; s is the substep whose test failed).
+// CLOSED (2-D): the own-cell test takes only inverse_map's closed form and
+// returns 2 where inverse_map would go on to its clearly-outside test and
+// Newton iteration (the point is outside the closed form's unit square, or
+// closed_form leaves it undecided); the search finishes that test
+// (relocate's `own`).  This keeps the Newton code, and its registers, out of
 // k_move: 94 instead of 167 registers, 5 instead of 3 wavefronts per SIMD.
 template <int DIM, int DEG = 1, bool CLOSED = false>
 __device__ __forceinline__ int advance64(const DevMesh<DIM>& m, const double* __restrict__ V, const DevParams& pp,
                                          const DevParticles& A, int i, int c, double* x, double* xi, double* vext,
-                                         int& s, const double (*P)[DIM], const double (*Vc)[DIM], double tol,
-                                         bool pending = false) {
-    for (;; ++s) {
-        if (!pending) {
-            if (s >= pp.substeps) return 0;
-            double u[DIM];
-            interp<DIM, DEG>(Vc, xi, u);
+                                         int& s, const double (*P)[DIM], const double (*Vc)[DIM], double tol) {
+    QuadCell qc;
+    if constexpr (CLOSED && DIM == 2) qc.init(P);
+    for (; s < pp.substeps; ++s) {
+        double u[DIM];
+        interp<DIM, DEG>(Vc, xi, u);
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) vext[d] = u[d];
+        for (int d = 0; d < DIM; ++d) vext[d] = u[d];
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) u[d] *= pp.h;
+        for (int d = 0; d < DIM; ++d) u[d] *= pp.h;
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) x[d] = x[d] + u[d];
-            if (pp.keep_vext && s == pp.substeps - 1)
+        for (int d = 0; d < DIM; ++d) x[d] = x[d] + u[d];
+        if (pp.keep_vext && s == pp.substeps - 1)
 #pragma unroll
-                for (int d = 0; d < DIM; ++d) A.vext[(size_t)d * A.cap + i] = vext[d];
-        }
-        pending = false;
+            for (int d = 0; d < DIM; ++d) A.vext[(size_t)d * A.cap + i] = vext[d];
         double r[DIM];
         if constexpr (CLOSED && DIM == 2) {
-            // inverse_map<2>(P, x, r, tol, false) up to its clearly-outside test
-            if (inverse_quadratic(P, x, r)) {
-                const double eps = 1e-15;
-                if (-eps <= r[1] && r[1] <= 1 + eps && -eps <= r[0] && r[0] <= 1 + eps) {
-                    if (!inside_unit<DIM>(r)) return 1;
+            const int st = closed_form(P, qc, x, r);
+            if (st) return st;
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) xi[d] = r[d];
-                    continue;
-                }
-            }
-            return 2;
+            for (int d = 0; d < DIM; ++d) xi[d] = r[d];
         } else {
             if (inverse_map<DIM>(P, x, r, tol, false) && inside_unit<DIM>(r)) {
 #pragma unroll
@@ -803,6 +851,7 @@ __device__ __forceinline__ int advance64(const DevMesh<DIM>& m, const double* __
             }
         }
     }
+    return 0;
 }
 
 // final bookkeeping of a particle whose substeps are complete (all lanes call)
@@ -977,89 +1026,40 @@ __device__ __forceinline__ void search_body(const Grid& G, const DevMesh<DIM>& m
         }
         if (__ballot(have) == 0) break;
         bool done = false;
-        if constexpr (RESORT) {
-            // re-sort after a mesh move: the own-cell test left by k_resort,
-            // then the relocation; no advection
-            if (have) {
-                double r[DIM];
-                bool own = false;
-                if (newton) {
-                    newton = false;
-                    own = !clearly_outside<DIM>(P, x, m.ftol[c]) && inverse_newton<DIM>(P, x, r) &&
-                          inside_unit<DIM>(r);
-                }
-                if (!own) {
-                    double Q[NV][DIM];
-                    ++searches;
-                    NoPrefetch pre;
-                    c = relocate<DIM>(m, c, P, xi, vext, x, r, Q, pre);
-                    if (c < 0) ++lost;
-                }
-                if (c >= 0)
+        if (have) {
+            // a particle whose own-cell test is pending (2-D): clearly
+            // outside, it goes to the search; otherwise relocate runs the rest
+            // of the test first
+            const bool own = DIM == 2 && newton && !clearly_outside<DIM>(P, x, m.ftol[c]);
+            newton = false;
+            // (3-D: the face-neighbour shortcut's registers push this kernel
+            // into heavy spilling)
+            double Q[NV][DIM], r[DIM];
+            const int cn =
+                relocate<DIM, DIM == 2 || RESORT, DIM == 2>(m, c, P, xi, vext, x, r, Q, searches, own);
+            done = cn == -1;
+            if (cn >= 0) {
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) xi[d] = r[d];
-                done = true;
-            }
-        } else if (DIM == 2 && have) {
-            // a particle k_move flagged has its own-cell test at x pending:
-            // clearly outside, it goes to the search; otherwise the test
-            // (inverse_map from its closed form, as in advance64) runs first
-            // in advance64, which goes on in the cell if x is inside
-            bool own = false;
-            if (newton) {
-                newton = false;
-                own = !clearly_outside<DIM>(P, x, m.ftol[c]);
-            }
-            double r[DIM];
-            PrefetchV64<DIM, DEG> pre{m.cellV};
-            int cn = c;
-            if (own) {
-                pre.load(c);
-            } else {
-                double Q[NV][DIM];
-                ++searches;
-                cn = relocate<DIM, PrefetchV64<DIM, DEG>, true>(m, c, P, xi, vext, x, r, Q, pre);
-                if (cn >= 0)
+                for (int d = 0; d < DIM; ++d) xi[d] = r[d];
+                if constexpr (RESORT) {
+                    done = true;   // re-sort after a mesh move: no advection
+                } else {
+                    ++s;
+                    double Vc[QF<DIM, DEG>::ND][DIM];
+                    load_nodes<DIM, DEG>(m.cellV, cn, Vc);
 #pragma unroll
                     for (int k = 0; k < NV; ++k)
 #pragma unroll
                         for (int d = 0; d < DIM; ++d) P[k][d] = Q[k][d];
-            }
-            if (cn < 0) {
-                c = -1;
-                ++lost;
-                done = true;
-            } else {
-                if (!own) {
-                    c = cn;
-#pragma unroll
-                    for (int d = 0; d < DIM; ++d) xi[d] = r[d];
-                    ++s;
+                    // (2-D: a test the closed form does not decide comes back
+                    // as pending, as from k_move)
+                    const int st = advance64<DIM, DEG, true>(m, V, pp, A, i, cn, x, xi, vext, s, P, Vc, m.ftol[cn]);
+                    done = st == 0;
+                    newton = st == 2;
                 }
-                done = advance64<DIM, DEG>(m, V, pp, A, i, c, x, xi, vext, s, P, pre.Vc, m.ftol[c], own) == 0;
             }
-        } else if (have) {
-            // 3-D (k_move finishes its own-cell tests)
-            double Q[NV][DIM], r[DIM];
-            ++searches;
-            PrefetchV64<DIM, DEG> pre{m.cellV};
-            // (the face-neighbour shortcut's registers push this kernel into heavy spilling)
-            const int cn = relocate<DIM, PrefetchV64<DIM, DEG>, false>(m, c, P, xi, vext, x, r, Q, pre);
-            if (cn < 0) {
-                c = -1;
-                ++lost;
-                done = true;
-            } else {
-                c = cn;
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) xi[d] = r[d];
-                ++s;
-#pragma unroll
-                for (int k = 0; k < NV; ++k)
-#pragma unroll
-                    for (int d = 0; d < DIM; ++d) P[k][d] = Q[k][d];
-                done = advance64<DIM, DEG>(m, V, pp, A, i, c, x, xi, vext, s, P, pre.Vc, m.ftol[c]) == 0;
-            }
+            if (cn != RELOC_AGAIN) c = cn;
+            if (cn == -1) ++lost;
         }
         finish_particle<DIM>(pp, A, w, done, i, c, x, xi, true, seg_end);
         if (done) have = false;
@@ -2357,13 +2357,9 @@ __global__ void __launch_bounds__(256) k_resort(DevMesh<DIM> m, DevParticles A, 
                 for (int d = 0; d < DIM; ++d) x[d] = A.x[(size_t)d * A.cap + i];
                 load_vertices<DIM>(m, c, P);
                 if constexpr (DIM == 2) {
-                    // inverse_map<2>(P, x, r, tol, false) up to its clearly-outside test
-                    st = 2;
-                    if (inverse_quadratic(P, x, r)) {
-                        const double eps = 1e-15;
-                        if (-eps <= r[1] && r[1] <= 1 + eps && -eps <= r[0] && r[0] <= 1 + eps)
-                            st = inside_unit<DIM>(r) ? 0 : 1;
-                    }
+                    QuadCell qc;
+                    qc.init(P);
+                    st = closed_form(P, qc, x, r);
                 } else {
                     st = inverse_map<DIM>(P, x, r, m.ftol[c], false) && inside_unit<DIM>(r) ? 0 : 1;
                 }

@@ -327,16 +327,6 @@ __device__ __forceinline__ void load_cell32(const float* __restrict__ geo, const
         for (int d = 0; d < DIM; ++d) Fc[k][d] = cellV32[((size_t)c * ND + k) * DIM + d];
 }
 
-// FP32 coefficients and nodal velocities of a candidate cell
-template <int DIM, int DEG = 1>
-struct PrefetchCell32 {
-    const float* geo;
-    const float* V32;
-    float g[DIM == 2 ? 6 : 21];
-    float Vc[QF<DIM, DEG>::ND][DIM];
-    __device__ void load(int cc) { load_cell32<DIM, DEG>(geo, V32, cc, g, Vc); }
-};
-
 template <int DIM>
 __device__ __forceinline__ int part_key32(const DevParams& pp, const float* xi) {
     double xd[DIM];
@@ -618,13 +608,11 @@ __global__ void __launch_bounds__(256) k_move32(DevMesh<DIM> m, const float* __r
 
 // FP64 relocation of queued particles (the reference rule), then the
 // remaining FP32 substeps
-// (LAST: the last round, which loops every particle to its end.  Its
-// particles cross several cells per step and the face-neighbour shortcut
-// misses more often there: measured 4-8% slower with it.  It runs few
-// wavefronts, so it takes the full register budget (2 per SIMD, no spills).
+// (LAST: the last round, which loops every particle to its end.  It runs
+// few wavefronts, so it takes the register budget of 2 per SIMD, no spills.
 // The first round is latency-bound with many wavefronts: in 2-D 4 per SIMD
-// (128 registers, 8 bytes per lane spilled) runs it 12% faster than 3
-// without spills; in 3-D 3 per SIMD (212 bytes spilled) 3% faster than 2.)
+// runs it in 71 us per step on 101,785 cells, 3 in 79, 5 in 80; in 3-D 3 per
+// SIMD with spills were 3% faster than 2.)
 template <int DIM, bool LAST, int DEG = 1>
 __device__ __forceinline__ void search32_body(const Grid& G, const DevMesh<DIM>& m, const float* __restrict__ V32, const float* __restrict__ geo, const int* __restrict__ pcell, const Rec32& R, double* __restrict__ pvext, long long cap, const DevParams& pp, const DevWork& w, const DevQueues& qu, int round) {
     constexpr int NV = Q1<DIM>::NV;
@@ -659,12 +647,11 @@ __device__ __forceinline__ void search32_body(const Grid& G, const DevMesh<DIM>&
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) u[d] = (float)qu.park_vext[(size_t)d * cap + i];
             }
-            // 2-D: the found cell's vertices and FP32 data are loaded with the
-            // candidate and reused; 3-D reloads them (register budget)
+            // 2-D: the found cell's vertices are kept for the next relocation;
+            // 3-D reloads them (register budget)
             double P[NV][DIM];
             load_vertices<DIM>(m, c, P);
             for (;;) {
-                ++searches;
                 double Q[NV][DIM], xid[DIM], x[DIM], vext[DIM], r[DIM];
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) {
@@ -674,33 +661,20 @@ __device__ __forceinline__ void search32_body(const Grid& G, const DevMesh<DIM>&
                 forward<DIM>(P, xid, x);
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) x[d] = x[d] + (double)(u[d] * h32);
-                int cn;
-                if constexpr (DIM == 2) {
-                    PrefetchCell32<DIM, DEG> pre{geo, V32};
-                    cn = relocate<DIM, PrefetchCell32<DIM, DEG>, !LAST>(m, c, P, xid, vext, x, r, Q, pre);
-                    if (cn >= 0) {
+                // (the last round's particles cross several cells and the
+                // face-neighbour shortcut misses more often: 58 us without it,
+                // 77 with it, on 101,785 cells)
+                const int cn = relocate<DIM, DIM == 3 || !LAST, false>(m, c, P, xid, vext, x, r, Q, searches, false);
+                if (cn >= 0) {
 #pragma unroll
-                        for (int d = 0; d < DIM; ++d) {
-                            const float t = (float)r[d];
-                            xi[d] = t < 0.0f ? 0.0f : (t > 1.0f ? 1.0f : t);
-                        }
-                        ++s;
-                        st = advance32<DIM, DEG>(pp, h32, i, pvext, cap, xi, u, s, pre.g, pre.Vc);
+                    for (int d = 0; d < DIM; ++d) {
+                        const float t = (float)r[d];
+                        xi[d] = t < 0.0f ? 0.0f : (t > 1.0f ? 1.0f : t);
                     }
-                } else {
-                    NoPrefetch pre;
-                    cn = relocate<DIM>(m, c, P, xid, vext, x, r, Q, pre);
-                    if (cn >= 0) {
-#pragma unroll
-                        for (int d = 0; d < DIM; ++d) {
-                            const float t = (float)r[d];
-                            xi[d] = t < 0.0f ? 0.0f : (t > 1.0f ? 1.0f : t);
-                        }
-                        float g[NG], Vc[ND][DIM];
-                        load_cell32<DIM, DEG>(geo, V32, cn, g, Vc);
-                        ++s;
-                        st = advance32<DIM, DEG>(pp, h32, i, pvext, cap, xi, u, s, g, Vc);
-                    }
+                    float g[NG], Vc[ND][DIM];
+                    load_cell32<DIM, DEG>(geo, V32, cn, g, Vc);
+                    ++s;
+                    st = advance32<DIM, DEG>(pp, h32, i, pvext, cap, xi, u, s, g, Vc);
                 }
                 if (cn < 0) {
                     c = -1;
@@ -1342,12 +1316,9 @@ __global__ void __launch_bounds__(256) k_resort32(DevMesh<DIM> m, const int* __r
                 for (int d = 0; d < DIM; ++d) x[d] = px[(size_t)d * cap + i];
                 load_vertices<DIM>(m, c, P);
                 if constexpr (DIM == 2) {
-                    st = 2;
-                    if (inverse_quadratic(P, x, r)) {
-                        const double eps = 1e-15;
-                        if (-eps <= r[1] && r[1] <= 1 + eps && -eps <= r[0] && r[0] <= 1 + eps)
-                            st = inside_unit<DIM>(r) ? 0 : 1;
-                    }
+                    QuadCell qc;
+                    qc.init(P);
+                    st = closed_form(P, qc, x, r);
                 } else {
                     st = inverse_map<DIM>(P, x, r, m.ftol[c], false) && inside_unit<DIM>(r) ? 0 : 1;
                 }
@@ -1399,15 +1370,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM ==
                 vext[d] = pvext ? pvext[(size_t)d * cap + i] : 0.0;
             }
             load_vertices<DIM>(m, c, P);
-            const bool own = qu.park_s[i] == PARK_NEWTON && !clearly_outside<DIM>(P, x, m.ftol[c]) &&
-                             inverse_newton<DIM>(P, x, r) && inside_unit<DIM>(r);
-            if (!own) {
-                ++searches;
-                double Q[NV][DIM];
-                NoPrefetch pre;
-                c = relocate<DIM>(m, c, P, xi, vext, x, r, Q, pre);
-                if (c < 0) ++lost;
-            }
+            bool own = DIM == 2 && qu.park_s[i] == PARK_NEWTON && !clearly_outside<DIM>(P, x, m.ftol[c]);
+            double Q[NV][DIM];
+            int cn;
+            while ((cn = relocate<DIM, true, DIM == 2>(m, c, P, xi, vext, x, r, Q, searches, own)) == RELOC_AGAIN)
+                own = false;
+            c = cn;
+            if (c < 0) ++lost;
             if (c >= 0) {
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) {
