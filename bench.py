@@ -171,24 +171,17 @@ def kernel_bytes(name, info, m, dim=2, vext=False):
     if name == "k_cell_count":
         return (n0 + arr) * 12 + arr * 4 + n0 * 4 + nc * (8 + 4 + 4 + 20)
     if name in ("k_cell_write", "k_cell_write32"):
-        wx = 8 if name == "k_cell_write" else 4
-        per_src = 4 + 4 + 4 + dim * wx * (3 if name == "k_cell_write" else 2) + (dim * 8 if vext else 0)
-        per_dst = 4 + 4 + dim * wx * (3 if name == "k_cell_write" else 2) + (dim * 8 if vext else 0)
-        return n1 * (per_src + per_dst) + nc * 32
+        # slot entry, id and record of each output position in, cell, id and
+        # record out; per cell: census results in, offset, resets and
+        # projection sums out
+        rec = dim * 8 * 3 if name == "k_cell_write" else (16 if dim == 2 else 24)
+        rec += dim * 8 if vext else 0
+        return n1 * (4 + 4 + rec + 4 + 4 + rec) + nc * (28 + 12 + nv * (dim + 1) * 8)
     if name == "k_cell_pend":
         # the pending layout after a re-sort (the census marked the
         # survivors): per cell the spawn count in and the resets out; new
         # particles written whole (few)
         return nc * (8 + 8)
-    if name == "k_cell_map":
-        # per-cell census results in, the output map and per-cell resets out
-        return nc * (36 + 12) + n1 * (4 + 4)
-    if name in ("k_cell_gather", "k_cell_gather32"):
-        # map and destination of each output position, the record copied in order
-        rec = dim * 8 * 3 if name == "k_cell_gather" else (16 if dim == 2 else 24)
-        per_src = 4 + 4 + 4 + rec + (dim * 8 if vext else 0)
-        per_dst = 4 + 4 + rec + (dim * 8 if vext else 0)
-        return n1 * (per_src + per_dst)
     if name in ("k_cell_partials", "k_cell_partials32"):
         wx = 8 if name == "k_cell_partials" else 4
         return n1 * dim * wx * 2 + nc * (4 + nv * (dim + 1) * 8)

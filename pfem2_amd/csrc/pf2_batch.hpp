@@ -2,7 +2,7 @@
 //
 // A batch lists simulations of the same dimension and precision.  Every
 // kernel of the step (field refresh, move, relocation rounds, census, offset
-// scan, write, bookkeeping, projection) is launched once for the whole
+// scan, write with the projection sums, bookkeeping, node sums) is launched once for the whole
 // batch: the launch's workgroups are split into consecutive ranges, one per
 // simulation (sized as that simulation's own launch would be), and each
 // workgroup runs the kernel body of its simulation with the range as its
@@ -20,7 +20,7 @@ namespace pf2 {
 
 enum BatchKind {
     BK_REFRESH = 0, BK_MOVE, BK_SEARCH0, BK_SEARCH1, BK_SEARCH2, BK_COUNT, BK_COUNT_L, BK_BIG, BK_TILES,
-    BK_WRITE, BK_PARTIALS, BK_NODE, BK_NKINDS
+    BK_WRITE, BK_NODE, BK_NKINDS
 };
 static_assert(MOVE_ROUNDS <= 2, "kinds for up to three relocation rounds");
 
@@ -38,6 +38,7 @@ struct BatchSim {
     float *V32, *dV32;
     const float* geo;
     double* partial;
+    int* omap;                    // positions of cells whose survivors outnumber the slot row
     int* qcount;
     unsigned long long* tiles;    // tile sums of the offset scan
     int ntiles;                   // tiles of SCAN_TILE entries of the n_cells + 1 counts
@@ -80,7 +81,7 @@ __global__ void __launch_bounds__(256) kb_refresh(BatchView<DIM> bv) {
 }
 
 template <int DIM>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 3 : 2))) kb_move(BatchView<DIM> bv) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 5 : 2))) kb_move(BatchView<DIM> bv) {
     Grid G;
     const BatchSim<DIM>& S = bv.at(BK_MOVE, G);
     move_body<DIM>(G, S.m, S.V, S.Vold, S.A, S.pp, S.w, S.qu, 1, 1);
@@ -204,15 +205,15 @@ template <int DIM>
 __global__ void __launch_bounds__(256) kb_write(BatchView<DIM> bv) {
     Grid G;
     const BatchSim<DIM>& S = bv.at(BK_WRITE, G);
-    cell_write_body<DIM, false, false>(G, S.m, S.V, S.old_off, S.A, S.B, S.pp, S.w, S.partial);
+    cell_write_body<DIM, false, true, 1>(G, S.m, S.old_off, S.A, S.B, S.pp, S.w, S.omap, S.partial);
 }
 
 template <int DIM>
 __global__ void __launch_bounds__(256) kb_write32(BatchView<DIM> bv) {
     Grid G;
     const BatchSim<DIM>& S = bv.at(BK_WRITE, G);
-    cell_write32_body<DIM, false>(G, S.m, S.V32, S.old_off, S.A.id, S.RA, S.B.cell, S.B.id, S.RB, S.A.vext,
-                                  S.B.vext, S.A.cap, S.pp, S.w, S.partial);
+    cell_write32_body<DIM, true, 1>(G, S.m.n_cells, S.V32, S.old_off, S.A.id, S.RA, S.B.cell, S.B.id, S.RB, S.A.vext,
+                                    S.B.vext, S.A.cap, S.pp, S.w, S.omap, S.partial);
 }
 
 // workgroup s: simulation s's bookkeeping after the write (k_finalize's work)
@@ -220,21 +221,6 @@ template <int DIM>
 __global__ void __launch_bounds__(QSHARDS) kb_finalize(BatchView<DIM> bv) {
     const BatchSim<DIM>& S = bv.sims[blockIdx.x];
     finalize_block(S.m.n_cells, S.w, S.qcount);
-}
-
-// after the write the other buffer holds the particles and new_off their offsets
-template <int DIM>
-__global__ void __launch_bounds__(256) kb_partials(BatchView<DIM> bv) {
-    Grid G;
-    const BatchSim<DIM>& S = bv.at(BK_PARTIALS, G);
-    partials_body<DIM>(G, S.m.n_cells, S.w.new_off, S.B, S.partial, S.w.counters);
-}
-
-template <int DIM>
-__global__ void __launch_bounds__(256) kb_partials32(BatchView<DIM> bv) {
-    Grid G;
-    const BatchSim<DIM>& S = bv.at(BK_PARTIALS, G);
-    partials32_body<DIM>(G, S.m.n_cells, S.w.new_off, S.RB, S.partial, S.w.counters);
 }
 
 template <int DIM>

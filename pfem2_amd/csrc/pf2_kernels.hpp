@@ -18,10 +18,10 @@
 //   k_cell_count   one 16-lane group per cell: part counts over stayers +
 //                  arrivals, survivors (MAX smallest ids per part), empty
 //                  parts to reseed, final count (k_cell_big: larger cells).
-//   k_cell_write   one 16-lane group per cell: survivors and new particles
-//                  into the other buffer at their final positions.
-//   k_cell_partials one group per cell: per-cell projection sums in
-//                  ascending id order.
+//   k_cell_write   survivors and new particles into the other buffer at
+//                  their final positions, and the cells' projection sums in
+//                  ascending id order (k_cell_partials: the sums alone, one
+//                  group per cell, for a projection without a move).
 //   k_node         one thread per DoF: sum of the cell partials in ascending
 //                  cell order, then division by the weight.
 // No floating-point atomics anywhere.  Integer atomics only build lists whose
@@ -1119,33 +1119,7 @@ constexpr int SMALL_ROW_SURVIVORS = GCAP - 8;
 __host__ __device__ inline bool census_small_row(int nparts, int max_per_part) {
     return nparts <= 16 || (long long)max_per_part * nparts <= SMALL_ROW_SURVIVORS;
 }
-constexpr int FCAP = 64;             // final particles per cell staged for the fused projection sums
-constexpr int WU = 4;                // survivors per lane and pass in the regroup write
 constexpr int NKMAX = 272;           // part keys counted per group in the census (prod(q_d + 1))
-
-// put(particle, position) for each survivor of cell c as the census left
-// them: listed in id order in the cell's slot row when they fit, else by
-// the position the census stored per candidate (the old segment's stayers,
-// the slots and the overflow list)
-template <class F>
-__device__ __forceinline__ void survivors_of(const DevWork& w, const int* old_off, int c, int n_st, int kin,
-                                             int nsurv, int gl, F put) {
-    if (nsurv <= w.aslots) {
-        for (int t = gl; t < nsurv; t += GS) put(w.arr_slot[(size_t)c * w.aslots + t], t);
-        return;
-    }
-    for (int j = gl; j < kin; j += GS) {
-        const int idx = candidate(w, old_off, c, n_st, j);
-        // arrivals are in this cell's slots because their destination is c
-        if (j < n_st && w.dest[idx] != c) continue;
-        const int pos = w.spos[idx];
-        if (pos >= 0) put(idx, pos);
-    }
-    for_overflow(w, c, gl, GS, [&](int, int idx) {
-        const int pos = w.spos[idx];
-        if (pos >= 0) put(idx, pos);
-    });
-}
 
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1521,366 +1495,241 @@ __global__ void __launch_bounds__(256) k_cell_big(const int* __restrict__ old_of
 }
 
 // ---------------------------------------------------------------------------
-// k_cell_write: survivors and reseeded particles into buffer B.
+// k_cell_write: the regroup write, survivors and reseeded particles into
+// buffer B at their final positions, with the projection sums of the cells
+// when SUMS is set (pf2_step).
+//
+// A cell's output segment starts at an arbitrary position, so stores per cell
+// (a few lanes, 8 bytes each) do not cover whole cache lines and L2 fills
+// every line it writes from memory first.  A workgroup therefore takes
+// RegroupShape::CB consecutive cells, whose segments are one contiguous range,
+// and walks that range in order: each position finds its cell by bisection of
+// the offsets in LDS and its source in the cell's slot row (the census's
+// survivors in id order), or creates the new particle.  The records pass
+// through LDS on the way, where LPC lanes per cell add the projection sums in
+// ascending id order (accumulators in registers across the passes, so any
+// number of particles per cell), and no other pass reads them again.
+// Bound by HBM: 64 (80 with velocity_ext) bytes in and out per 2-D FP64
+// particle, 80-90% of a large copy's rate.  It takes the place of a map of the
+// positions, a gather by it, a pass of sums and its own bookkeeping launch:
+// per step 114 -> 86 us (FP64) and 76 -> 47 us (FP32) on 101,785 cells with
+// 2.4M particles, 576 -> 480 and 360 -> 274 on 407,140 with 11M.  One position
+// per thread and pass: two or four, for more loads in flight, cost registers
+// (98-124 us).
+//
 // New particles: reference point at the part centre, location mapped,
 // velocity interpolated from V (cylinder2D/pfem2particle.cpp:533-549), ids
 // continuing the counter in ascending cell, then part, order.
-// FP64 projection sums of one cell over n staged particles in order, the
-// expressions of k_cell_partials (accumulator a: vertex a / (DIM + 1),
-// component a % (DIM + 1), the last one the weight); NA accumulators a0,
-// a0 + GS, ... in one pass (their chains are independent, so they overlap)
-template <int DIM, int NA, int DEG = 1>
-__device__ __forceinline__ void cell_sums64(const double* __restrict__ sxi, const double* __restrict__ sv, int n,
-                                            int a0, double* out) {
-    constexpr int NACC = QF<DIM, DEG>::ND * (DIM + 1);
-    ShapeOne<DIM, DEG> sh[NA];
-    double acc[NA];
-    int comp[NA];
-#pragma unroll
-    for (int u = 0; u < NA; ++u) {
-        const int a = a0 + u * GS;
-        const int kk = (a < NACC ? a : 0) / (DIM + 1);
-        comp[u] = a - kk * (DIM + 1);
-        sh[u].init(kk);
-        acc[u] = 0.0;
-    }
-    for (int q = 0; q < n; ++q) {
-        double xi[DIM], v[DIM];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            xi[d] = sxi[q * DIM + d];
-            v[d] = sv[q * DIM + d];
-        }
-#pragma unroll
-        for (int u = 0; u < NA; ++u) {
-            const double nk = sh[u](xi);
-            if (comp[u] < DIM) {
-                double vc = v[0];
-#pragma unroll
-                for (int d = 1; d < DIM; ++d)
-                    if (d == comp[u]) vc = v[d];
-                acc[u] += nk * vc;
-            } else {
-                acc[u] += nk;
-            }
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < NA; ++u) out[u] = acc[u];
-}
+template <int DIM, int DEG>
+struct RegroupShape {
+    static constexpr int NACC = QF<DIM, DEG>::ND * (DIM + 1);   // sums per cell
+    // cells per workgroup: 16 (8 and 32 were 5-10% slower in 2-D), 32 of the
+    // few particles of a hexahedron (78 -> 68 us per FP32 step on 202,240)
+    static constexpr int CB = DIM == 3 && DEG == 1 ? 32 : 16;
+    static constexpr int LPC = 256 / CB;                        // lanes per cell in the sums
+    static constexpr int NA = (NACC + LPC - 1) / LPC;           // sums per lane
+};
 
-template <int DIM, bool GATHER, bool FUSE, int DEG = 1>
-__device__ __forceinline__ void cell_write_one(const DevMesh<DIM>& m, const double* __restrict__ V,
-                                               const int* __restrict__ old_off, const DevParticles& A,
-                                               const DevParticles& B, const DevParams& pp, const DevWork& w, int c,
-                                               int gl, double* __restrict__ sxi, double* __restrict__ sv,
-                                               double* __restrict__ partial) {
-    constexpr int NV = Q1<DIM>::NV;
-    constexpr int ND = QF<DIM, DEG>::ND;
-    const int n_st = old_off[c + 1] - old_off[c];
-    const int na = w.arr_cnt[c];
-    const int kin = n_st + (na < w.aslots ? na : w.aslots);
-    const unsigned long long fo = w.fs_off[c];
-    const long long out0 = (long long)(fo >> 32);
-    const int nsurv = w.nsurv[c];
-    const int nfinal = (int)(w.fs_cnt[c] >> 32);
-    if (gl == 0) w.new_off[c] = (int)out0;
-    if (out0 + nfinal > B.cap) {
-        if (gl == 0) atomicOr(&w.counters[2], 1);
-        return;
-    }
-    auto put = [&](int idx, int pos) {
-        const long long o = out0 + pos;
-        B.cell[o] = c;
-        B.id[o] = A.id[idx];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            const double xi = A.xi[(size_t)d * A.cap + idx], v = A.v[(size_t)d * A.cap + idx];
-            B.x[(size_t)d * B.cap + o] = A.x[(size_t)d * A.cap + idx];
-            B.xi[(size_t)d * B.cap + o] = xi;
-            B.v[(size_t)d * B.cap + o] = v;
-            if constexpr (FUSE) {
-                sxi[pos * DIM + d] = xi;
-                sv[pos * DIM + d] = v;
-            }
-        }
-        if (pp.keep_vext)
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) B.vext[(size_t)d * B.cap + o] = A.vext[(size_t)d * A.cap + idx];
-    };
-    if (nsurv <= w.aslots) {
-        // survivors listed in the slot row: WU of a lane's survivors per
-        // pass, all their loads issued before any store, so that a lane has
-        // several independent loads in flight
-        for (int t0 = 0; t0 < nsurv; t0 += GS * WU) {
-            int src[WU];
-#pragma unroll
-            for (int u = 0; u < WU; ++u) {
-                const int t = t0 + gl + u * GS;
-                src[u] = t < nsurv ? w.arr_slot[(size_t)c * w.aslots + t] : -1;
-            }
-            uint32_t pid[WU];
-            double px[WU][DIM], pxi[WU][DIM], pv[WU][DIM], pe[WU][DIM];
-#pragma unroll
-            for (int u = 0; u < WU; ++u) {
-                if (src[u] < 0) continue;
-                const int idx = src[u];
-                pid[u] = A.id[idx];
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) {
-                    px[u][d] = A.x[(size_t)d * A.cap + idx];
-                    pxi[u][d] = A.xi[(size_t)d * A.cap + idx];
-                    pv[u][d] = A.v[(size_t)d * A.cap + idx];
-                    pe[u][d] = pp.keep_vext ? A.vext[(size_t)d * A.cap + idx] : 0.0;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < WU; ++u) {
-                if (src[u] < 0) continue;
-                const int pos = t0 + gl + u * GS;
-                const long long o = out0 + pos;
-                B.cell[o] = c;
-                B.id[o] = pid[u];
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) {
-                    B.x[(size_t)d * B.cap + o] = px[u][d];
-                    B.xi[(size_t)d * B.cap + o] = pxi[u][d];
-                    B.v[(size_t)d * B.cap + o] = pv[u][d];
-                    if constexpr (FUSE) {
-                        sxi[pos * DIM + d] = pxi[u][d];
-                        sv[pos * DIM + d] = pv[u][d];
-                    }
-                }
-                if (pp.keep_vext)
-#pragma unroll
-                    for (int d = 0; d < DIM; ++d) B.vext[(size_t)d * B.cap + o] = pe[u][d];
-            }
-        }
-    } else {
-        survivors_of(w, old_off, c, n_st, kin, nsurv, gl, put);
-    }
-    const int spawns = nfinal - nsurv;
-    if (spawns > 0) {
-        const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
-        const unsigned long long empty = all & ~w.hitmask[c];
-        const uint32_t id0 = *w.particle_counter + (uint32_t)fo;
-        for (int o = gl; o < pp.nparts_in; o += GS) {
-            if (!((empty >> o) & 1)) continue;
-            const int r = __popcll(empty & ((1ull << o) - 1));
-            double xi[DIM], P[NV][DIM], Vc[ND][DIM], x[DIM], v[DIM];
-            lattice_point<DIM>(pp, o, xi);
-            load_cell<DIM, GATHER, DEG>(m, c, P, Vc);
-            forward<DIM>(P, xi, x);
-            interp<DIM, DEG>(Vc, xi, v);
-            const long long q = out0 + nsurv + r;
-            B.cell[q] = c;
-            B.id[q] = id0 + (uint32_t)r + 1u;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-                B.x[(size_t)d * B.cap + q] = x[d];
-                B.xi[(size_t)d * B.cap + q] = xi[d];
-                B.v[(size_t)d * B.cap + q] = v[d];
-                if constexpr (FUSE) {
-                    sxi[(nsurv + r) * DIM + d] = xi[d];
-                    sv[(nsurv + r) * DIM + d] = v[d];
-                }
-            }
-            if (pp.keep_vext)
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) B.vext[(size_t)d * B.cap + q] = 0.0;
-        }
-    }
-    if (gl == 0) {
-        w.arr_cnt[c] = 0;
-        w.ovf_head[c] = -1;
-    }
-    if constexpr (FUSE) {
-        constexpr int NACC = ND * (DIM + 1);
-        wave_sync();
-        // sums per lane: Q1 1 in 2-D (12 lanes), 2 in 3-D; Q2 2 in 2-D, 7 in 3-D
-        constexpr int NA = (NACC + GS - 1) / GS;
-        if (gl < NACC) {
-            double out[NA];
-            cell_sums64<DIM, NA, DEG>(sxi, sv, nfinal, gl, out);
-#pragma unroll
-            for (int u = 0; u < NA; ++u)
-                if (gl + u * GS < NACC) partial[(size_t)c * NACC + gl + u * GS] = out[u];
-        }
-        wave_sync();
-    }
-}
+// a workgroup's cells in LDS
+template <int CB>
+struct RegroupCells {
+    long long base;                  // first output position
+    int off[CB + 1];                 // each cell's first position after it, then the end
+    int nsurv[CB];
+    unsigned long long empty[CB];    // parts to reseed
+    uint32_t spawn0[CB];             // new particles of earlier cells
+};
 
-// GATHER: an FP32-mixed handle's FP64 regroup (no FP64 per-cell velocity copy).
-// FUSE (final count per cell <= FCAP): the group stages the cell's final
-// particles in LDS and writes its projection sums, as k_cell_partials does.
-template <int DIM, bool GATHER, bool FUSE, int DEG = 1>
-__device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM>& m, const double* __restrict__ V, const int* __restrict__ old_off, const DevParticles& A, const DevParticles& B, const DevParams& pp, const DevWork& w, double* __restrict__ partial) {
-    __shared__ double s_xi[FUSE ? GROUPS : 1][FUSE ? FCAP * DIM : 1];
-    __shared__ double s_v[FUSE ? GROUPS : 1][FUSE ? FCAP * DIM : 1];
-    if (state_dead(w.counters)) return;
-    const int g = threadIdx.x / GS, gl = threadIdx.x % GS;
-    for (int c = G.bid * GROUPS + g; c < m.n_cells; c += G.nblk * GROUPS)
-        cell_write_one<DIM, GATHER, FUSE, DEG>(m, V, old_off, A, B, pp, w, c, gl, s_xi[FUSE ? g : 0],
-                                               s_v[FUSE ? g : 0], partial);
-}
-
-template <int DIM, bool GATHER, bool FUSE, int DEG = 1>
-__global__ void __launch_bounds__(256) k_cell_write(DevMesh<DIM> m, const double* __restrict__ V,
-                                                    const int* __restrict__ old_off, DevParticles A,
-                                                    DevParticles B, DevParams pp, DevWork w,
-                                                    double* __restrict__ partial) {
-    cell_write_body<DIM, GATHER, FUSE, DEG>(hw_grid(), m, V, old_off, A, B, pp, w, partial);
-}
-
-// ---------------------------------------------------------------------------
-// The regroup write in two passes (regroups without fused projection sums).
-// A cell's output segment starts at an arbitrary position, so the stores of
-// k_cell_write's 16-lane groups never cover a whole cache line and L2 fills
-// every line it writes from memory first (the write volume again in reads).
-// k_cell_map does the per-cell work (offsets, survivors, spawn slots,
-// resets) and writes one int per output position: the source particle, or
-// for a new particle -1 - (cell * 64 + lattice ordinal).  k_cell_gather then
-// walks the output positions in order and copies or creates each particle,
-// so every wavefront stores whole, consecutive lines.  Cell indices below
-// 2^25 (the map's encoding), which the host checks.
-template <int DIM>
-__device__ __forceinline__ void cell_map_body(const Grid& G, int n_cells, const int* __restrict__ old_off,
+// Fills s for the cells cb, cb + 1, ... (all threads call; a barrier at the
+// end): offsets, overflow flag, and for cells whose survivors outnumber the
+// slot row (rare) their sources in omap.
+template <int CB>
+__device__ __forceinline__ void regroup_cells(RegroupCells<CB>& s, int cb, int nc, const int* __restrict__ old_off,
                                               long long cap, const DevParams& pp, const DevWork& w,
                                               int* __restrict__ omap) {
-    if (state_dead(w.counters)) return;
-    const int g = threadIdx.x / GS, gl = threadIdx.x % GS;
-    for (int c = G.bid * GROUPS + g; c < n_cells; c += G.nblk * GROUPS) {
-        const int n_st = old_off[c + 1] - old_off[c];
-        const int na = w.arr_cnt[c];
-        const int kin = n_st + (na < w.aslots ? na : w.aslots);
+    constexpr int LPC = 256 / CB;
+    static_assert(CB <= WAVE && (CB & (CB - 1)) == 0, "one wavefront loads the cells, bisection over them");
+    const int t = threadIdx.x;
+    const int last = nc - cb < CB ? nc - cb : CB;
+    bool past = false;
+    if (t < CB) {
+        const int c = cb + (t < last ? t : last - 1);
         const unsigned long long fo = w.fs_off[c];
-        const long long out0 = (long long)(fo >> 32);
-        const int nsurv = w.nsurv[c];
         const int nfinal = (int)(w.fs_cnt[c] >> 32);
-        if (gl == 0) w.new_off[c] = (int)out0;
-        if (out0 + nfinal > cap) {
-            if (gl == 0) atomicOr(&w.counters[2], 1);
-            continue;
+        const long long out0 = (long long)(fo >> 32), b0 = __shfl(out0, 0);
+        const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
+        if (t == 0) s.base = out0;
+        s.off[t] = (int)(out0 - b0) + (t < last ? 0 : nfinal);
+        if (t == CB - 1) s.off[CB] = (int)(out0 - b0) + nfinal;
+        s.nsurv[t] = w.nsurv[c];
+        s.empty[t] = all & ~w.hitmask[c];
+        s.spawn0[t] = (uint32_t)fo;
+        if (t < last) {
+            w.new_off[c] = (int)out0;
+            past = w.nsurv[c] > w.aslots;
+            if (out0 + nfinal > cap) atomicOr(&w.counters[2], 1);
         }
-        if (nsurv <= w.aslots) {
-            for (int t = gl; t < nsurv; t += GS) omap[out0 + t] = w.arr_slot[(size_t)c * w.aslots + t];
-        } else {
-            survivors_of(w, old_off, c, n_st, kin, nsurv, gl, [&](int idx, int pos) { omap[out0 + pos] = idx; });
-        }
-        if (nfinal > nsurv) {
-            const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
-            const unsigned long long empty = all & ~w.hitmask[c];
-            for (int o = gl; o < pp.nparts_in; o += GS) {
-                if (!((empty >> o) & 1)) continue;
-                const int r = __popcll(empty & ((1ull << o) - 1));
-                omap[out0 + nsurv + r] = -1 - (c * 64 + o);
+    }
+    if (__syncthreads_or(past)) {
+        const int g = t / LPC, gl = t % LPC, c = cb + g;
+        if (g < last && s.nsurv[g] > w.aslots) {
+            const int n_st = old_off[c + 1] - old_off[c], na = w.arr_cnt[c];
+            const long long out0 = s.base + s.off[g];
+            auto put = [&](int idx) {
+                const int pos = w.spos[idx];
+                if (pos >= 0 && out0 + pos < cap) omap[out0 + pos] = idx;
+            };
+            const int kin = n_st + (na < w.aslots ? na : w.aslots);
+            for (int j = gl; j < kin; j += LPC) {
+                const int idx = candidate(w, old_off, c, n_st, j);
+                // arrivals are in this cell's slots because their destination is c
+                if (j >= n_st || w.dest[idx] == c) put(idx);
             }
+            for_overflow(w, c, gl, LPC, [&](int, int idx) { put(idx); });
         }
-        if (gl == 0) {
-            w.arr_cnt[c] = 0;
-            w.ovf_head[c] = -1;
-        }
+        __syncthreads();
+    }
+    // (the arrival lists of the cells have been read)
+    if (t < last) {
+        w.arr_cnt[cb + t] = 0;
+        w.ovf_head[cb + t] = -1;
     }
 }
 
-template <int DIM>
-__global__ void __launch_bounds__(256) k_cell_map(int n_cells, const int* __restrict__ old_off, long long cap,
-                                                  DevParams pp, DevWork w, int* __restrict__ omap) {
-    cell_map_body<DIM>(hw_grid(), n_cells, old_off, cap, pp, w, omap);
+// source of the output position p after s.base: a particle, or for a new one
+// -1 - its lattice ordinal; k is its cell within the workgroup's
+template <int CB>
+__device__ __forceinline__ int regroup_source(const RegroupCells<CB>& s, int cb, int p, const DevWork& w,
+                                              const int* __restrict__ omap, int& k) {
+    k = 0;
+#pragma unroll
+    for (int h = CB / 2; h > 0; h >>= 1)
+        if (s.off[k + h] <= p) k += h;
+    const int t = p - s.off[k], ns = s.nsurv[k];
+    if (t < ns) return ns <= w.aslots ? w.arr_slot[(size_t)(cb + k) * w.aslots + t] : omap[s.base + p];
+    unsigned long long e = s.empty[k];
+    for (int r = t - ns; r > 0; --r) e &= e - 1;
+    return -__ffsll((long long)e);
 }
 
-constexpr int GU = 4;   // output positions per thread and pass of the regroup gather
-
-// a new particle at output position o: code = cell * 64 + lattice ordinal
-template <int DIM, bool GATHER, int DEG>
-__device__ __forceinline__ void gather_spawn(const DevMesh<DIM>& m, const DevParticles& B, const DevParams& pp,
-                                             const DevWork& w, long long o, int code) {
+// GATHER: velocities of new particles through the DoF map (FP32-mixed handles,
+// or stale per-cell copies)
+template <int DIM, bool GATHER, bool SUMS, int DEG>
+__device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM>& m, const int* __restrict__ old_off,
+                                                const DevParticles& A, const DevParticles& B, const DevParams& pp,
+                                                const DevWork& w, int* __restrict__ omap,
+                                                double* __restrict__ partial) {
+    using S = RegroupShape<DIM, DEG>;
     constexpr int NV = Q1<DIM>::NV;
     constexpr int ND = QF<DIM, DEG>::ND;
-    const int c = code >> 6, lo = code & 63;
-    const unsigned long long fo = w.fs_off[c];
-    const int r = (int)(o - (long long)(fo >> 32)) - w.nsurv[c];
-    double xi[DIM], P[NV][DIM], Vc[ND][DIM], x[DIM], v[DIM];
-    lattice_point<DIM>(pp, lo, xi);
-    load_cell<DIM, GATHER, DEG>(m, c, P, Vc);
-    forward<DIM>(P, xi, x);
-    interp<DIM, DEG>(Vc, xi, v);
-    B.cell[o] = c;
-    B.id[o] = *w.particle_counter + (uint32_t)fo + (uint32_t)r + 1u;
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-        B.x[(size_t)d * B.cap + o] = x[d];
-        B.xi[(size_t)d * B.cap + o] = xi[d];
-        B.v[(size_t)d * B.cap + o] = v[d];
-        if (pp.keep_vext) B.vext[(size_t)d * B.cap + o] = 0.0;
-    }
-}
-
-// one output position per lane and slice, GU slices of the workgroup's
-// positions per pass, all loads of a pass issued before its stores: a
-// survivor's record is copied (its cell is its destination), a new particle
-// is created at its lattice point as k_cell_write creates it (id after the
-// cell's spawn offset, velocity interpolated from the cell's DoFs,
-// velocity_ext zero)
-template <int DIM, bool GATHER, int DEG = 1>
-__device__ __forceinline__ void cell_gather_body(const Grid& G, const DevMesh<DIM>& m, const DevParticles& A,
-                                                 const DevParticles& B, const DevParams& pp, const DevWork& w,
-                                                 const int* __restrict__ omap) {
+    constexpr int CH = 256;   // positions per pass
+    __shared__ RegroupCells<S::CB> s;
+    __shared__ double s_xi[SUMS ? DIM : 1][SUMS ? CH : 1];
+    __shared__ double s_v[SUMS ? DIM : 1][SUMS ? CH : 1];
     if (state_dead(w.counters)) return;
-    const long long total = (long long)(w.fs_off[m.n_cells] >> 32);
-    const long long n = total < B.cap ? total : B.cap;
-    const long long bd = blockDim.x, span = (long long)G.nblk * bd * GU;
-    for (long long o0 = (long long)G.bid * bd * GU + threadIdx.x; o0 < n; o0 += span) {
-        int src[GU];
-        bool act[GU];
+    const int tid = threadIdx.x, g = tid / S::LPC, gl = tid % S::LPC;
+    // the lane's sums: vertex a / (DIM + 1), component a % (DIM + 1) (the last
+    // one the weight) for a = gl, gl + LPC, ...
+    ShapeOne<DIM, DEG> sh[S::NA];
+    int comp[S::NA];
+    if constexpr (SUMS)
 #pragma unroll
-        for (int u = 0; u < GU; ++u) {
-            const long long o = o0 + u * bd;
-            act[u] = o < n;
-            src[u] = act[u] ? omap[o] : -1;
+        for (int u = 0; u < S::NA; ++u) {
+            const int a = gl + u * S::LPC;
+            const int kk = (a < S::NACC ? a : 0) / (DIM + 1);
+            comp[u] = a - kk * (DIM + 1);
+            sh[u].init(kk);
         }
-        int pc[GU];
-        uint32_t pid[GU];
-        double px[GU][DIM], pxi[GU][DIM], pv[GU][DIM], pe[GU][DIM];
+    for (int cb = G.bid * S::CB; cb < m.n_cells; cb += G.nblk * S::CB) {
+        regroup_cells<S::CB>(s, cb, m.n_cells, old_off, A.cap, pp, w, omap);
+        const long long base = s.base;
+        const int total = base + s.off[S::CB] <= B.cap ? s.off[S::CB] : (int)(B.cap > base ? B.cap - base : 0);
+        double acc[S::NA];
 #pragma unroll
-        for (int u = 0; u < GU; ++u) {
-            if (!act[u] || src[u] < 0) continue;
-            const int s = src[u];
-            pc[u] = w.dest[s];
-            pid[u] = A.id[s];
+        for (int u = 0; u < S::NA; ++u) acc[u] = 0.0;
+        for (int p0 = 0; p0 < total; p0 += CH) {
+            const int p = p0 + tid;
+            if (p < total) {
+                int k;
+                const int src = regroup_source<S::CB>(s, cb, p, w, omap, k);
+                const int c = cb + k;
+                uint32_t id = 0;
+                double x[DIM], xi[DIM], v[DIM], e[DIM];
+                if (src >= 0) {
+                    id = A.id[src];
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-                px[u][d] = A.x[(size_t)d * A.cap + s];
-                pxi[u][d] = A.xi[(size_t)d * A.cap + s];
-                pv[u][d] = A.v[(size_t)d * A.cap + s];
-                pe[u][d] = pp.keep_vext ? A.vext[(size_t)d * A.cap + s] : 0.0;
+                    for (int d = 0; d < DIM; ++d) {
+                        x[d] = A.x[(size_t)d * A.cap + src];
+                        xi[d] = A.xi[(size_t)d * A.cap + src];
+                        v[d] = A.v[(size_t)d * A.cap + src];
+                        e[d] = pp.keep_vext ? A.vext[(size_t)d * A.cap + src] : 0.0;
+                    }
+                }
+                // a new particle: most wavefronts hold one or two, so its
+                // loads go out behind the records' and before any wait
+                if (src < 0) {
+                    double P[NV][DIM], Vc[ND][DIM];
+                    load_cell<DIM, GATHER, DEG>(m, c, P, Vc);
+                    id = *w.particle_counter + s.spawn0[k] + (uint32_t)(p - s.off[k] - s.nsurv[k]) + 1u;
+                    lattice_point<DIM>(pp, -1 - src, xi);
+                    forward<DIM>(P, xi, x);
+                    interp<DIM, DEG>(Vc, xi, v);
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) e[d] = 0.0;
+                }
+                const long long o = base + p;
+                B.cell[o] = c;
+                B.id[o] = id;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) {
+                    B.x[(size_t)d * B.cap + o] = x[d];
+                    B.xi[(size_t)d * B.cap + o] = xi[d];
+                    B.v[(size_t)d * B.cap + o] = v[d];
+                    if (pp.keep_vext) B.vext[(size_t)d * B.cap + o] = e[d];
+                    if constexpr (SUMS) {
+                        s_xi[d][tid] = xi[d];
+                        s_v[d][tid] = v[d];
+                    }
+                }
+            }
+            if constexpr (SUMS) {
+                __syncthreads();
+                const int q0 = s.off[g] > p0 ? s.off[g] - p0 : 0;
+                const int e = s.off[g + 1] < total ? s.off[g + 1] : total;
+                const int q1 = e - p0 < CH ? e - p0 : CH;
+                for (int q = q0; q < q1; ++q) {
+                    double xi[DIM], v[DIM];
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) {
+                        xi[d] = s_xi[d][q];
+                        v[d] = s_v[d][q];
+                    }
+#pragma unroll
+                    for (int u = 0; u < S::NA; ++u) {
+                        double vc = 1.0;   // the weight term is N_k itself
+#pragma unroll
+                        for (int d = 0; d < DIM; ++d)
+                            if (d == comp[u]) vc = v[d];
+                        acc[u] += sh[u](xi) * vc;
+                    }
+                }
+                __syncthreads();
             }
         }
+        if constexpr (SUMS)
+            if (cb + g < m.n_cells)
 #pragma unroll
-        for (int u = 0; u < GU; ++u) {
-            if (!act[u]) continue;
-            const long long o = o0 + u * bd;
-            if (src[u] < 0) {
-                gather_spawn<DIM, GATHER, DEG>(m, B, pp, w, o, -1 - src[u]);
-                continue;
-            }
-            B.cell[o] = pc[u];
-            B.id[o] = pid[u];
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-                B.x[(size_t)d * B.cap + o] = px[u][d];
-                B.xi[(size_t)d * B.cap + o] = pxi[u][d];
-                B.v[(size_t)d * B.cap + o] = pv[u][d];
-                if (pp.keep_vext) B.vext[(size_t)d * B.cap + o] = pe[u][d];
-            }
-        }
+                for (int u = 0; u < S::NA; ++u)
+                    if (gl + u * S::LPC < S::NACC) partial[(size_t)(cb + g) * S::NACC + gl + u * S::LPC] = acc[u];
+        __syncthreads();   // s is refilled
     }
 }
 
-template <int DIM, bool GATHER, int DEG = 1>
-__global__ void __launch_bounds__(256) k_cell_gather(DevMesh<DIM> m, DevParticles A, DevParticles B, DevParams pp,
-                                                     DevWork w, const int* __restrict__ omap) {
-    cell_gather_body<DIM, GATHER, DEG>(hw_grid(), m, A, B, pp, w, omap);
+template <int DIM, bool GATHER, bool SUMS, int DEG>
+__global__ void __launch_bounds__(256) k_cell_write(DevMesh<DIM> m, const int* __restrict__ old_off, DevParticles A,
+                                                    DevParticles B, DevParams pp, DevWork w, int* __restrict__ omap,
+                                                    double* __restrict__ partial) {
+    cell_write_body<DIM, GATHER, SUMS, DEG>(hw_grid(), m, old_off, A, B, pp, w, omap, partial);
 }
 
 // totals after the scans: particle count, id counter, statistics; resets the
@@ -1930,7 +1779,7 @@ __global__ void __launch_bounds__(QSHARDS) k_finalize(int n_cells, DevWork w, in
 // particles are not moved into a new buffer: the census's survivors are
 // marked in place (destination = cell | DEST_KEPT), its
 // new particles are created after the current segments (position seg_end +
-// the cell's spawn offset + rank, ids and values as k_cell_gather creates
+// the cell's spawn offset + rank, ids and values as k_cell_write creates
 // them), and counters[6], [7] record the slots and seg_end.  The next move
 // takes a particle's cell from dest, skips the unmarked ones and makes the
 // new ones arrive in their cell, so its census regroups the pending layout

@@ -40,7 +40,8 @@ int fail(int code, const std::string& msg) {
     } while (0)
 
 // Timing ids of pf2_kernel_times / pf2_kernel_name.  The ids of kernels that
-// no longer exist (K_GROUP, K_QPREFIX) stay reserved, so that a caller's
+// no longer exist (K_GROUP, K_QPREFIX, K_CELL_MAP, K_CELL_GATHER,
+// K_CELL_GATHER32) stay reserved, so that a caller's
 // numbering does not shift; they report no launches.
 enum KernelId {
     K_MOVE = 0, K_GROUP, K_CELL_COUNT, K_CELL_WRITE, K_SCAN, K_FINALIZE, K_PARTIALS, K_NODE, K_WALL,
@@ -142,7 +143,7 @@ struct pf2_handle_s {
     int cur_off = 0;
     // work
     int *dest = nullptr, *pkey = nullptr, *spos = nullptr;
-    int* omap = nullptr;   // regroup output map (k_cell_map -> k_cell_gather)
+    int* omap = nullptr;   // sources of the cells whose survivors outnumber the slot row (k_cell_write)
     unsigned char* dcmoved = nullptr;   // per cell: the last geometry update changed it
     int geo_updates = 0;                // geometry updates since the last re-sort
     int *arr_cnt = nullptr, *arr_slot = nullptr, *ovf_head = nullptr;
@@ -251,13 +252,6 @@ int cell_grid(int n_cells, int cap = 4096) {
 
 int pack_fields(pf2_handle_s* h);
 int ensure_packed(pf2_handle_s* h);
-
-// bound of the per-cell particle count after a census with reseed
-long long fuse_bound(const pf2_handle_s* h) {
-    long long b = h->params.max_per_part;
-    for (int d = 0; d < h->dim; ++d) b *= h->params.quantities[d] + 1;
-    return b;
-}
 
 // search grid per round: the first round sees most parked particles; later
 // rounds see fewer, the last one loops every remaining particle to the end
@@ -559,79 +553,34 @@ int regroup(pf2_handle_s* h, int reseed, bool fuse_sums = false, bool defer_fina
         h->pending = true;
         return 0;
     }
-    const bool two_pass = !fuse_sums && h->omap && nc < (1 << 25);
-    // the one-pass write of an FP64 handle reads the per-cell copies of V
-    if (!two_pass && !mixed(h))
-        if (int r = ensure_packed(h)) return r;
-    if (two_pass) {
-        // per-cell map, then the output positions in order (pf2_kernels.hpp)
-        Timed t(h, K_CELL_MAP);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_map<DIM>), dim3(cell_grid(nc)), dim3(256), 0, h->stream, nc,
-                           old_off, h->cap, pp, w, h->omap);
-    }
-    if (mixed(h) && !fp64_state && two_pass) {
-        Timed t(h, K_CELL_GATHER32);
-        const dim3 g(grid_for(h->n_est, 256 * GU, 65535));   // one pass of GU positions per thread
-        const PBufs &a = h->buf[h->cur], &b = h->buf[1 - h->cur];
-        if (h->deg == 2)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_gather32<DIM, 2>), g, dim3(256), 0, h->stream, dev_mesh<DIM>(h),
-                               h->dV32, a.id, rec32(a), b.cell, b.id, rec32(b), a.vext, b.vext, h->cap, pp, w, h->omap);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_gather32<DIM>), g, dim3(256), 0, h->stream, dev_mesh<DIM>(h),
-                               h->dV32, a.id, rec32(a), b.cell, b.id, rec32(b), a.vext, b.vext, h->cap, pp, w, h->omap);
-    } else if (mixed(h) && !fp64_state) {
+    // one workgroup per RegroupShape::CB cells
+    const int cb = h->deg == 2 ? RegroupShape<DIM, 2>::CB : RegroupShape<DIM, 1>::CB;
+    const dim3 g((nc + cb - 1) / cb);
+    if (mixed(h) && !fp64_state) {
         Timed t(h, K_CELL_WRITE32);
-        launch_cell_write32<DIM>(h->stream, cell_grid(nc), dev_mesh<DIM>(h), h->dV32, old_off, h->buf[h->cur].id,
-                                 rec32(h->buf[h->cur]), h->buf[1 - h->cur].cell, h->buf[1 - h->cur].id,
-                                 rec32(h->buf[1 - h->cur]), h->buf[h->cur].vext, h->buf[1 - h->cur].vext, h->cap, pp,
-                                 w, fuse_sums, h->partial, h->deg);
-    } else if (two_pass) {
-        Timed t(h, K_CELL_GATHER);
-        const dim3 g(grid_for(h->n_est, 256 * GU, 65535));   // one pass of GU positions per thread
-        DevParticles a = dev_particles(h, h->cur), b = dev_particles(h, 1 - h->cur);
-        // (an FP32-mixed handle's FP64 regroup, and a regroup after a
-        // projection left the per-cell copies stale, gather V through the
-        // DoF map: the same values)
-        const bool gather_v = !h->dcellV || !h->packed;
-        if (gather_v && h->deg == 2)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_gather<DIM, true, 2>), g, dim3(256), 0, h->stream,
-                               dev_mesh<DIM>(h), a, b, pp, w, h->omap);
-        else if (gather_v)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_gather<DIM, true>), g, dim3(256), 0, h->stream,
-                               dev_mesh<DIM>(h), a, b, pp, w, h->omap);
-        else if (h->deg == 2)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_gather<DIM, false, 2>), g, dim3(256), 0, h->stream,
-                               dev_mesh<DIM>(h), a, b, pp, w, h->omap);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_gather<DIM, false>), g, dim3(256), 0, h->stream,
-                               dev_mesh<DIM>(h), a, b, pp, w, h->omap);
+        const PBufs &a = h->buf[h->cur], &b = h->buf[1 - h->cur];
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, g, dim3(256), 0, h->stream, nc, h->dV32, old_off, a.id, rec32(a), b.cell, b.id,
+                               rec32(b), a.vext, b.vext, h->cap, pp, w, h->omap, h->partial);
+        };
+        if (h->deg == 2) fuse_sums ? launch(k_cell_write32<DIM, true, 2>) : launch(k_cell_write32<DIM, false, 2>);
+        else fuse_sums ? launch(k_cell_write32<DIM, true, 1>) : launch(k_cell_write32<DIM, false, 1>);
     } else {
         Timed t(h, K_CELL_WRITE);
-        // (an FP32-mixed handle's FP64 regroup gathers V and never fuses)
-        if (!h->dcellV && h->deg == 2)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write<DIM, true, false, 2>), dim3(cell_grid(nc)), dim3(256), 0,
-                               h->stream, dev_mesh<DIM>(h), h->dV, old_off, dev_particles(h, h->cur),
-                               dev_particles(h, 1 - h->cur), pp, w, h->partial);
-        else if (!h->dcellV)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write<DIM, true, false>), dim3(cell_grid(nc)), dim3(256), 0,
-                               h->stream, dev_mesh<DIM>(h), h->dV, old_off, dev_particles(h, h->cur),
-                               dev_particles(h, 1 - h->cur), pp, w, h->partial);
-        else if (fuse_sums && h->deg == 2)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write<DIM, false, true, 2>), dim3(cell_grid(nc)), dim3(256), 0,
-                               h->stream, dev_mesh<DIM>(h), h->dV, old_off, dev_particles(h, h->cur),
-                               dev_particles(h, 1 - h->cur), pp, w, h->partial);
-        else if (fuse_sums)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write<DIM, false, true>), dim3(cell_grid(nc)), dim3(256), 0,
-                               h->stream, dev_mesh<DIM>(h), h->dV, old_off, dev_particles(h, h->cur),
-                               dev_particles(h, 1 - h->cur), pp, w, h->partial);
+        // (an FP32-mixed handle's FP64 regroup, and a regroup after a
+        // projection left the per-cell copies stale, gather V through the
+        // DoF map: the same values; neither takes the sums)
+        const bool gather_v = !h->dcellV || !h->packed;
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, g, dim3(256), 0, h->stream, dev_mesh<DIM>(h), old_off, dev_particles(h, h->cur),
+                               dev_particles(h, 1 - h->cur), pp, w, h->omap, h->partial);
+        };
+        if (gather_v)
+            h->deg == 2 ? launch(k_cell_write<DIM, true, false, 2>) : launch(k_cell_write<DIM, true, false, 1>);
         else if (h->deg == 2)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write<DIM, false, false, 2>), dim3(cell_grid(nc)), dim3(256), 0,
-                               h->stream, dev_mesh<DIM>(h), h->dV, old_off, dev_particles(h, h->cur),
-                               dev_particles(h, 1 - h->cur), pp, w, h->partial);
+            fuse_sums ? launch(k_cell_write<DIM, false, true, 2>) : launch(k_cell_write<DIM, false, false, 2>);
         else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write<DIM, false, false>), dim3(cell_grid(nc)), dim3(256), 0,
-                               h->stream, dev_mesh<DIM>(h), h->dV, old_off, dev_particles(h, h->cur),
-                               dev_particles(h, 1 - h->cur), pp, w, h->partial);
+            fuse_sums ? launch(k_cell_write<DIM, false, true, 1>) : launch(k_cell_write<DIM, false, false, 1>);
     }
     if (!defer_finalize) {
         Timed t(h, K_FINALIZE);
@@ -756,8 +705,7 @@ int run_project(pf2_handle_s* h, bool sums_done = false, double* partial = nullp
     if (!partial) partial = h->partial;
     w.partial = partial;
     if (sums_done) {
-        // the projection sums came with the regroup (k_cell_write<DIM, false, true>,
-        // k_cell_write32<DIM, true>)
+        // the projection sums came with the regroup write
     } else if (mixed(h)) {
         Timed t(h, K_PARTIALS32);
         launch_partials32<DIM>(h->stream, cell_grid(nc), nc, h->off[h->cur_off], rec32(h->buf[h->cur]), partial,
@@ -983,11 +931,9 @@ int step_body(pf2_handle_s* h, const double* field) {
         Timed t(h, K_MISC);
         if (int r = pack_fields(h)) return r;
     }
-    // steps whose per-cell final count is bounded by the LDS rows compute
-    // the projection sums while regrouping
-    const bool fuse = fuse_bound(h) <= FCAP;
-    if (int r = (h->dim == 2 ? run_move<2>(h, 1, 1, fuse) : run_move<3>(h, 1, 1, fuse))) return r;
-    return h->dim == 2 ? run_project<2>(h, fuse) : run_project<3>(h, fuse);
+    // the projection sums come with the regroup write
+    if (int r = (h->dim == 2 ? run_move<2>(h, 1, 1, true) : run_move<3>(h, 1, 1, true))) return r;
+    return h->dim == 2 ? run_project<2>(h, true) : run_project<3>(h, true);
 }
 
 // the step as a HIP graph: captured once per buffer parity, replayed after.
@@ -1090,6 +1036,7 @@ void batch_fill(pf2_handle_s* h, const double* field, BatchSim<DIM>& S, int* gri
     S.dV32 = h->dVold32;
     S.geo = h->dgeo32;
     S.partial = h->partial;
+    S.omap = h->omap;
     S.qcount = h->qcount;
     S.tiles = h->scan_tiles;
     const int nc = h->n_cells;
@@ -1106,8 +1053,7 @@ void batch_fill(pf2_handle_s* h, const double* field, BatchSim<DIM>& S, int* gri
     grid[BK_COUNT_L] = small ? 0 : cell_grid(nc, 8192);
     grid[BK_BIG] = 32;
     grid[BK_TILES] = S.ntiles;
-    grid[BK_WRITE] = cell_grid(nc);
-    grid[BK_PARTIALS] = cell_grid(nc);
+    grid[BK_WRITE] = (nc + RegroupShape<DIM, 1>::CB - 1) / RegroupShape<DIM, 1>::CB;
     grid[BK_NODE] = grid_for(h->n_dofs, 256);
 }
 
@@ -1164,8 +1110,6 @@ int batch_step(pf2_batch_s* b, int n, const pf2_handle* hs, const double* const*
     if (mx) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_write32<DIM>), dim3(tot[BK_WRITE]), dim3(256), 0, st, bv);
     else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_write<DIM>), dim3(tot[BK_WRITE]), dim3(256), 0, st, bv);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_finalize<DIM>), dim3(n), dim3(QSHARDS), 0, st, bv);
-    if (mx) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_partials32<DIM>), dim3(tot[BK_PARTIALS]), dim3(256), 0, st, bv);
-    else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_partials<DIM>), dim3(tot[BK_PARTIALS]), dim3(256), 0, st, bv);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_node<DIM>), dim3(tot[BK_NODE]), dim3(256), 0, st, bv);
     HIPC(hipGetLastError());
     // every simulation's later work after the batch

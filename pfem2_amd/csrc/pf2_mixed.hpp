@@ -742,313 +742,146 @@ void launch_search_resume32(hipStream_t s, int grid, DevMesh<DIM> m, const float
                            pcell, R, pvext, cap, pp, w, qu, round);
 }
 
-// rows of the fused projection sums (FCAP, pf2_kernels.hpp): a cell's final
-// particles (records; in 3-D the second part of each record in a row of its
-// own)
-
-// Kahan-compensated FP32 projection sums of one cell over n staged records
-// in order (accumulator a < NACC: vertex a / (DIM + 1), component a % (DIM +
-// 1), the last one the weight), as k_cell_partials32 computes them
-template <int DIM, int NA, int DEG = 1>
-__device__ __forceinline__ void cell_sums32(const float4* __restrict__ rec, const float2* __restrict__ recb, int n,
-                                            int a0, double* out) {
-    // NA accumulators a0, a0 + GS, ... in one pass over the records (their
-    // Kahan chains are independent, so they overlap); accumulators past
-    // NACC are computed for node 0 and not stored by the caller
-    constexpr int NACC = QF<DIM, DEG>::ND * (DIM + 1);
-    ShapeOne32<DIM, DEG> sh[NA];
-    float sum[NA], cmp[NA];
-    int comp[NA];
-#pragma unroll
-    for (int u = 0; u < NA; ++u) {
-        const int a = a0 + u * GS;
-        const int kk = (a < NACC ? a : 0) / (DIM + 1);
-        comp[u] = a - kk * (DIM + 1);
-        sh[u].init(kk);
-        sum[u] = 0.0f;
-        cmp[u] = 0.0f;
-    }
-    for (int q = 0; q < n; ++q) {
-        const float4 r = rec[q];
-        float xi[DIM], v[DIM];
-        if constexpr (DIM == 2) {
-            xi[0] = r.x;
-            xi[1] = r.y;
-            v[0] = r.z;
-            v[1] = r.w;
-        } else {
-            const float2 rb = recb[q];
-            xi[0] = r.x;
-            xi[1] = r.y;
-            xi[2] = r.z;
-            v[0] = r.w;
-            v[1] = rb.x;
-            v[2] = rb.y;
-        }
-#pragma unroll
-        for (int u = 0; u < NA; ++u) {
-            const float nk = sh[u](xi);
-            float vc = 1.0f;   // the weight term (comp == DIM) is N_k itself
-#pragma unroll
-            for (int d = 0; d < DIM; ++d)
-                if (d == comp[u]) vc = v[d];
-            const float term = nk * vc;
-            const float y = term - cmp[u];
-            const float tt = sum[u] + y;
-            cmp[u] = (tt - sum[u]) - y;
-            sum[u] = tt;
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < NA; ++u) out[u] = (double)sum[u] - (double)cmp[u];
-}
-
-// FUSE (final count per cell <= FCAP): the group also stages the cell's
-// final records in LDS and writes its projection sums, so no separate
-// partials pass re-reads the particles (3-D: each lane of the group owns two
-// of the 32 sums)
-template <int DIM, bool FUSE, int DEG = 1>
-__device__ __forceinline__ void cell_write32_one(const DevMesh<DIM>& m, const float* __restrict__ V32c,
-                                                 const int* __restrict__ old_off, const uint32_t* __restrict__ aid,
-                                                 const Rec32& A, int* __restrict__ bcell, uint32_t* __restrict__ bid,
-                                                 const Rec32& B, const double* __restrict__ avext,
-                                                 double* __restrict__ bvext, long long cap, const DevParams& pp,
-                                                 const DevWork& w, int c, int gl, float4* __restrict__ srec,
-                                                 float2* __restrict__ srecb, double* __restrict__ partial) {
+// k_cell_write (pf2_kernels.hpp) for FP32 records: the sums in FP32 with Kahan
+// compensation, new particles' velocities from the cell's FP32 copy of V (this
+// handle keeps no FP64 per-cell copy), interpolated in FP64.
+template <int DIM, bool SUMS, int DEG>
+__device__ __forceinline__ void cell_write32_body(const Grid& G, int n_cells, const float* __restrict__ V32c,
+                                                  const int* __restrict__ old_off, const uint32_t* __restrict__ aid,
+                                                  const Rec32& A, int* __restrict__ bcell,
+                                                  uint32_t* __restrict__ bid, const Rec32& B,
+                                                  const double* __restrict__ avext, double* __restrict__ bvext,
+                                                  long long cap, const DevParams& pp, const DevWork& w,
+                                                  int* __restrict__ omap, double* __restrict__ partial) {
+    using S = RegroupShape<DIM, DEG>;
     constexpr int ND = QF<DIM, DEG>::ND;
-    const int n_st = old_off[c + 1] - old_off[c];
-    const int na = w.arr_cnt[c];
-    const int kin = n_st + (na < w.aslots ? na : w.aslots);
-    const unsigned long long fo = w.fs_off[c];
-    const long long out0 = (long long)(fo >> 32);
-    const int nsurv = w.nsurv[c];
-    const int nfinal = (int)(w.fs_cnt[c] >> 32);
-    if (gl == 0) w.new_off[c] = (int)out0;
-    if (out0 + nfinal > cap) {
-        if (gl == 0) atomicOr(&w.counters[2], 1);
-        return;
-    }
-    auto put = [&](int idx, int pos) {
-        const long long o = out0 + pos;
-        bcell[o] = c;
-        bid[o] = aid[idx];
-        if constexpr (FUSE) {
-            const float4 r = A.a[idx];
-            B.a[o] = r;
-            srec[pos] = r;
-            if constexpr (DIM == 3) {
-                const float2 rb = A.b[idx];
-                B.b[o] = rb;
-                srecb[pos] = rb;
-            }
-        } else {
-            rec_copy<DIM>(A, idx, B, o);
+    constexpr int CH = 256;   // positions per pass
+    __shared__ RegroupCells<S::CB> s;
+    __shared__ float4 s_a[SUMS ? CH : 1];
+    __shared__ float2 s_b[SUMS && DIM == 3 ? CH : 1];
+    if (state_dead(w.counters)) return;
+    const int tid = threadIdx.x, g = tid / S::LPC, gl = tid % S::LPC;
+    ShapeOne32<DIM, DEG> sh[S::NA];
+    int comp[S::NA];
+    if constexpr (SUMS)
+#pragma unroll
+        for (int u = 0; u < S::NA; ++u) {
+            const int a = gl + u * S::LPC;
+            const int kk = (a < S::NACC ? a : 0) / (DIM + 1);
+            comp[u] = a - kk * (DIM + 1);
+            sh[u].init(kk);
         }
-        if (pp.keep_vext)
+    for (int cb = G.bid * S::CB; cb < n_cells; cb += G.nblk * S::CB) {
+        regroup_cells<S::CB>(s, cb, n_cells, old_off, cap, pp, w, omap);
+        const long long base = s.base;
+        const int total = base + s.off[S::CB] <= cap ? s.off[S::CB] : (int)(cap > base ? cap - base : 0);
+        float sum[S::NA], cmp[S::NA];
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) bvext[(size_t)d * cap + o] = avext[(size_t)d * cap + idx];
-    };
-    survivors_of(w, old_off, c, n_st, kin, nsurv, gl, put);
-    const int spawns = nfinal - nsurv;
-    if (spawns > 0) {
-        const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
-        const unsigned long long empty = all & ~w.hitmask[c];
-        const uint32_t id0 = *w.particle_counter + (uint32_t)fo;
-        for (int o = gl; o < pp.nparts_in; o += GS) {
-            if (!((empty >> o) & 1)) continue;
-            const int r = __popcll(empty & ((1ull << o) - 1));
-            // velocity from the cell's FP32 copy of V (this handle keeps no
-            // FP64 per-cell copy), interpolated in FP64
-            double xi[DIM], Vc[ND][DIM], v[DIM];
-            lattice_point<DIM>(pp, o, xi);
+        for (int u = 0; u < S::NA; ++u) sum[u] = cmp[u] = 0.0f;
+        for (int p0 = 0; p0 < total; p0 += CH) {
+            const int p = p0 + tid;
+            if (p < total) {
+                int k;
+                const int src = regroup_source<S::CB>(s, cb, p, w, omap, k);
+                const int c = cb + k;
+                uint32_t id = 0;
+                float4 a;
+                float2 b = make_float2(0.0f, 0.0f);
+                double e[DIM];
+                if (src >= 0) {
+                    id = aid[src];
+                    a = A.a[src];
+                    if constexpr (DIM == 3) b = A.b[src];
 #pragma unroll
-            for (int k = 0; k < ND; ++k)
+                    for (int d = 0; d < DIM; ++d) e[d] = pp.keep_vext ? avext[(size_t)d * cap + src] : 0.0;
+                }
+                if (src < 0) {   // a new particle
+                    double xi[DIM], Vc[ND][DIM], v[DIM];
 #pragma unroll
-                for (int d = 0; d < DIM; ++d) Vc[k][d] = (double)V32c[((size_t)c * ND + k) * DIM + d];
-            interp<DIM, DEG>(Vc, xi, v);
-            const long long q = out0 + nsurv + r;
-            bcell[q] = c;
-            bid[q] = id0 + (uint32_t)r + 1u;
-            float xf[DIM], vf[DIM];
+                    for (int n = 0; n < ND; ++n)
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-                xf[d] = (float)xi[d];
-                vf[d] = (float)v[d];
-                if (pp.keep_vext) bvext[(size_t)d * cap + q] = 0.0;
-            }
-            rec_store<DIM>(B, q, xf, vf);
-            if constexpr (FUSE) {
-                if constexpr (DIM == 2) {
-                    srec[nsurv + r] = make_float4(xf[0], xf[1], vf[0], vf[1]);
-                } else {
-                    srec[nsurv + r] = make_float4(xf[0], xf[1], xf[2], vf[0]);
-                    srecb[nsurv + r] = make_float2(vf[1], vf[2]);
+                        for (int d = 0; d < DIM; ++d) Vc[n][d] = (double)V32c[((size_t)c * ND + n) * DIM + d];
+                    id = *w.particle_counter + s.spawn0[k] + (uint32_t)(p - s.off[k] - s.nsurv[k]) + 1u;
+                    lattice_point<DIM>(pp, -1 - src, xi);
+                    interp<DIM, DEG>(Vc, xi, v);
+                    if constexpr (DIM == 2) {
+                        a = make_float4((float)xi[0], (float)xi[1], (float)v[0], (float)v[1]);
+                    } else {
+                        a = make_float4((float)xi[0], (float)xi[1], (float)xi[2], (float)v[0]);
+                        b = make_float2((float)v[1], (float)v[2]);
+                    }
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) e[d] = 0.0;
+                }
+                const long long o = base + p;
+                bcell[o] = c;
+                bid[o] = id;
+                B.a[o] = a;
+                if constexpr (DIM == 3) B.b[o] = b;
+                if (pp.keep_vext)
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) bvext[(size_t)d * cap + o] = e[d];
+                if constexpr (SUMS) {
+                    s_a[tid] = a;
+                    if constexpr (DIM == 3) s_b[tid] = b;
                 }
             }
-        }
-    }
-    if (gl == 0) {
-        w.arr_cnt[c] = 0;
-        w.ovf_head[c] = -1;
-    }
-    if constexpr (FUSE) {
-        constexpr int NACC = PartialsShape<DIM, DEG>::NACC;
-        wave_sync();
-        // sums per lane: Q1 1 in 2-D (12 lanes), 2 in 3-D; Q2 2 in 2-D, 7 in 3-D
-        constexpr int NA = (NACC + GS - 1) / GS;
-        if (gl < NACC) {
-            double out[NA];
-            cell_sums32<DIM, NA, DEG>(srec, srecb, nfinal, gl, out);
+            if constexpr (SUMS) {
+                __syncthreads();
+                const int q0 = s.off[g] > p0 ? s.off[g] - p0 : 0;
+                const int e = s.off[g + 1] < total ? s.off[g + 1] : total;
+                const int q1 = e - p0 < CH ? e - p0 : CH;
+                for (int q = q0; q < q1; ++q) {
+                    const float4 r = s_a[q];
+                    float xi[DIM], v[DIM];
+                    if constexpr (DIM == 2) {
+                        xi[0] = r.x;
+                        xi[1] = r.y;
+                        v[0] = r.z;
+                        v[1] = r.w;
+                    } else {
+                        const float2 t = s_b[q];
+                        xi[0] = r.x;
+                        xi[1] = r.y;
+                        xi[2] = r.z;
+                        v[0] = r.w;
+                        v[1] = t.x;
+                        v[2] = t.y;
+                    }
 #pragma unroll
-            for (int u = 0; u < NA; ++u)
-                if (gl + u * GS < NACC) partial[(size_t)c * NACC + gl + u * GS] = out[u];
+                    for (int u = 0; u < S::NA; ++u) {
+                        float vc = 1.0f;   // the weight term is N_k itself
+#pragma unroll
+                        for (int d = 0; d < DIM; ++d)
+                            if (d == comp[u]) vc = v[d];
+                        const float y = sh[u](xi) * vc - cmp[u];
+                        const float tt = sum[u] + y;
+                        cmp[u] = (tt - sum[u]) - y;
+                        sum[u] = tt;
+                    }
+                }
+                __syncthreads();
+            }
         }
-        wave_sync();
+        if constexpr (SUMS)
+            if (cb + g < n_cells)
+#pragma unroll
+                for (int u = 0; u < S::NA; ++u)
+                    if (gl + u * S::LPC < S::NACC)
+                        partial[(size_t)(cb + g) * S::NACC + gl + u * S::LPC] = (double)sum[u] - (double)cmp[u];
+        __syncthreads();   // s is refilled
     }
 }
 
-template <int DIM, bool FUSE, int DEG = 1>
-__device__ __forceinline__ void cell_write32_body(const Grid& G, const DevMesh<DIM>& m, const float* __restrict__ V32c, const int* __restrict__ old_off, const uint32_t* __restrict__ aid, const Rec32& A, int* __restrict__ bcell, uint32_t* __restrict__ bid, const Rec32& B, const double* __restrict__ avext, double* __restrict__ bvext, long long cap, const DevParams& pp, const DevWork& w, double* __restrict__ partial) {
-    constexpr bool FB = FUSE && DIM == 3;
-    __shared__ float4 s_rec[FUSE ? GROUPS : 1][FUSE ? FCAP : 1];
-    __shared__ float2 s_recb[FB ? GROUPS : 1][FB ? FCAP : 1];
-    if (state_dead(w.counters)) return;
-    const int g = threadIdx.x / GS, gl = threadIdx.x % GS;
-    for (int c = G.bid * GROUPS + g; c < m.n_cells; c += G.nblk * GROUPS)
-        cell_write32_one<DIM, FUSE, DEG>(m, V32c, old_off, aid, A, bcell, bid, B, avext, bvext, cap, pp, w, c, gl,
-                                         s_rec[FUSE ? g : 0], s_recb[FB ? g : 0], partial);
-}
-
-template <int DIM, bool FUSE, int DEG = 1>
-__global__ void __launch_bounds__(256) k_cell_write32(DevMesh<DIM> m, const float* __restrict__ V32c,
+template <int DIM, bool SUMS, int DEG>
+__global__ void __launch_bounds__(256) k_cell_write32(int n_cells, const float* __restrict__ V32c,
                                                      const int* __restrict__ old_off, const uint32_t* __restrict__ aid,
                                                      Rec32 A, int* __restrict__ bcell, uint32_t* __restrict__ bid,
                                                      Rec32 B, const double* __restrict__ avext,
                                                      double* __restrict__ bvext, long long cap, DevParams pp,
-                                                     DevWork w, double* __restrict__ partial) {
-    cell_write32_body<DIM, FUSE, DEG>(hw_grid(), m, V32c, old_off, aid, A, bcell, bid, B, avext, bvext, cap, pp, w,
-                                      partial);
-}
-
-// The second pass of the two-pass regroup write (k_cell_map, pf2_kernels.hpp)
-// for FP32 records: output positions in order (GU slices per pass, loads
-// before stores), a survivor's record copied (its cell is its destination),
-// a new particle created as k_cell_write32 creates it.  Every wavefront
-// stores whole, consecutive lines.
-template <int DIM, int DEG>
-__device__ __forceinline__ void gather32_spawn(const float* __restrict__ V32c, int* __restrict__ bcell,
-                                               uint32_t* __restrict__ bid, const Rec32& B, double* __restrict__ bvext,
-                                               long long cap, const DevParams& pp, const DevWork& w, long long o,
-                                               int code) {
-    constexpr int ND = QF<DIM, DEG>::ND;
-    const int c = code >> 6, lo = code & 63;
-    const unsigned long long fo = w.fs_off[c];
-    const int r = (int)(o - (long long)(fo >> 32)) - w.nsurv[c];
-    // velocity from the cell's FP32 copy of V, interpolated in FP64
-    double xi[DIM], Vc[ND][DIM], v[DIM];
-    lattice_point<DIM>(pp, lo, xi);
-#pragma unroll
-    for (int k = 0; k < ND; ++k)
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) Vc[k][d] = (double)V32c[((size_t)c * ND + k) * DIM + d];
-    interp<DIM, DEG>(Vc, xi, v);
-    float xf[DIM], vf[DIM];
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-        xf[d] = (float)xi[d];
-        vf[d] = (float)v[d];
-    }
-    bcell[o] = c;
-    bid[o] = *w.particle_counter + (uint32_t)fo + (uint32_t)r + 1u;
-    rec_store<DIM>(B, o, xf, vf);
-    if (pp.keep_vext)
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) bvext[(size_t)d * cap + o] = 0.0;
-}
-
-template <int DIM, int DEG = 1>
-__device__ __forceinline__ void cell_gather32_body(const Grid& G, const DevMesh<DIM>& m, const float* __restrict__ V32c,
-                                                   const uint32_t* __restrict__ aid, const Rec32& A,
-                                                   int* __restrict__ bcell, uint32_t* __restrict__ bid, const Rec32& B,
-                                                   const double* __restrict__ avext, double* __restrict__ bvext,
-                                                   long long cap, const DevParams& pp, const DevWork& w,
-                                                   const int* __restrict__ omap) {
-    if (state_dead(w.counters)) return;
-    const long long total = (long long)(w.fs_off[m.n_cells] >> 32);
-    const long long n = total < cap ? total : cap;
-    const long long bd = blockDim.x, span = (long long)G.nblk * bd * GU;
-    for (long long o0 = (long long)G.bid * bd * GU + threadIdx.x; o0 < n; o0 += span) {
-        int src[GU];
-        bool act[GU];
-#pragma unroll
-        for (int u = 0; u < GU; ++u) {
-            const long long o = o0 + u * bd;
-            act[u] = o < n;
-            src[u] = act[u] ? omap[o] : -1;
-        }
-        int pc[GU];
-        uint32_t pid[GU];
-        float4 ra[GU];
-        float2 rb[GU];
-        double pe[GU][DIM];
-#pragma unroll
-        for (int u = 0; u < GU; ++u) {
-            if (!act[u] || src[u] < 0) continue;
-            const int s = src[u];
-            pc[u] = w.dest[s];
-            pid[u] = aid[s];
-            ra[u] = A.a[s];
-            if constexpr (DIM == 3) rb[u] = A.b[s];
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) pe[u][d] = pp.keep_vext ? avext[(size_t)d * cap + s] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < GU; ++u) {
-            if (!act[u]) continue;
-            const long long o = o0 + u * bd;
-            if (src[u] < 0) {
-                gather32_spawn<DIM, DEG>(V32c, bcell, bid, B, bvext, cap, pp, w, o, -1 - src[u]);
-                continue;
-            }
-            bcell[o] = pc[u];
-            bid[o] = pid[u];
-            B.a[o] = ra[u];
-            if constexpr (DIM == 3) B.b[o] = rb[u];
-            if (pp.keep_vext)
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) bvext[(size_t)d * cap + o] = pe[u][d];
-        }
-    }
-}
-
-template <int DIM, int DEG = 1>
-__global__ void __launch_bounds__(256) k_cell_gather32(DevMesh<DIM> m, const float* __restrict__ V32c,
-                                                       const uint32_t* __restrict__ aid, Rec32 A,
-                                                       int* __restrict__ bcell, uint32_t* __restrict__ bid, Rec32 B,
-                                                       const double* __restrict__ avext, double* __restrict__ bvext,
-                                                       long long cap, DevParams pp, DevWork w,
-                                                       const int* __restrict__ omap) {
-    cell_gather32_body<DIM, DEG>(hw_grid(), m, V32c, aid, A, bcell, bid, B, avext, bvext, cap, pp, w, omap);
-}
-
-// fuse = the projection sums are computed here (final counts per cell
-// bounded by FCAP, i.e. MAX * prod(q_d + 1) <= FCAP and a census with reseed)
-template <int DIM>
-void launch_cell_write32(hipStream_t s, int grid, DevMesh<DIM> m, const float* V32c, const int* old_off, const uint32_t* aid,
-                         Rec32 A, int* bcell, uint32_t* bid, Rec32 B, const double* avext, double* bvext, long long cap,
-                         DevParams pp, DevWork w, bool fuse, double* partial, int deg) {
-    if (fuse && deg == 2)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write32<DIM, true, 2>), dim3(grid), dim3(256), 0, s, m, V32c,
-                           old_off, aid, A, bcell, bid, B, avext, bvext, cap, pp, w, partial);
-    else if (deg == 2)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write32<DIM, false, 2>), dim3(grid), dim3(256), 0, s, m, V32c,
-                           old_off, aid, A, bcell, bid, B, avext, bvext, cap, pp, w, partial);
-    else if (fuse)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write32<DIM, true>), dim3(grid), dim3(256), 0, s, m, V32c, old_off,
-                           aid, A, bcell, bid, B, avext, bvext, cap, pp, w, partial);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_write32<DIM, false>), dim3(grid), dim3(256), 0, s, m, V32c, old_off,
-                           aid, A, bcell, bid, B, avext, bvext, cap, pp, w, partial);
+                                                     DevWork w, int* __restrict__ omap, double* __restrict__ partial) {
+    cell_write32_body<DIM, SUMS, DEG>(hw_grid(), n_cells, V32c, old_off, aid, A, bcell, bid, B, avext, bvext, cap, pp,
+                                      w, omap, partial);
 }
 
 // per-cell projection sums in FP32 with Kahan compensation, ascending id order
@@ -1395,7 +1228,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM ==
 }
 
 // the pending layout of an FP32-mixed handle after a re-sort (k_cell_pend):
-// new particles created as k_cell_gather32 creates them, after the current
+// new particles created as k_cell_write32 creates them, after the current
 // segments (the census marked the survivors)
 template <int DIM, int DEG = 1>
 __global__ void __launch_bounds__(256) k_cell_pend32(int n_cells, const int* __restrict__ old_off, int* __restrict__ pcell,
