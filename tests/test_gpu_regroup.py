@@ -46,7 +46,7 @@ def _setup(case):
 @pytest.mark.parametrize("case", list(CASES))
 def test_fp64_bitwise(case):
     m, V, q, mx, cell, xi = _setup(case)
-    g = ParticleStage(m, 0.05, 4, mx, q, FP64)
+    g = ParticleStage(m, 0.05, 4, mx, q, FP64, capacity=20000)
     o = Oracle(m, 0.05, 4, mx, q)
     for s in (g, o):
         s.upload_fields(V, V)
@@ -61,7 +61,7 @@ def test_fp64_bitwise(case):
 @pytest.mark.parametrize("case", list(CASES))
 def test_fp32_fused_equals_separate(case):
     m, V, q, mx, cell, xi = _setup(case)
-    a, b = (ParticleStage(m, 0.05, 4, mx, q, FP32_MIXED) for _ in range(2))
+    a, b = (ParticleStage(m, 0.05, 4, mx, q, FP32_MIXED, capacity=20000) for _ in range(2))
     for s in (a, b):
         s.upload_fields(V, V)
         s.insert_particles(cell, xi)
