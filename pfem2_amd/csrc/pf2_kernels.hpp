@@ -133,7 +133,8 @@ struct DevMesh {
     const double* star_dir;
     const int* dof_off;
     const int* dof_cell;   // packed: cell * ND + local DoF
-    const double* ftol;    // per cell: tolerance of the clearly-outside test (-1: none)
+    const double* ftol;    // per cell: 2-D the tolerance of the clearly-outside test (-1: none), 3-D the
+                           // HEX_N values of HexCell
     const double* cellX;   // per cell: its vertex coordinates packed [NV][DIM] (copies of X)
     const int2* cell_star; // per cell and local vertex: [begin, end) of that vertex's star
     const int4* cell_nbr;  // per cell, the neighbours across faces 0..2*DIM-1 (-1 on the boundary or past
@@ -326,17 +327,6 @@ __device__ __forceinline__ void lattice_point(const DevParams& pp, int ordinal, 
 // that is the containing cell with the largest key, earliest star position on
 // ties, which is what the loop below selects.  Returns -1 if no star cell
 // contains the point.
-// nodal velocities of cell c (FP64 path)
-template <int DIM, int DEG = 1>
-__device__ __forceinline__ void load_nodes(const double* __restrict__ cellV, int c, double (*Vc)[DIM]) {
-    constexpr int ND = QF<DIM, DEG>::ND;
-    const double* cf = cellV + (size_t)c * ND * DIM;
-#pragma unroll
-    for (int k = 0; k < ND; ++k)
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) Vc[k][d] = cf[k * DIM + d];
-}
-
 // Face through which the step from xold to x most likely left the cell: the
 // linearised reference displacement J(xi_old)^-1 (x - xold) added to xi_old,
 // the component furthest outside [0, 1] (face 2a + s is xi_a = s), -1 if
@@ -479,14 +469,21 @@ __device__ __forceinline__ bool inside_margin(const double* r) {
 // closed form first, the clearly-outside test only where it does not decide
 // (both orders give the same answer).
 template <int DIM, bool CLOSED>
-__device__ __forceinline__ bool contains(const double (*Q)[DIM], const double* x, double* r, double tol) {
-    if constexpr (CLOSED && DIM == 2) {
-        QuadCell qc;
-        qc.init(Q);
-        const int st = closed_form(Q, qc, x, r);
-        if (st != 2) return st == 0;
+__device__ __forceinline__ bool contains(const DevMesh<DIM>& m, int c, const double (*Q)[DIM], const double* x,
+                                         double* r) {
+    if constexpr (DIM == 3) {
+        HexCell H;
+        H.load(m.ftol + (size_t)c * HEX_N);
+        return hex_map(Q, H, x, r) && inside_unit<DIM>(r);
+    } else {
+        if constexpr (CLOSED) {
+            QuadCell qc;
+            qc.init(Q);
+            const int st = closed_form(Q, qc, x, r);
+            if (st != 2) return st == 0;
+        }
+        return inverse_map<DIM>(Q, x, r, m.ftol[c], true) && inside_unit<DIM>(r);
     }
-    return inverse_map<DIM>(Q, x, r, tol, true) && inside_unit<DIM>(r);
 }
 
 // `Q` returns the vertices of the cell found.  (A caller's other data of the
@@ -550,7 +547,9 @@ __device__ __forceinline__ int relocate(const DevMesh<DIM>& m, int c, const doub
                     qc.init(Q);
                     in = closed_form(Q, qc, x, r) == 0;
                 } else {
-                    in = inverse_map<DIM>(Q, x, r, m.ftol[g], true);
+                    HexCell H;
+                    H.load(m.ftol + (size_t)g * HEX_N);
+                    in = hex_map(Q, H, x, r);
                 }
                 if (in && inside_margin<DIM>(r)) {
 #pragma unroll
@@ -616,7 +615,7 @@ __device__ __forceinline__ int relocate(const DevMesh<DIM>& m, int c, const doub
         }
         double r[DIM];
         load_vertices<DIM>(m, cc, Q);
-        if (contains<DIM, !SHORTCUT>(Q, x, r, m.ftol[cc])) {
+        if (contains<DIM, !SHORTCUT>(m, cc, Q, x, r)) {
 #pragma unroll
             for (int d = 0; d < DIM; ++d) xi_out[d] = r[d];
             return cc;
@@ -812,21 +811,50 @@ constexpr int DEST_KEPT = 1 << 30;
 
 // Runs substeps until done (returns 0) or the own-cell test fails (returns
 // 1; s is the substep whose test failed).
-// CLOSED (2-D): the own-cell test takes only inverse_map's closed form and
-// returns 2 where inverse_map would go on to its clearly-outside test and
+// 2-D: the own-cell test takes only inverse_map's closed form and returns 2
+// where inverse_map would go on to its clearly-outside test and
 // Newton iteration (the point is outside the closed form's unit square, or
 // closed_form leaves it undecided); the search finishes that test
 // (relocate's `own`).  This keeps the Newton code, and its registers, out of
 // k_move: 94 instead of 167 registers, 5 instead of 3 wavefronts per SIMD.
-template <int DIM, int DEG = 1, bool CLOSED = false>
-__device__ __forceinline__ int advance64(const DevMesh<DIM>& m, const double* __restrict__ V, const DevParams& pp,
-                                         const DevParticles& A, int i, int c, double* x, double* xi, double* vext,
-                                         int& s, const double (*P)[DIM], const double (*Vc)[DIM], double tol) {
+//
+// 3-D, degree 2: the 81 nodal velocities of a cell are read in every substep
+// (the lanes of a wavefront share a few cells, so the reads hit L1) instead of
+// held in 162 registers, which spilled.
+template <int DIM, int DEG = 1>
+__device__ __forceinline__ int advance64(const DevMesh<DIM>& m, const DevParams& pp, const DevParticles& A, int i, int c,
+                                         double* x, double* xi, double* vext, int& s, const double (*P)[DIM]) {
+    constexpr int ND = QF<DIM, DEG>::ND;
+    constexpr bool REREAD = DIM == 3 && DEG == 2;
+    const double* cf = m.cellV + (size_t)c * ND * DIM;
+    double Vc[REREAD ? 1 : ND][DIM];
+    if constexpr (!REREAD)
+#pragma unroll
+        for (int k = 0; k < ND; ++k)
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) Vc[k][d] = cf[k * DIM + d];
     QuadCell qc;
-    if constexpr (CLOSED && DIM == 2) qc.init(P);
+    HexCell H;
+    if constexpr (DIM == 2) qc.init(P);
+    else H.load(m.ftol + (size_t)c * HEX_N);
     for (; s < pp.substeps; ++s) {
         double u[DIM];
-        interp<DIM, DEG>(Vc, xi, u);
+        if constexpr (REREAD) {
+            // (an address the compiler cannot carry from one substep to the
+            // next, or it loads the values once and spills them)
+            const double* f = cf;
+            asm volatile("" : "+v"(f));
+            double N[ND];
+            shape_q<DIM, DEG>(xi, N);
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) u[d] = 0.0;
+#pragma unroll
+            for (int k = 0; k < ND; ++k)
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) u[d] += N[k] * f[k * DIM + d];
+        } else {
+            interp<DIM, DEG>(Vc, xi, u);
+        }
 #pragma unroll
         for (int d = 0; d < DIM; ++d) vext[d] = u[d];
 #pragma unroll
@@ -837,19 +865,12 @@ __device__ __forceinline__ int advance64(const DevMesh<DIM>& m, const double* __
 #pragma unroll
             for (int d = 0; d < DIM; ++d) A.vext[(size_t)d * A.cap + i] = vext[d];
         double r[DIM];
-        if constexpr (CLOSED && DIM == 2) {
-            const int st = closed_form(P, qc, x, r);
-            if (st) return st;
+        int st;
+        if constexpr (DIM == 2) st = closed_form(P, qc, x, r);
+        else st = hex_map(P, H, x, r) && inside_unit<DIM>(r) ? 0 : 1;
+        if (st) return st;
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) xi[d] = r[d];
-        } else {
-            if (inverse_map<DIM>(P, x, r, tol, false) && inside_unit<DIM>(r)) {
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) xi[d] = r[d];
-            } else {
-                return 1;
-            }
-        }
+        for (int d = 0; d < DIM; ++d) xi[d] = r[d];
     }
     return 0;
 }
@@ -944,9 +965,9 @@ __device__ __forceinline__ void move_body(const Grid& G, const DevMesh<DIM>& m, 
         if (valid) {
 #pragma unroll
             for (int d = 0; d < DIM; ++d) x[d] = A.x[(size_t)d * A.cap + i];
-            double P[NV][DIM], Vc[ND][DIM];
-            load_cell<DIM, false, DEG>(m, c, P, Vc);
-            st = advance64<DIM, DEG, true>(m, V, pp, A, i, c, x, xi, vext, s, P, Vc, m.ftol[c]);
+            double P[NV][DIM];
+            load_vertices<DIM>(m, c, P);
+            st = advance64<DIM, DEG>(m, pp, A, i, c, x, xi, vext, s, P);
         }
         park_particle<DIM>(A, w, qu, 0, L.shard, valid && st != 0, i, c, x, xi, vext, st == 2 ? s | PARK_NEWTON : s);
         finish_particle<DIM>(pp, A, w, valid && st == 0, i, c, x, xi, true, seg_end);
@@ -1045,15 +1066,13 @@ __device__ __forceinline__ void search_body(const Grid& G, const DevMesh<DIM>& m
                     done = true;   // re-sort after a mesh move: no advection
                 } else {
                     ++s;
-                    double Vc[QF<DIM, DEG>::ND][DIM];
-                    load_nodes<DIM, DEG>(m.cellV, cn, Vc);
 #pragma unroll
                     for (int k = 0; k < NV; ++k)
 #pragma unroll
                         for (int d = 0; d < DIM; ++d) P[k][d] = Q[k][d];
                     // (2-D: a test the closed form does not decide comes back
                     // as pending, as from k_move)
-                    const int st = advance64<DIM, DEG, true>(m, V, pp, A, i, cn, x, xi, vext, s, P, Vc, m.ftol[cn]);
+                    const int st = advance64<DIM, DEG>(m, pp, A, i, cn, x, xi, vext, s, P);
                     done = st == 0;
                     newton = st == 2;
                 }
@@ -2210,7 +2229,7 @@ __global__ void __launch_bounds__(256) k_resort(DevMesh<DIM> m, DevParticles A, 
                     qc.init(P);
                     st = closed_form(P, qc, x, r);
                 } else {
-                    st = inverse_map<DIM>(P, x, r, m.ftol[c], false) && inside_unit<DIM>(r) ? 0 : 1;
+                    st = contains<DIM, false>(m, c, P, x, r) ? 0 : 1;
                 }
                 if (st == 0) {
 #pragma unroll

@@ -887,7 +887,8 @@ size_t estimate_bytes(int dim, long long nc, long long nvt, long long nd, long l
     b += nvt * dim * 8 + nck * 4 + ndc * 4 + (nvt + 1) * 4 + nck * 4 + nck * dim * 8;  // X, cv, cd, star
     b += nc;                                                                             // moved-cell flags
     b += nc * 16 * (dim - 1) + nvt * 5;                                                  // face neighbours, vertex flags
-    b += (nd + 1) * 4 + ndc * 4 + nc * 8 + nck * dim * 8 + nck * 8;                    // dof map, ftol, cellX/star
+    b += (nd + 1) * 4 + ndc * 4 + nck * dim * 8 + nck * 8;                              // dof map, cellX/star
+    b += nc * 8 * (dim == 3 ? HEX_N : 1);                                                // ftol / hexahedra
     if (p->precision != PF2_FP32_MIXED) b += ndc * dim * 8 * 2;                          // FP64 cell V / dV copies
     b += nd * dim * 8 * 3;                                                              // V, V_old, staging
     b += (nc + 1) * 4 * 10 + nc * 4 * (1 + arrival_slots(dim, p));                     // per-cell work, arrival slots
@@ -1312,7 +1313,7 @@ int pf2_create_in(const pf2_mesh* mesh, const pf2_params* params, long long capa
     if (dalloc(&h->dX, (size_t)nvt * dim) || dalloc(&h->dcv, nck) || dalloc(&h->dcd, ndc) ||
         dalloc(&h->dstar_off, nvt + 1) || dalloc(&h->dstar_cell, h->star_cell.size()) ||
         dalloc(&h->dstar_dir, h->star_dir.size()) || dalloc(&h->ddof_off, nd + 1) ||
-        dalloc(&h->ddof_cell, h->dof_cell.size()) || dalloc(&h->dftol, nc) || dalloc(&h->dcellX, nck * dim) || dalloc(&h->dcell_star, nck) ||
+        dalloc(&h->ddof_cell, h->dof_cell.size()) || dalloc(&h->dftol, (size_t)nc * (dim == 3 ? HEX_N : 1)) || dalloc(&h->dcellX, nck * dim) || dalloc(&h->dcell_star, nck) ||
         dalloc(&h->dcell_nbr, (size_t)h->n_cells * (h->dim - 1)) || dalloc(&h->dvbnd, nvt) || dalloc(&h->dcmoved, nc) ||
         dalloc(&h->dvdof, nvt) ||
         (!mixed(h) && (dalloc(&h->dcellV, ndc * dim) || dalloc(&h->dcellDV, ndc * dim))) ||

@@ -131,8 +131,8 @@ __global__ void k_geo32(DevMesh<DIM> m, float* __restrict__ geo) {
     }
 }
 
-// per-cell FP64 tolerance of the clearly-outside test, the packed vertex
-// copy, and whether the copy changed (cmoved: any coordinate differs from
+// per-cell FP64 tolerance of the clearly-outside test (3-D: the table of
+// HexCell), the packed vertex copy, and whether the copy changed (cmoved: any coordinate differs from
 // the one it replaces)
 template <int DIM>
 __global__ void k_ftol(DevMesh<DIM> m, double* __restrict__ ftol, double* __restrict__ cellX,
@@ -140,7 +140,13 @@ __global__ void k_ftol(DevMesh<DIM> m, double* __restrict__ ftol, double* __rest
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < m.n_cells; c += gridDim.x * blockDim.x) {
         double P[Q1<DIM>::NV][DIM];
         gather_vertices<DIM>(m, c, P);
-        ftol[c] = outside_tol<DIM>(P);
+        if constexpr (DIM == 2) {
+            ftol[c] = outside_tol<DIM>(P);
+        } else {
+            HexCell H;
+            H.init(P);
+            H.store(ftol + (size_t)c * HEX_N);
+        }
         bool moved = false;
 #pragma unroll
         for (int k = 0; k < Q1<DIM>::NV; ++k)
@@ -1153,7 +1159,7 @@ __global__ void __launch_bounds__(256) k_resort32(DevMesh<DIM> m, const int* __r
                     qc.init(P);
                     st = closed_form(P, qc, x, r);
                 } else {
-                    st = inverse_map<DIM>(P, x, r, m.ftol[c], false) && inside_unit<DIM>(r) ? 0 : 1;
+                    st = contains<DIM, false>(m, c, P, x, r) ? 0 : 1;
                 }
                 if (st == 0) {
 #pragma unroll

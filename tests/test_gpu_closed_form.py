@@ -57,3 +57,36 @@ def test_cell_shapes_bitwise(shape):
     sg, so = g.stats(), o.stats()
     assert sg["searches"] == so["searches"] and sg["lost"] == so["lost"] and sg["deleted"] == so["deleted"]
     g.close()
+
+
+@pytest.mark.parametrize("degree", [1, 2])
+@pytest.mark.parametrize("shape", ["general", "box", "sheared", "far", "tiny", "large"])
+def test_hexahedron_shapes_bitwise(shape, degree):
+    """The tabulated inverse map of hexahedra (hex_map): affine cells that end
+    at its early out, general ones through its Newton iteration, residuals
+    near the rounding of far coordinates, small and large lengths."""
+    m = M.box_3d(5, 4, 3, (0.0, 0.0, 0.0), (1.0, 0.8, 0.6), jitter=0.0 if shape in ("box", "sheared") else 0.2, seed=4)
+    X, size = m.vertices.copy(), {"tiny": 1e-60, "large": 1e60}.get(shape, 1.0)
+    if shape == "sheared":
+        X[:, 0] += 0.3 * X[:, 1] - 0.2 * X[:, 2]
+    if shape == "far":
+        X += np.array([2.0e5, -1.0e5, 3.0e4])
+    m.vertices = np.ascontiguousarray(size * X)
+    if degree == 2:
+        m = M.q2(m)
+    rng = np.random.default_rng(12)
+    V = size * (np.array([[0.7], [0.3], [-0.2]]) + rng.uniform(-0.4, 0.4, size=(3, m.n_dofs)))
+    g = ParticleStage(m, 0.1, 5, 2, [2, 2, 2], FP64)
+    o = Oracle(m, 0.1, 5, 2, [2, 2, 2])
+    cell, xi = M.jittered_lattice(m, [2, 2, 2], 0.1, 7)
+    edge = np.array([[0.0, 0.0, 0.0], [1.0, 1.0, 1.0], [0.0, 0.5, 1.0]])
+    cell = np.concatenate([cell, np.repeat(np.arange(5, dtype=np.int32) * 3, len(edge))])
+    xi = np.concatenate([xi, np.tile(edge, (5, 1))])
+    for s in (g, o):
+        s.upload_fields(V, V)
+        s.insert_particles(cell, xi)
+    for step in range(3):
+        assert bitwise_equal(g.step(download=True), o.step()), step
+    assert_particles_match(g.particles(), o.particles(), 0.0, shape, bitwise=True)
+    assert g.stats()["searches"] == o.stats()["searches"] and g.stats()["lost"] == o.stats()["lost"]
+    g.close()
