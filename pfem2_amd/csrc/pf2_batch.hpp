@@ -1,7 +1,7 @@
 // pf2_batch.hpp — one step of many simulations with one launch per kernel.
 //
 // A batch lists simulations of the same dimension and precision.  Every
-// kernel of the step (field refresh, move, relocation rounds, census, offset
+// kernel of the step (field refresh, move, search, census, offset
 // scan, write with the projection sums, bookkeeping, node sums) is launched once for the whole
 // batch: the launch's workgroups are split into consecutive ranges, one per
 // simulation (sized as that simulation's own launch would be), and each
@@ -19,10 +19,9 @@
 namespace pf2 {
 
 enum BatchKind {
-    BK_REFRESH = 0, BK_MOVE, BK_SEARCH0, BK_SEARCH1, BK_SEARCH2, BK_COUNT, BK_COUNT_L, BK_BIG, BK_TILES,
+    BK_REFRESH = 0, BK_MOVE, BK_SEARCH, BK_COUNT, BK_COUNT_L, BK_BIG, BK_TILES,
     BK_WRITE, BK_NODE, BK_NKINDS
 };
-static_assert(MOVE_ROUNDS <= 2, "kinds for up to three relocation rounds");
 
 template <int DIM>
 struct BatchSim {
@@ -95,17 +94,17 @@ __global__ void __launch_bounds__(256) kb_move32(BatchView<DIM> bv) {
 }
 
 template <int DIM>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 3 : 2))) kb_search(BatchView<DIM> bv, int round) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 3 : 2))) kb_search(BatchView<DIM> bv) {
     Grid G;
-    const BatchSim<DIM>& S = bv.at(BK_SEARCH0 + round, G);
-    search_body<DIM>(G, S.m, S.V, S.A, S.pp, S.w, S.qu, round);
+    const BatchSim<DIM>& S = bv.at(BK_SEARCH, G);
+    search_body<DIM>(G, S.m, S.V, S.A, S.pp, S.w, S.qu, 0);
 }
 
-template <int DIM, bool LAST>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LAST ? 2 : (DIM == 2 ? 4 : 3)))) kb_search32(BatchView<DIM> bv, int round) {
+template <int DIM>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 4 : 3))) kb_search32(BatchView<DIM> bv) {
     Grid G;
-    const BatchSim<DIM>& S = bv.at(BK_SEARCH0 + round, G);
-    search32_body<DIM, LAST>(G, S.m, S.V32, S.geo, S.A.cell, S.RA, S.A.vext, S.A.cap, S.pp, S.w, S.qu, round);
+    const BatchSim<DIM>& S = bv.at(BK_SEARCH, G);
+    search32_body<DIM>(G, S.m, S.V32, S.geo, S.A.cell, S.RA, S.A.vext, S.A.cap, S.pp, S.w, S.qu);
 }
 
 template <int DIM, int CAP>

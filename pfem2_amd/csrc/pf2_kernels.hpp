@@ -11,8 +11,8 @@
 //   k_move         one thread per particle: correction, then substeps of
 //                  advection in registers until done or the first failed
 //                  own-cell test; such particles are parked in a queue.
-//   k_search_resume  MOVE_ROUNDS + 1 rounds over the queue: vertex-star
-//                  search in full wavefronts, then the remaining substeps.
+//   k_search_resume  over the queue: vertex-star search in full wavefronts,
+//                  then the remaining substeps.
 //                  A particle that ends in another cell takes a slot in that
 //                  cell's arrival row (add_arrival).
 //   k_cell_count   one 16-lane group per cell: part counts over stayers +
@@ -634,42 +634,34 @@ __device__ __forceinline__ int relocate(const DevMesh<DIM>& m, int c, const doub
 // substep index stored) and queued; the vertex-star searches of all queued
 // particles then run the vertex-star search in full wavefronts, which
 // continue the remaining substeps.
-//   FP64 path: one search round (k_search_resume) whose lanes follow their
-//   particle through every further crossing and refill from the queue when
-//   it is done (search_body).
-//   FP32-mixed path: MOVE_ROUNDS parking rounds (k_search_resume32 parks a
-//   particle that leaves its new cell again), then a last round that loops
-//   every remaining particle to its end.
-#ifndef PF2_MOVE_ROUNDS
-#define PF2_MOVE_ROUNDS 1
-#endif
-constexpr int MOVE_ROUNDS = PF2_MOVE_ROUNDS;
-static_assert(MOVE_ROUNDS == 1, "one parking round (two measured slower)");
+//   One search round (k_search_resume, k_search_resume32), whose lanes follow
+//   their particle through every further crossing and refill from the queue
+//   when it is done (search_body).
 // the queue segments of the refilling search (one cursor each, on its own
 // cache line: a single cursor for the whole grid serialises the wavefronts'
 // atomics) and the idle lanes a wavefront gathers before it refills
 constexpr int RSEGS = 256;
 constexpr int REFILL_MIN = 16;
-// the round whose shard counters hold the cursors: after the FP32-mixed
-// path's last round, so no search pushes to it; the counters are cleared
-// with the other queue counters after each regroup
-constexpr int CURSOR_ROUND = MOVE_ROUNDS + 1;
+// the counters of the move's queue are round 0's; the next round's hold the
+// cursors (cleared with the queue counters after each regroup)
+constexpr int CURSOR_ROUND = 1;
 // the queue of the re-sort's relocations after a mesh move (both paths)
-constexpr int RESORT_QUEUE = MOVE_ROUNDS + 2;
-// queues (rounds) of the counters: the moves' rounds, the cursors, the re-sort
-constexpr int NQROUNDS = MOVE_ROUNDS + 3;
+constexpr int RESORT_QUEUE = 2;
+// rounds of the counters: the move's queue, the cursors, the re-sort
+constexpr int NQROUNDS = 3;
 
-// Queues of parked particles, one per round, ping-ponging between two
-// buffers.  A queue is QSHARDS shards of shard_cap entries plus an overflow
+// Queues of parked particles, the move's and the re-sort's (never filled at
+// the same time) in one buffer.  A queue is QSHARDS shards of shard_cap entries plus an overflow
 // region of cap entries; each shard's counter sits on its own 128-byte line
 // and a wavefront appends to shard (wavefront id mod QSHARDS) with one atomic.
 constexpr int QSHARDS = 256;
 constexpr int QSTRIDE = 32;   // ints between shard counters
 
 struct DevQueues {
-    int2* data[2];        // ping-pong buffers of (particle, cell): QSHARDS * shard_cap + overflow
+    int2* data;           // (particle, cell): QSHARDS * shard_cap + overflow
     int* count;           // NQROUNDS rounds x (QSHARDS + 1) counters, QSTRIDE apart
-    int* prefix;          // per round: QSHARDS + 2 ints (exclusive prefix, overflow start, total)
+    int* prefix;          // per round: QSHARDS + 2 ints (exclusive prefix, overflow start, total); round 1:
+                          // QSHARDS partial counts of particles searched for again (FP32-mixed)
     int shard_cap;
     double* park_vext;    // DIM x cap: velocity_ext of a parked particle
     int* park_s;          // substep index of a parked particle
@@ -742,7 +734,7 @@ __device__ __forceinline__ void queue_push(const DevQueues& qu, int round, bool 
     base = __shfl(base, leader);
     const int slot = base + __popcll(mask & ((1ull << lane) - 1));
     const bool spill = pred && slot >= qu.shard_cap;
-    int2* data = qu.data[round & 1];
+    int2* data = qu.data;
     if (pred && !spill) data[(size_t)sh * qu.shard_cap + slot] = value;
     const unsigned long long smask = __ballot(spill);
     if (smask == 0) return;
@@ -790,8 +782,8 @@ __device__ __forceinline__ int queue_prefix(const DevQueues& qu, int round, int*
 }
 
 // particle index of queue entry j
-__device__ __forceinline__ int2 queue_get(const DevQueues& qu, int round, const int* s_pref, int j) {
-    const int2* data = qu.data[round & 1];
+__device__ __forceinline__ int2 queue_get(const DevQueues& qu, const int* s_pref, int j) {
+    const int2* data = qu.data;
     if (j >= s_pref[QSHARDS]) return data[(size_t)QSHARDS * qu.shard_cap + (j - s_pref[QSHARDS])];
     int lo = 0, hi = QSHARDS - 1;   // last shard with s_pref <= j
     while (lo < hi) {
@@ -981,6 +973,46 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM ==
     move_body<DIM, DEG>(hw_grid(), m, V, Vold, A, pp, w, qu, do_correct, do_move);
 }
 
+// Queue entries for the lanes of a search wavefront that hold no particle.
+// The queue is dealt in chunks of WAVE entries to segments (as many as the
+// grid has wavefronts, up to RSEGS, so every segment has a wavefront), chunk k
+// to segment k mod nseg: the particles with long crossing chains lie together
+// (around the obstacle), and with one contiguous range a segment its few
+// wavefronts were still searching when the others had left (FP64 search 197 ->
+// 159 us per step on 101,785 cells with 2.4M particles).  The segment's cursor
+// advances by one returning atomic once REFILL_MIN lanes are idle or all are
+// (8 or 32: the same).
+struct Refill {
+    int* cursor;
+    int n, seg, nseg;
+    bool more;   // wavefront-uniform: the segment may hold further entries
+    __device__ __forceinline__ Refill(const DevQueues& qu, int n_, const Grid& G) : n(n_), more(true) {
+        const unsigned wpb = blockDim.x / WAVE, nwv = G.nblk * wpb;
+        const unsigned gw = G.bid * wpb + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+        nseg = (int)(nwv < (unsigned)RSEGS ? nwv : (unsigned)RSEGS);
+        seg = (int)(gw % (unsigned)nseg);
+        cursor = queue_count(qu, CURSOR_ROUND, seg);
+    }
+    // queue entry of position p in the segment
+    __device__ __forceinline__ long long entry(int p) const {
+        return ((long long)(p / WAVE) * nseg + seg) * WAVE + p % WAVE;
+    }
+    // the queue entry for this lane or -1 (all lanes call; have: it holds a particle)
+    __device__ __forceinline__ int next(bool have, int lane) {
+        if (!more) return -1;
+        const unsigned long long need = __ballot(!have);
+        const int k = __popcll(need);
+        if (need == 0 || (k < REFILL_MIN && need != ~0ull)) return -1;
+        const int leader = __ffsll((long long)need) - 1;
+        int base = 0;
+        if (lane == leader) base = atomicAdd(cursor, k);
+        base = __builtin_amdgcn_readlane(base, leader);
+        more = entry(base + k) < n;
+        const long long j = entry(base + __popcll(need & ((1ull << lane) - 1)));
+        return !have && j < n ? (int)j : -1;
+    }
+};
+
 // k_search_resume: the vertex-star search of the parked particles, then
 // their remaining substeps, in one round.  A lane follows its particle
 // through every further crossing and, when the particle is done, refills
@@ -998,52 +1030,33 @@ __device__ __forceinline__ void search_body(const Grid& G, const DevMesh<DIM>& m
     constexpr int NV = Q1<DIM>::NV;
     __shared__ int s_pref[QSHARDS + 2];
     const int n = queue_prefix(qu, round, s_pref, G);
-    // the wavefront's segment of the queue and its cursor: as many segments
-    // as the grid has wavefronts, up to RSEGS, so every segment has one
-    const unsigned wpb = blockDim.x / WAVE, nwv = G.nblk * wpb;
-    const unsigned gw = G.bid * wpb + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int nseg = (int)(nwv < (unsigned)RSEGS ? nwv : (unsigned)RSEGS);
-    const int seg = (int)(gw % (unsigned)nseg);
-    const int s0 = (int)((long long)n * seg / nseg), s1 = (int)((long long)n * (seg + 1) / nseg);
-    int* cursor = queue_count(qu, CURSOR_ROUND, seg);
     // new particles of a pending layout (from its segment end on) arrive in their cell
     const int seg_end = !RESORT && w.counters[6] > 0 ? w.counters[7] : 0x7fffffff;
     const int lane = threadIdx.x & (WAVE - 1);
-    const unsigned long long below = (1ull << lane) - 1;
+    Refill F(qu, n, G);
     int lost = 0, searches = 0;
-    bool have = false, more = true, newton = false;
+    bool have = false, newton = false;
     int i = 0, c = 0, s = 0;
     double x[DIM], xi[DIM], vext[DIM], P[NV][DIM];
 #pragma unroll
     for (int d = 0; d < DIM; ++d) x[d] = xi[d] = vext[d] = 0.0;
     for (;;) {
-        if (more) {   // wavefront-uniform
-            const unsigned long long need = __ballot(!have);
-            if (need && (__popcll(need) >= REFILL_MIN || need == ~0ull)) {
-                const int k = __popcll(need);
-                const int leader = __ffsll((long long)need) - 1;
-                int base = 0;
-                if (lane == leader) base = atomicAdd(cursor, k);
-                base = s0 + __shfl(base, leader);
-                more = base + k < s1;
-                const int j = base + __popcll(need & below);
-                if (!have && j < s1) {
-                    const int2 e = queue_get(qu, round, s_pref, j);
-                    i = e.x;
-                    c = e.y;
-                    const int ps = qu.park_s[i];
-                    s = ps & ~PARK_NEWTON;
-                    newton = (ps & PARK_NEWTON) != 0;
+        const int j = F.next(have, lane);
+        if (j >= 0) {
+            const int2 e = queue_get(qu, s_pref, j);
+            i = e.x;
+            c = e.y;
+            const int ps = qu.park_s[i];
+            s = ps & ~PARK_NEWTON;
+            newton = (ps & PARK_NEWTON) != 0;
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) {
-                        x[d] = A.x[(size_t)d * A.cap + i];
-                        xi[d] = A.xi[(size_t)d * A.cap + i];
-                        vext[d] = qu.park_vext[(size_t)d * A.cap + i];
-                    }
-                    load_vertices<DIM>(m, c, P);
-                    have = true;
-                }
+            for (int d = 0; d < DIM; ++d) {
+                x[d] = A.x[(size_t)d * A.cap + i];
+                xi[d] = A.xi[(size_t)d * A.cap + i];
+                vext[d] = qu.park_vext[(size_t)d * A.cap + i];
             }
+            load_vertices<DIM>(m, c, P);
+            have = true;
         }
         if (__ballot(have) == 0) break;
         bool done = false;

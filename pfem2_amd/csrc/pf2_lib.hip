@@ -159,7 +159,7 @@ struct pf2_handle_s {
     int* qcount = nullptr;
     int* qprefix = nullptr;
     long long shard_cap = 0;
-    int2* queue[2] = {nullptr, nullptr};
+    int2* queue = nullptr;
     double* park_vext = nullptr;
     int* park_s = nullptr;
     uint32_t* pcounter = nullptr;
@@ -253,12 +253,7 @@ int cell_grid(int n_cells, int cap = 4096) {
 int pack_fields(pf2_handle_s* h);
 int ensure_packed(pf2_handle_s* h);
 
-// search grid per round: the first round sees most parked particles; later
-// rounds see fewer, the last one loops every remaining particle to the end
-int round_grid(int qgrid, int r) {
-    if (r == 0) return qgrid;
-    return r == MOVE_ROUNDS ? qgrid / 2 + 1 : qgrid / 4 + 1;
-}
+constexpr int SEARCH_GRID = 1024;   // workgroups of a move's search at most (run_move)
 
 int grid_for(long long n, int block, int cap_blocks = 65535 * 4) {
     long long g = (n + block - 1) / block;
@@ -308,8 +303,7 @@ DevParticles dev_particles(pf2_handle_s* h, int which) {
 
 DevQueues dev_queues(pf2_handle_s* h) {
     DevQueues q;
-    q.data[0] = h->queue[0];
-    q.data[1] = h->queue[1];
+    q.data = h->queue;
     q.count = h->qcount;
     q.prefix = h->qprefix;
     q.shard_cap = (int)h->shard_cap;
@@ -427,7 +421,7 @@ int alloc_particles(pf2_handle_s* h) {
     h->shard_cap = 2 * ((h->cap + QSHARDS - 1) / QSHARDS) + 64;
     const long long qlen = QSHARDS * h->shard_cap + h->cap;
     if (dalloc(&h->dest, h->cap) || dalloc(&h->pkey, h->cap) || dalloc(&h->spos, h->cap) || dalloc(&h->omap, h->cap) ||
-        dalloc(&h->ovf, h->cap) || dalloc(&h->queue[0], qlen) || dalloc(&h->queue[1], qlen) ||
+        dalloc(&h->ovf, h->cap) || dalloc(&h->queue, qlen) ||
         dalloc(&h->park_s, h->cap) || dalloc(&h->park_vext, h->cap * h->dim))
         return PF2_E_HIP;
     return 0;
@@ -442,10 +436,10 @@ void free_particles(pf2_handle_s* h) {
         pb = PBufs();
     }
     hipFree(h->dest); hipFree(h->pkey); hipFree(h->spos); hipFree(h->omap); hipFree(h->ovf);
-    hipFree(h->queue[0]); hipFree(h->queue[1]); hipFree(h->park_s); hipFree(h->park_vext);
+    hipFree(h->queue); hipFree(h->park_s); hipFree(h->park_vext);
     h->dest = h->pkey = h->spos = h->omap = h->park_s = nullptr;
     h->ovf = nullptr;
-    h->queue[0] = h->queue[1] = nullptr;
+    h->queue = nullptr;
     h->park_vext = nullptr;
 }
 
@@ -625,12 +619,11 @@ int run_move(pf2_handle_s* h, int do_correct, int do_move, bool fuse_sums = fals
     DevQueues qu = dev_queues(h);
     // the move: up to 8192 workgroups, about one wavefront-sized chunk per
     // wavefront on the cylinder workload (a smaller grid looping over
-    // several chunks was 1% slower); the searches: up to 2048 (FP64) or
-    // 4096 (FP32: its rounds take contiguous queue ranges per workgroup,
-    // 0.8% faster on the 14.6M-particle moving step, the same on smaller
-    // ones)
+    // several chunks was 1% slower); the search: up to 1024, all the
+    // chip holds at 4 wavefronts per SIMD, whose lanes refill (2048 the same,
+    // 512 20% slower)
     const int grid = grid_for(h->n_est, 256, 8192);
-    const int qgrid = grid_for(h->n_est / 2 + 1, 256, mixed(h) ? 4096 : 2048);
+    const int qgrid = grid_for(h->n_est / 2 + 1, 256, SEARCH_GRID);
     if (mixed(h)) {
         h->fp64_valid = false;
         PBufs& b = h->buf[h->cur];
@@ -639,12 +632,11 @@ int run_move(pf2_handle_s* h, int do_correct, int do_move, bool fuse_sums = fals
             launch_move32<DIM>(h->stream, grid, dev_mesh<DIM>(h), h->dV32, h->dVold32, h->dgeo32, b.cell, rec32(b),
                                b.vext, h->cap, pp, w, qu, do_correct, do_move, h->deg);
         }
-        if (do_move)
-            for (int r = 0; r <= MOVE_ROUNDS; ++r) {
-                Timed t(h, r == 0 ? K_SEARCH32 : (r == 1 ? K_SEARCH32_R1 : K_SEARCH32_R2));
-                launch_search_resume32<DIM>(h->stream, round_grid(qgrid, r), dev_mesh<DIM>(h), h->dV32,
-                                            h->dgeo32, b.cell, rec32(b), b.vext, h->cap, pp, w, qu, r, h->deg);
-            }
+        if (do_move) {
+            Timed t(h, K_SEARCH32);
+            launch_search_resume32<DIM>(h->stream, qgrid, dev_mesh<DIM>(h), h->dV32, h->dgeo32, b.cell, rec32(b),
+                                        b.vext, h->cap, pp, w, qu, h->deg);
+        }
     } else {
         {
             Timed t(h, K_MOVE);
@@ -658,7 +650,6 @@ int run_move(pf2_handle_s* h, int do_correct, int do_move, bool fuse_sums = fals
                                    do_move);
         }
         if (do_move) {
-            // one search round with refilling lanes (queue 0)
             Timed t(h, K_SEARCH);
             if (h->deg == 2)
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume<DIM, 2>), dim3(qgrid), dim3(256), 0, h->stream,
@@ -905,7 +896,7 @@ size_t estimate_bytes(int dim, long long nc, long long nvt, long long nd, long l
     b += 2 * cap * per;                                                                 // two particle buffers
     const long long shard_cap = 2 * ((cap + QSHARDS - 1) / QSHARDS) + 64;
     const long long qlen = QSHARDS * shard_cap + cap;
-    b += cap * 4 * 6 + 2 * qlen * 8 + cap * 4 + cap * dim * 8;                          // work, map, overflow, queues, parking
+    b += cap * 4 * 6 + qlen * 8 + cap * 4 + cap * dim * 8;                              // work, map, overflow, queue, parking
     return b + (1u << 20);
 }
 
@@ -1043,10 +1034,10 @@ void batch_fill(pf2_handle_s* h, const double* field, BatchSim<DIM>& S, int* gri
     const int nc = h->n_cells;
     S.ntiles = (nc + 1 + SCAN_TILE - 1) / SCAN_TILE;
     // each kernel's grid as the simulation's own step would launch it
-    const int qgrid = grid_for(h->n_est / 2 + 1, 256, 2048);
+    const int qgrid = grid_for(h->n_est / 2 + 1, 256, SEARCH_GRID);
     grid[BK_REFRESH] = grid_for(std::max((long long)nc * h->nd, (long long)h->n_dofs), 256, 4096);
     grid[BK_MOVE] = grid_for(h->n_est, 256, 8192);
-    for (int r = 0; r <= MOVE_ROUNDS; ++r) grid[BK_SEARCH0 + r] = round_grid(qgrid, r);
+    grid[BK_SEARCH] = qgrid;
     // (batched steps keep rows of GCAP_L for lattices of more than 16 parts:
     // they have no second census pass)
     const bool small = S.pp.nparts_in <= 16;
@@ -1092,14 +1083,8 @@ int batch_step(pf2_batch_s* b, int n, const pf2_handle* hs, const double* const*
     hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_refresh<DIM>), dim3(tot[BK_REFRESH]), dim3(256), 0, st, bv);
     if (mx) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_move32<DIM>), dim3(tot[BK_MOVE]), dim3(256), 0, st, bv);
     else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_move<DIM>), dim3(tot[BK_MOVE]), dim3(256), 0, st, bv);
-    if (!mx)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_search<DIM>), dim3(tot[BK_SEARCH0]), dim3(256), 0, st, bv, 0);
-    else
-        for (int r = 0; r <= MOVE_ROUNDS; ++r) {
-            const dim3 g(tot[BK_SEARCH0 + r]);
-            if (r == MOVE_ROUNDS) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_search32<DIM, true>), g, dim3(256), 0, st, bv, r);
-            else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_search32<DIM, false>), g, dim3(256), 0, st, bv, r);
-        }
+    if (mx) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_search32<DIM>), dim3(tot[BK_SEARCH]), dim3(256), 0, st, bv);
+    else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_search<DIM>), dim3(tot[BK_SEARCH]), dim3(256), 0, st, bv);
     if (tot[BK_COUNT])
         hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_count<DIM, GCAP>), dim3(tot[BK_COUNT]), dim3(256), 0, st, bv);
     if (tot[BK_COUNT_L])
@@ -1359,6 +1344,7 @@ int pf2_create_in(const pf2_mesh* mesh, const pf2_params* params, long long capa
         hipMemsetAsync(h->counters, 0, sizeof(int) * 8, h->stream) ||
         hipMemsetAsync(h->big, 0, sizeof(int) * (nc + 1), h->stream) ||
         hipMemsetAsync(h->big2, 0, sizeof(int) * (nc + 1), h->stream) ||
+        hipMemsetAsync(h->qprefix, 0, sizeof(int) * NQROUNDS * (QSHARDS + 2), h->stream) ||
         hipMemsetAsync(h->qcount, 0, sizeof(int) * NQROUNDS * (QSHARDS + 1) * QSTRIDE, h->stream) ||
         hipMemsetAsync(h->pcounter, 0, sizeof(uint32_t), h->stream) ||
         hipMemsetAsync(h->stats, 0, sizeof(unsigned long long) * STAT_SHARDS * NSTAT, h->stream))
@@ -2117,9 +2103,11 @@ int pf2_step_info(pf2_handle h, long long* out, int cap) {
     long long vals[6] = {};
     vals[0] = cnt[3];
     vals[1] = cnt[0];
-    // queued per round of the last move (the FP64 path searches in one
-    // round), then the relocations of the last re-sort after a mesh move
-    for (int r = 0; r <= (mixed(h) ? MOVE_ROUNDS : 0); ++r) vals[2 + r] = pref[(size_t)r * (QSHARDS + 2) + QSHARDS + 1];
+    // queued in the last move, those of them searched for again (FP32-mixed),
+    // then the relocations of the last re-sort after a mesh move
+    vals[2] = pref[QSHARDS + 1];
+    if (mixed(h))
+        for (int t = 0; t < QSHARDS; ++t) vals[3] += pref[(QSHARDS + 2) + t];
     vals[4] = pref[(size_t)RESORT_QUEUE * (QSHARDS + 2) + QSHARDS + 1];
     vals[5] = arrivals;
     int k = 0;

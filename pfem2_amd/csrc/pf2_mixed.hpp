@@ -549,6 +549,8 @@ __device__ __forceinline__ void move32_body(const Grid& G, const DevMesh<DIM>& m
     // the particles that exist now end this advection with xi from the
     // local step or an inverse map in their cell (see k_resort32)
     if (do_move && G.bid == 0 && threadIdx.x == 0) w.counters[5] = (int)*w.particle_counter;
+    // (search32_body's count of repeated searches)
+    if (do_move && G.bid == 0) qu.prefix[(QSHARDS + 2) + threadIdx.x] = 0;
     const WaveLoop L = stride_loop(n, G);
     for (int base = L.begin; base < L.end; base += L.step) {
         const int i = base + lane;
@@ -613,35 +615,41 @@ __global__ void __launch_bounds__(256) k_move32(DevMesh<DIM> m, const float* __r
 }
 
 // FP64 relocation of queued particles (the reference rule), then the
-// remaining FP32 substeps
-// (LAST: the last round, which loops every particle to its end.  It runs
-// few wavefronts, so it takes the register budget of 2 per SIMD, no spills.
-// The first round is latency-bound with many wavefronts: in 2-D 4 per SIMD
-// runs it in 71 us per step on 101,785 cells, 3 in 79, 5 in 80; in 3-D 3 per
-// SIMD with spills were 3% faster than 2.)
-template <int DIM, bool LAST, int DEG = 1>
-__device__ __forceinline__ void search32_body(const Grid& G, const DevMesh<DIM>& m, const float* __restrict__ V32, const float* __restrict__ geo, const int* __restrict__ pcell, const Rec32& R, double* __restrict__ pvext, long long cap, const DevParams& pp, const DevWork& w, const DevQueues& qu, int round) {
+// remaining FP32 substeps, in one round with refilling lanes as in search_body
+// (pf2_kernels.hpp).  Bound by the latency of its dependent reads and the
+// relocations' FP64 instructions.  It takes the place of a round that parked
+// a particle again and a round that looped the rest to the end, whose
+// wavefronts waited for their longest chain: per step 165 -> 153 us on 101,785
+// quads with 2.4M particles, 459 -> 378 on 407,140 with 11M, 192 -> 138 on
+// 202,240 hexahedra, 35 -> 19 on a channel of 2,000 (one launch less).  4
+// wavefronts per SIMD in 2-D (3: the same, 5: spills, 5% slower), 3 in 3-D
+// (spills; 2 without: 4% slower).  The face-neighbour shortcut misses more
+// often on later crossings, and without it 101,785 quads take 148 us, but
+// 407,140 take 424.
+template <int DIM, int DEG = 1>
+__device__ __forceinline__ void search32_body(const Grid& G, const DevMesh<DIM>& m, const float* __restrict__ V32, const float* __restrict__ geo, const int* __restrict__ pcell, const Rec32& R, double* __restrict__ pvext, long long cap, const DevParams& pp, const DevWork& w, const DevQueues& qu) {
     constexpr int NV = Q1<DIM>::NV;
     constexpr int ND = QF<DIM, DEG>::ND;
     constexpr int NG = DIM == 2 ? 6 : 21;
     __shared__ int s_pref[QSHARDS + 2];
-    const int n = queue_prefix(qu, round, s_pref, G);
+    const int n = queue_prefix(qu, 0, s_pref, G);
     const int seg_end = w.counters[6] > 0 ? w.counters[7] : 0x7fffffff;
-    constexpr bool last = LAST;
     const float h32 = (float)pp.h;
     const int lane = threadIdx.x & (WAVE - 1);
-    const WaveLoop L = range_loop(n, G);
-    int lost = 0, searches = 0;
-    for (int base = L.begin; base < L.end; base += L.step) {
-        const int j = base + lane;
-        const bool valid = j < L.end;
-        const int2 e = valid ? queue_get(qu, round, s_pref, j) : make_int2(-1, -1);
-        const int i = e.x;
-        int c = e.y;
-        int s = valid ? qu.park_s[i] : 0;
-        int st = 0;
-        float xi[DIM], u[DIM];
-        if (valid) {
+    Refill F(qu, n, G);
+    int lost = 0, searches = 0, again = 0;
+    bool have = false, first = false;
+    int i = 0, c = 0, s = 0;
+    float xi[DIM], u[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) xi[d] = u[d] = 0.0f;
+    for (;;) {
+        const int j = F.next(have, lane);
+        if (j >= 0) {
+            const int2 e = queue_get(qu, s_pref, j);
+            i = e.x;
+            c = e.y;
+            s = qu.park_s[i];
             if constexpr (DIM == 2) {
                 const float4 pk = reinterpret_cast<const float4*>(qu.park_vext)[i];
                 xi[0] = pk.x;
@@ -653,67 +661,53 @@ __device__ __forceinline__ void search32_body(const Grid& G, const DevMesh<DIM>&
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) u[d] = (float)qu.park_vext[(size_t)d * cap + i];
             }
-            // 2-D: the found cell's vertices are kept for the next relocation;
-            // 3-D reloads them (register budget)
-            double P[NV][DIM];
+            have = first = true;
+        }
+        if (__ballot(have) == 0) break;
+        bool done = false;
+        if (have) {
+            double P[NV][DIM], Q[NV][DIM], xid[DIM], x[DIM], vext[DIM], r[DIM];
             load_vertices<DIM>(m, c, P);
-            for (;;) {
-                double Q[NV][DIM], xid[DIM], x[DIM], vext[DIM], r[DIM];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) {
+                xid[d] = (double)xi[d];
+                vext[d] = (double)u[d];
+            }
+            forward<DIM>(P, xid, x);
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) x[d] = x[d] + (double)(u[d] * h32);
+            c = relocate<DIM, true, false>(m, c, P, xid, vext, x, r, Q, searches, false);
+            done = c < 0;
+            if (c < 0) ++lost;
+            if (c >= 0) {
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) {
-                    xid[d] = (double)xi[d];
-                    vext[d] = (double)u[d];
+                    const float t = (float)r[d];
+                    xi[d] = t < 0.0f ? 0.0f : (t > 1.0f ? 1.0f : t);
                 }
-                forward<DIM>(P, xid, x);
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) x[d] = x[d] + (double)(u[d] * h32);
-                // (the last round's particles cross several cells and the
-                // face-neighbour shortcut misses more often: 58 us without it,
-                // 77 with it, on 101,785 cells)
-                const int cn = relocate<DIM, DIM == 3 || !LAST, false>(m, c, P, xid, vext, x, r, Q, searches, false);
-                if (cn >= 0) {
-#pragma unroll
-                    for (int d = 0; d < DIM; ++d) {
-                        const float t = (float)r[d];
-                        xi[d] = t < 0.0f ? 0.0f : (t > 1.0f ? 1.0f : t);
-                    }
-                    float g[NG], Vc[ND][DIM];
-                    load_cell32<DIM, DEG>(geo, V32, cn, g, Vc);
-                    ++s;
-                    st = advance32<DIM, DEG>(pp, h32, i, pvext, cap, xi, u, s, g, Vc);
-                }
-                if (cn < 0) {
-                    c = -1;
-                    ++lost;
-                    st = 0;
-                    break;
-                }
-                c = cn;
-                if (st == 0 || !last) break;
-                if constexpr (DIM == 2) {
-#pragma unroll
-                    for (int k = 0; k < NV; ++k)
-#pragma unroll
-                        for (int d = 0; d < DIM; ++d) P[k][d] = Q[k][d];
-                } else {
-                    load_vertices<DIM>(m, c, P);
-                }
+                float g[NG], Vc[ND][DIM];
+                load_cell32<DIM, DEG>(geo, V32, c, g, Vc);
+                ++s;
+                done = advance32<DIM, DEG>(pp, h32, i, pvext, cap, xi, u, s, g, Vc) == 0;
+                again += first && !done ? 1 : 0;
+                first = false;
             }
         }
-        if (!last) park32<DIM>(R, cap, w, qu, round + 1, L.shard, valid && st == 1, i, c, xi, u, s);
-        finish32<DIM>(pp, pcell, R, w, valid && st == 0, i, c, xi, seg_end);
+        finish32<DIM>(pp, pcell, R, w, done, i, c, xi, seg_end);
+        if (done) have = false;
     }
     wave_stat(w.stats, 0, lost);
     wave_stat(w.stats, 3, searches);
+    again = wave_sum(again);
+    if (lane == 0 && again) atomicAdd(qu.prefix + (QSHARDS + 2) + wave_shard(), again);
 }
 
-template <int DIM, bool LAST, int DEG = 1>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LAST ? 2 : (DIM == 2 ? 4 : 3)))) k_search_resume32(DevMesh<DIM> m, const float* __restrict__ V32,
+template <int DIM, int DEG = 1>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 4 : 3))) k_search_resume32(DevMesh<DIM> m, const float* __restrict__ V32,
                                                          const float* __restrict__ geo, const int* __restrict__ pcell,
                                                          Rec32 R, double* __restrict__ pvext,
-                                                         long long cap, DevParams pp, DevWork w, DevQueues qu,
-                                                         int round) {
-    search32_body<DIM, LAST, DEG>(hw_grid(), m, V32, geo, pcell, R, pvext, cap, pp, w, qu, round);
+                                                         long long cap, DevParams pp, DevWork w, DevQueues qu) {
+    search32_body<DIM, DEG>(hw_grid(), m, V32, geo, pcell, R, pvext, cap, pp, w, qu);
 }
 
 // deg: the velocity field's degree (1 or 2)
@@ -732,20 +726,13 @@ void launch_move32(hipStream_t s, int grid, DevMesh<DIM> m, const float* V32, co
 template <int DIM>
 void launch_search_resume32(hipStream_t s, int grid, DevMesh<DIM> m, const float* V32, const float* geo,
                             const int* pcell, Rec32 R, double* pvext, long long cap, DevParams pp, DevWork w,
-                            DevQueues qu, int round, int deg) {
-    const bool last = round == MOVE_ROUNDS;
-    if (deg == 2 && last)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume32<DIM, true, 2>), dim3(grid), dim3(256), 0, s, m, V32, geo,
-                           pcell, R, pvext, cap, pp, w, qu, round);
-    else if (deg == 2)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume32<DIM, false, 2>), dim3(grid), dim3(256), 0, s, m, V32,
-                           geo, pcell, R, pvext, cap, pp, w, qu, round);
-    else if (last)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume32<DIM, true>), dim3(grid), dim3(256), 0, s, m, V32, geo,
-                           pcell, R, pvext, cap, pp, w, qu, round);
+                            DevQueues qu, int deg) {
+    if (deg == 2)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume32<DIM, 2>), dim3(grid), dim3(256), 0, s, m, V32, geo, pcell,
+                           R, pvext, cap, pp, w, qu);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume32<DIM, false>), dim3(grid), dim3(256), 0, s, m, V32, geo,
-                           pcell, R, pvext, cap, pp, w, qu, round);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume32<DIM>), dim3(grid), dim3(256), 0, s, m, V32, geo, pcell, R,
+                           pvext, cap, pp, w, qu);
 }
 
 // k_cell_write (pf2_kernels.hpp) for FP32 records: the sums in FP32 with Kahan
@@ -1195,7 +1182,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM ==
     for (int base = L.begin; base < L.end; base += L.step) {
         const int j = base + lane;
         const bool valid = j < L.end;
-        const int2 e = valid ? queue_get(qu, RESORT_QUEUE, s_pref, j) : make_int2(0, -1);
+        const int2 e = valid ? queue_get(qu, s_pref, j) : make_int2(0, -1);
         const int i = e.x;
         int c = e.y;
         if (valid) {
