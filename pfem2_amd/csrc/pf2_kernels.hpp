@@ -190,7 +190,6 @@ struct DevWork {
                         // [5] id counter at the last advection (ids up to it hold an inverse-mapped xi),
                         // [6] slots of a pending layout (0: none; see k_cell_pend), [7] its segment end
     int* big;           // [0] number of cells listed for k_cell_big, then the cells
-    int* big2;          // the same for the cells that the second census pass (rows of GCAP_L) lists
     int pend_mark;      // census of a pending regroup: survivors' destinations get DEST_KEPT
     uint32_t* particle_counter;
     unsigned long long* stats;   // STAT_SHARDS rows: lost, deleted, spawned, searches, zero-weight
@@ -1143,10 +1142,10 @@ constexpr int GCAP_L = 128;          // the same for larger lattices
 // the census row of a lattice: GCAP for up to 16 parts, or when the
 // survivors of a full cell (MAX per part) leave 8 of GCAP's entries for
 // arrivals; else GCAP_L.  A cell whose candidates do not fit goes to
-// the second pass in rows of GCAP_L (and k_cell_big) either way; on the 5x5
+// k_cell_big either way; on the 5x5
 // lattice with MAX 2 of the moving-mesh workload the smaller rows (LDS for 8
 // workgroups per CU instead of 4) take the census from 0.62 to 0.40 ms per
-// step, the second pass and k_cell_big adding ~0.04 ms.
+// step, the listed cells adding ~0.04 ms.
 constexpr int SMALL_ROW_SURVIVORS = GCAP - 8;
 __host__ __device__ inline bool census_small_row(int nparts, int max_per_part) {
     return nparts <= 16 || (long long)max_per_part * nparts <= SMALL_ROW_SURVIVORS;
@@ -1215,8 +1214,8 @@ __device__ __forceinline__ void cell_count_body(const Grid& G, int n_cells, cons
     const bool by_count = nk <= NKC;
     for (int t = gl; t < NKC / 4; t += GS) s_cnt[g][t] = 0;
     int deleted = 0, arrivals = 0;
-    // LIST: the cells that the first pass listed (w.big), in rows of CAP;
-    // the cells that do not fit either are listed again in w.big2
+    // LIST: the cells that the first pass listed (w.big), in rows of CAP
+    // (those that do not fit either are left to cell_big_body)
     const int ncl = LIST ? w.big[0] : n_cells;
     for (int cb = G.bid * GROUPS; cb < ncl; cb += G.nblk * GROUPS) {
         const bool cv = cb + g < ncl;
@@ -1313,12 +1312,10 @@ __device__ __forceinline__ void cell_count_body(const Grid& G, int n_cells, cons
                 nsurv += surv ? 1 : 0;
                 if (surv) s_sid[g][j] = mi;
             }
-        else if (cv && gl == 0) {
-            // more than CAP candidates: census by k_cell_big (or by the
-            // second pass with larger rows)
-            int* list = LIST ? w.big2 : w.big;
-            const int slot = atomicAdd(&list[0], 1);
-            list[1 + slot] = c;
+        else if (!LIST && cv && gl == 0) {
+            // more than CAP candidates: census by k_cell_big
+            const int slot = atomicAdd(&w.big[0], 1);
+            w.big[1 + slot] = c;
         }
         wave_sync();
         if (counted)   // back to zero for the next cell (the words hold only this cell's parts)
@@ -1396,14 +1393,19 @@ __global__ void __launch_bounds__(256) k_cell_count(int n_cells, const int* __re
     cell_count_body<DIM, CAP, LIST>(hw_grid(), n_cells, old_off, pid, pp, w, reseed);
 }
 
-// The census of k_cell_count for the cells it listed (more than CAP
-// candidates): one 256-thread block per cell, candidates staged in LDS.
+// k_cell_big: the census of k_cell_count for the cells it listed, those of up
+// to GCAP_L candidates by a 16-lane group each, then the others by a 256-thread
+// block each, candidates staged in LDS.  Bound by the latency of a cell's chain
+// of dependent reads and barriers, so the groups' 16 cells a block matter: with
+// a block for every listed cell (and a launch of its own for the group pass on
+// lattices of more than 16 parts) the few thousand of 101,785 cells with a 4x4
+// lattice took 32 us, now 20.
 // A cell with more than BIGCAP candidates sets overflow flag 2 and keeps no
 // particle.
 constexpr int BIGCAP = 2048;
 
 template <int DIM>
-__device__ __forceinline__ void cell_big_body(const Grid& G, const int* __restrict__ old_off, const uint32_t* __restrict__ pid, const DevParams& pp, const DevWork& w, int reseed, const int* __restrict__ list) {
+__device__ __forceinline__ void cell_big_body(const Grid& G, const int* __restrict__ old_off, const uint32_t* __restrict__ pid, const DevParams& pp, const DevWork& w, int reseed) {
     __shared__ int s_idx[BIGCAP];
     __shared__ __align__(16) unsigned long long s_kid[BIGCAP];
     __shared__ __align__(16) uint32_t s_sid[BIGCAP];
@@ -1412,13 +1414,16 @@ __device__ __forceinline__ void cell_big_body(const Grid& G, const int* __restri
     if (state_dead(w.counters)) return;
     const int tid = threadIdx.x;
     const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
-    const int nbig = list[0];
+    const int nbig = w.big[0];
+    if (nbig == 0) return;
+    cell_count_body<DIM, GCAP_L, true>(G, 0, old_off, pid, pp, w, reseed);
     int deleted = 0;
     for (int b = G.bid; b < nbig; b += G.nblk) {
-        const int c = list[1 + b];
+        const int c = w.big[1 + b];
         const int n_st = old_off[c + 1] - old_off[c];
         const int na = w.arr_cnt[c];
         const int k = n_st + na;
+        if (k <= GCAP_L && na <= w.aslots) continue;   // done by a group
         const int kin = n_st + (na < w.aslots ? na : w.aslots);   // candidates in the old segment and slots
         if (k > BIGCAP) {
             for (int j = tid; j < kin; j += blockDim.x) w.spos[candidate(w, old_off, c, n_st, j)] = -1;
@@ -1519,11 +1524,10 @@ __device__ __forceinline__ void cell_big_body(const Grid& G, const int* __restri
     if (tid == 0 && deleted) stat_add(w.stats, 1, (unsigned long long)deleted);
 }
 
-// second: the cells listed by the second census pass (w.big2)
 template <int DIM>
 __global__ void __launch_bounds__(256) k_cell_big(const int* __restrict__ old_off, const uint32_t* __restrict__ pid,
-                                                  DevParams pp, DevWork w, int reseed, int second) {
-    cell_big_body<DIM>(hw_grid(), old_off, pid, pp, w, reseed, second ? w.big2 : w.big);
+                                                  DevParams pp, DevWork w, int reseed) {
+    cell_big_body<DIM>(hw_grid(), old_off, pid, pp, w, reseed);
 }
 
 // ---------------------------------------------------------------------------
@@ -1799,7 +1803,6 @@ __device__ __forceinline__ void finalize_block(int n_cells, const DevWork& w, in
     // a regroup consumes a pending layout; k_cell_pend has just set one up
     if (!keep_pending) w.counters[6] = 0;
     w.big[0] = 0;
-    w.big2[0] = 0;
 }
 
 __global__ void __launch_bounds__(QSHARDS) k_finalize(int n_cells, DevWork w, int* queue_count, int keep_pending) {
