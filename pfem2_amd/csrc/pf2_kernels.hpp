@@ -2354,6 +2354,21 @@ __global__ void k_to_node_major(const double* __restrict__ src, double* __restri
         for (int d = 0; d < DIM; ++d) dst[(size_t)i * DIM + d] = src[(size_t)d * n + i];
 }
 
+// particle vectors of a download: src (component-major, components `cap`
+// apart) to rows dst[n][DIM] for up to three arrays (blockIdx.y)
+struct RowCopies {
+    const double* src[3];
+    double* dst[3];
+};
+template <int DIM>
+__global__ void k_particle_rows(RowCopies r, long long n, long long cap) {
+    const double* __restrict__ s = r.src[blockIdx.y];
+    double* __restrict__ o = r.dst[blockIdx.y];
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) o[i * DIM + d] = s[(size_t)d * cap + i];
+}
+
 template <int DIM>
 __global__ void k_to_comp_major(const double* __restrict__ src, double* __restrict__ dst, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
