@@ -2035,7 +2035,7 @@ int pf2_calculate_loads(pf2_handle h, const double* V, const double* P, int n_fa
     if (n_faces)
         hipLaunchKernelGGL(k_loads_terms, dim3(grid_for(2LL * n_faces, 256)), dim3(256), 0, h->stream, dev_mesh<2>(h),
                            dF, n_faces, dV, dP, lp->mu, dT);
-    hipLaunchKernelGGL(k_loads_sum, dim3(1), dim3(64), 0, h->stream, dT, 2 * n_faces, dP, lp->rho, lp->u_mean,
+    hipLaunchKernelGGL(k_loads_sum, dim3(1), dim3(256), 0, h->stream, dT, 2 * n_faces, dP, lp->rho, lp->u_mean,
                        lp->diam, lp->dof_a, lp->dof_e, dO);
     if (hipGetLastError() != hipSuccess || hipMemcpyAsync(out5, dO, 5 * 8, hipMemcpyDeviceToHost, h->stream))
         return done(fail(PF2_E_HIP, "loads failed"));
