@@ -40,7 +40,7 @@ struct BatchSim {
     int* omap;                    // positions of cells whose survivors outnumber the slot row
     int* qcount;
     unsigned long long* tiles;    // tile sums of the offset scan
-    int ntiles;                   // tiles of SCAN_TILE entries of the n_cells + 1 counts
+    int ntiles;                   // tiles of SCAN_TILE entries of the n_cells + 1 counts; 0: no scan (CellSums)
 };
 
 constexpr int SCAN_TILE = 1024;   // entries per workgroup of the offset scan (4 per thread)
@@ -111,7 +111,8 @@ template <int DIM, int CAP>
 __global__ void __launch_bounds__(256) kb_count(BatchView<DIM> bv) {
     Grid G;
     const BatchSim<DIM>& S = bv.at(CAP == GCAP ? BK_COUNT : BK_COUNT_L, G);
-    cell_count_body<DIM, CAP>(G, S.m.n_cells, S.old_off, S.A.id, S.pp, S.w, 1);
+    __shared__ CountRows<CAP> rows;
+    cell_count_body<DIM, CAP>(rows, G, S.m.n_cells, S.old_off, S.A.id, S.pp, S.w, 1);
 }
 
 template <int DIM>

@@ -166,6 +166,31 @@ struct DevParams {
     int keep_vext;
 };
 
+// Offsets from the census's per-cell counts (fs_cnt: particles << 32 | new
+// ones, whose total stays below 2^32, so the low halves never carry): an
+// exclusive scan, two launches, or on meshes of up to SUMS_CELLS cells sums over
+// groups of cells, from which a write workgroup reads its own offset: the tiles
+// before its own and the cells before it in that, a few loads a lane at once.
+//   fine     per wavefront of k_cell_count (4 cells): the cells it counted
+//   tile     per TILE cells: k_cell_big adds the fine sums and the cells it
+//            counts itself (which fine leaves out).  Two sets: a census adds to
+//            one and the write after it clears the other for the next
+//            (counters[8] says which).
+// Two launches less are 3% of a step on 2,000 cells; from about 100,000 on the
+// sums cost more than the scan (per step on 407,140: census +14 us, write +17).
+// Tiles added by the census itself, an atomic per wavefront, cost it 40 us on
+// 101,785 cells: atomics on neighbouring sums serialise.
+constexpr int TILE = 256;
+constexpr int SUMS_CELLS = 128 * TILE;   // (two tiles a lane)
+struct CellSums {
+    unsigned long long* fine;   // null: scanned offsets
+    unsigned long long* tile;   // 2 sets of ntile
+    int nfine, ntile;
+    __device__ __forceinline__ unsigned long long* tiles(int set) const { return tile + (size_t)(set & 1) * ntile; }
+};
+inline int fine_sums(int n_cells) { return (n_cells + 15) / 16 * 4; }
+inline int tile_sums(int n_cells) { return (n_cells + TILE - 1) / TILE; }
+
 struct DevWork {
     int* dest;          // per particle: new cell or -1
     int* pkey;          // per particle: part key of the final position
@@ -175,20 +200,18 @@ struct DevWork {
     int aslots;
     int2* ovf;          // arrivals past a cell's slots: (particle, next entry) lists
     int* ovf_head;      // per cell: first overflow entry or -1
-    // per cell (n_cells + 1 for the scan): final count << 32 | spawns, and
-    // its exclusive scan (particle offset << 32 | spawn offset): one 64-bit
-    // scan gives both offsets (the spawn total stays below 2^32, so the low
-    // halves never carry)
-    unsigned long long* fs_cnt;
-    unsigned long long* fs_off;
-    int* new_off;       // n_cells + 1: particle offsets, written from fs_off by the cell writes
+    unsigned long long* fs_cnt;    // per cell: final count << 32 | spawns
+    unsigned long long* fs_off;    // its exclusive scan (n_cells + 1) where sums.fine is null
+    CellSums sums;      // else the counts' sums over groups of cells
+    int* new_off;       // n_cells + 1: particle offsets, written by the cell writes
     unsigned long long* hitmask;   // per cell: in-range parts that hold a particle
     int* nsurv;         // per cell: survivors
     double* partial;    // per cell: NV * (DIM + 1) projection sums
     int* counters;      // [0] n_particles, [1] arrivals of the last regroup, [2] overflow flags,
                         // [3] count before the last regroup, [4] overflow entries in use,
                         // [5] id counter at the last advection (ids up to it hold an inverse-mapped xi),
-                        // [6] slots of a pending layout (0: none; see k_cell_pend), [7] its segment end
+                        // [6] slots of a pending layout (0: none; see k_cell_pend), [7] its segment end,
+                        // [8] the set of CellSums of the current census
     int* big;           // [0] number of cells listed for k_cell_big, then the cells
     int pend_mark;      // census of a pending regroup: survivors' destinations get DEST_KEPT
     uint32_t* particle_counter;
@@ -262,6 +285,61 @@ __device__ __forceinline__ void gather_vertices(const DevMesh<DIM>& m, int c, do
 #pragma unroll
         for (int d = 0; d < DIM; ++d) P[k][d] = m.X[(size_t)gv * DIM + d];
     }
+}
+
+// sum over the wavefront (all lanes must call)
+__device__ __forceinline__ unsigned long long wave_sum64(unsigned long long v) {
+#pragma unroll
+    for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return v;
+}
+
+// this lane's share of a[lo] + ... + a[hi - 1]
+__device__ __forceinline__ unsigned long long lane_share(const unsigned long long* __restrict__ a, int lo, int hi,
+                                                         int lane, int lanes) {
+    unsigned long long v = 0;
+    for (int i = lo + lane; i < hi; i += 4 * lanes) {
+        unsigned long long q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = i + u * lanes < hi ? a[i + u * lanes] : 0ull;
+        v += (q[0] + q[1]) + (q[2] + q[3]);
+    }
+    return v;
+}
+
+// a count of cell c (one lane) added to its tile
+__device__ __forceinline__ void add_cell_sum(const DevWork& w, int set, int c, unsigned long long v) {
+    if (w.sums.fine && v) atomicAdd(&w.sums.tiles(set)[c / TILE], v);
+}
+
+// the fine sums into the tiles, a wavefront per tile (workgroups of 256)
+__device__ __forceinline__ void add_fine_sums(const DevWork& w, int set, int bid, int nblk) {
+    static_assert(TILE == 4 * WAVE, "a tile's fine sums: one per lane");
+    if (!w.sums.fine) return;
+    const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
+    for (int t = bid * 4 + wv; t < w.sums.ntile; t += nblk * 4) {
+        const int f = t * WAVE + lane;
+        const unsigned long long v = wave_sum64(f < w.sums.nfine ? w.sums.fine[f] : 0ull);
+        if (lane == 0 && v) atomicAdd(&w.sums.tiles(set)[t], v);
+    }
+}
+
+// exclusive prefix of fs_cnt at cell c0 (a whole wavefront calls)
+__device__ __forceinline__ unsigned long long cell_offset(const DevWork& w, int set, int c0) {
+    if (!w.sums.fine) return w.fs_off[c0];
+    const int lane = threadIdx.x & (WAVE - 1), t = c0 / TILE;
+    return wave_sum64(lane_share(w.sums.tiles(set), 0, t, lane, WAVE) + lane_share(w.fs_cnt, t * TILE, c0, lane, WAVE));
+}
+
+// sum of all cells (a whole wavefront calls)
+__device__ __forceinline__ unsigned long long cell_total(const DevWork& w, int set, int n_cells) {
+    if (!w.sums.fine) return w.fs_off[n_cells];
+    return wave_sum64(lane_share(w.sums.tiles(set), 0, w.sums.ntile, threadIdx.x & (WAVE - 1), WAVE));
+}
+
+// the first cell of a tile clears it in the set that the next census adds to
+__device__ __forceinline__ void clear_next_sums(const DevWork& w, int set, int c) {
+    if (w.sums.fine && c % TILE == 0) w.sums.tiles(set + 1)[c / TILE] = 0;
 }
 
 // u = sum_k N_k * F_k accumulated from zero over the cell's DoFs in order
@@ -1162,22 +1240,55 @@ __device__ __forceinline__ int load_agent(const int* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// sum / OR over a 16-lane group
+// sum / OR over a 16-lane group, all of whose lanes are active: a row of the
+// data-parallel primitives, rotated by 8, 4, 2, 1 (no LDS permutes)
+template <int N>
+__device__ __forceinline__ int row_ror(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x120 + N, 0xf, 0xf, true);
+}
+
 __device__ __forceinline__ int group_sum(int v) {
-#pragma unroll
-    for (int off = 1; off < GS; off <<= 1) v += __shfl_xor(v, off);
-    return v;
+    static_assert(GS == 16, "a group is a row of 16 lanes");
+    v += row_ror<8>(v);
+    v += row_ror<4>(v);
+    v += row_ror<2>(v);
+    return v + row_ror<1>(v);
+}
+
+__device__ __forceinline__ int group_or32(int v) {
+    v |= row_ror<8>(v);
+    v |= row_ror<4>(v);
+    v |= row_ror<2>(v);
+    return v | row_ror<1>(v);
 }
 
 __device__ __forceinline__ unsigned long long group_or(unsigned long long v) {
-#pragma unroll
-    for (int off = 1; off < GS; off <<= 1) {
-        const unsigned lo = __shfl_xor((unsigned)(v & 0xffffffffu), off);
-        const unsigned hi = __shfl_xor((unsigned)(v >> 32), off);
-        v |= ((unsigned long long)hi << 32) | lo;
-    }
-    return v;
+    const unsigned lo = (unsigned)group_or32((int)(unsigned)v), hi = (unsigned)group_or32((int)(unsigned)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
 }
+
+// Staged rows of the census in LDS, compacted to the cell's valid candidates
+// (stayers whose destination is c, then the arrivals): candidate index; part
+// key << 32 | id; id of a survivor, all ones otherwise.  Rows are padded to a
+// multiple of 4 entries with fill values (key all ones, id all ones), so the
+// scans read 16 bytes at a time, and their strides put the four groups of a
+// wavefront on different LDS banks.
+template <int CAP>
+struct CountRows {
+    // particles per part key counted in rows of more than 32, one byte each
+    // (four to a word, counted with word atomics; counts stay below CAP <= 128)
+    // (rows of GCAP count up to 64 keys: 2-D lattices up to 7 x 7, 3-D up to
+    // 3 x 3 x 3)
+    static constexpr int NKC = CAP == GCAP ? 64 : NKMAX;
+    // rows of GCAP on lattices of up to NKM keys: the row's entries of each
+    // part key as a bit mask
+    static constexpr int NKM = CAP == GCAP ? 36 : 0;
+    __attribute__((aligned(16))) unsigned long long kid[GROUPS][CAP + 2];
+    __attribute__((aligned(16))) uint32_t sid[GROUPS][CAP + 4];
+    int idx[GROUPS][CAP + 4];
+    unsigned int cnt[GROUPS][NKC / 4];
+    unsigned long long mask[NKM ? GROUPS : 1][NKM + 1];
+};
 
 // k_cell_count: per-cell part census (check_cell_for_empty_parts,
 // cylinder2D/pfem2particle.cpp:510-561).  Part index per direction is
@@ -1189,31 +1300,26 @@ __device__ __forceinline__ unsigned long long group_or(unsigned long long v) {
 // in LDS when there are at most CAP of them (GCAP or GCAP_L), else listed
 // for k_cell_big.
 template <int DIM, int CAP, bool LIST = false>
-__device__ __forceinline__ void cell_count_body(const Grid& G, int n_cells, const int* __restrict__ old_off, const uint32_t* __restrict__ pid, const DevParams& pp, const DevWork& w, int reseed) {
-    // Staged rows, compacted to the cell's valid candidates (stayers whose
-    // destination is c, then the arrivals): candidate index; part key << 32 |
-    // id; id of a survivor, all ones otherwise.  Rows are padded to a
-    // multiple of 4 entries with fill values (key all ones, id all ones), so
-    // the scans below read 16 bytes at a time, and their strides put the four
-    // groups of a wavefront on different LDS banks.
-    __shared__ int s_idx[GROUPS][CAP + 4];
-    __shared__ __align__(16) unsigned long long s_kid[GROUPS][CAP + 2];
-    __shared__ __align__(16) uint32_t s_sid[GROUPS][CAP + 4];
-    // per group: the cell's particles per part key, one byte each (four to
-    // a word, counted with word atomics; counts stay below CAP <= 128)
-    // (rows of GCAP count up to 64 keys: 2-D lattices up to 7 x 7, 3-D up to
-    // 3 x 3 x 3; the smaller LDS lets 8 instead of 7 workgroups share a CU)
-    constexpr int NKC = CAP == GCAP ? 64 : NKMAX;
-    __shared__ unsigned int s_cnt[GROUPS][NKC / 4];
+__device__ __forceinline__ void cell_count_body(CountRows<CAP>& rows, const Grid& G, int n_cells, const int* __restrict__ old_off, const uint32_t* __restrict__ pid, const DevParams& pp, const DevWork& w, int reseed) {
+    constexpr int NKC = CountRows<CAP>::NKC, NKM = CountRows<CAP>::NKM;
+    auto &s_idx = rows.idx;
+    auto &s_kid = rows.kid;
+    auto &s_sid = rows.sid;
+    auto &s_cnt = rows.cnt;
+    auto &s_mask = rows.mask;
     if (state_dead(w.counters)) return;
     const int g = threadIdx.x / GS, gl = threadIdx.x % GS;
     const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
     int nk = 1;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) nk *= pp.q[d] + 1;
-    const bool by_count = nk <= NKC;
+    const bool by_mask = nk <= NKM && reseed;
+    const bool by_count = nk <= NKC && !by_mask;
+    if constexpr (NKM > 0)
+        for (int t = gl; t < NKM; t += GS) s_mask[g][t] = 0;
     for (int t = gl; t < NKC / 4; t += GS) s_cnt[g][t] = 0;
     int deleted = 0, arrivals = 0;
+    const int set = w.counters[8];
     // LIST: the cells that the first pass listed (w.big), in rows of CAP
     // (those that do not fit either are left to cell_big_body)
     const int ncl = LIST ? w.big[0] : n_cells;
@@ -1283,6 +1389,13 @@ __device__ __forceinline__ void cell_count_body(const Grid& G, int n_cells, cons
         // 32 candidates the parts' counts first, then a scan of the row for
         // the particles of such parts (in shorter rows a scan for every
         // candidate costs less than the counting)
+        if constexpr (NKM > 0)
+            if (by_mask) {
+                if (small)
+                    for (int j = gl; j < nv; j += GS)
+                        atomicOr(&s_mask[g][(uint32_t)(s_kid[g][j] >> 32) & 0xffffu], 1ull << j);
+                wave_sync();
+            }
         const bool counted = small && reseed && by_count && nv > 32;
         if (counted) {
             for (int j = gl; j < nv; j += GS) {
@@ -1301,7 +1414,13 @@ __device__ __forceinline__ void cell_count_body(const Grid& G, int n_cells, cons
                 int rank = 0;
                 const uint32_t key = mk & 0xffffu;
                 const unsigned cnt = counted ? (s_cnt[g][key >> 2] >> (8 * (key & 3))) & 0xffu : 0xffu;
-                if (reseed && cnt > (unsigned)pp.max_per_part) {
+                if (by_mask) {
+                    if constexpr (NKM > 0) {
+                        unsigned long long mm = s_mask[g][key];
+                        if (__popcll(mm) > pp.max_per_part)
+                            for (; mm; mm &= mm - 1) rank += (uint32_t)s_kid[g][__ffsll((long long)mm) - 1] < mi ? 1 : 0;
+                    }
+                } else if (reseed && cnt > (unsigned)pp.max_per_part) {
                     for (int t = 0; t < nvr; t += 2) {
                         const ulonglong2 v = *reinterpret_cast<const ulonglong2*>(&s_kid[g][t]);
                         rank += ((uint32_t)(v.x >> 32) == mk && (uint32_t)v.x < mi) ? 1 : 0;
@@ -1318,6 +1437,9 @@ __device__ __forceinline__ void cell_count_body(const Grid& G, int n_cells, cons
             w.big[1 + slot] = c;
         }
         wave_sync();
+        if constexpr (NKM > 0)
+            if (by_mask && small)   // back to zero for the next cell
+                for (int j = gl; j < nv; j += GS) s_mask[g][(uint32_t)(s_kid[g][j] >> 32) & 0xffffu] = 0;
         if (counted)   // back to zero for the next cell (the words hold only this cell's parts)
             for (int j = gl; j < nv; j += GS) s_cnt[g][((uint32_t)(s_kid[g][j] >> 32) & 0xffffu) >> 2] = 0u;
         nsurv = group_sum(nsurv);
@@ -1373,12 +1495,20 @@ __device__ __forceinline__ void cell_count_body(const Grid& G, int n_cells, cons
             }
         wave_sync();
         hit = group_or(hit);
+        unsigned long long fs = 0;
         if (cv && small && gl == 0) {
             const int spawns = reseed ? __popcll(all & ~hit) : 0;
+            fs = ((unsigned long long)(nsurv + spawns) << 32) | (unsigned)spawns;
             w.hitmask[c] = reseed ? hit : all;
             w.nsurv[c] = nsurv;
-            w.fs_cnt[c] = ((unsigned long long)(nsurv + spawns) << 32) | (unsigned)spawns;
+            w.fs_cnt[c] = fs;
             deleted += nv - nsurv;
+            if (LIST) add_cell_sum(w, set, c, fs);
+        }
+        if (!LIST && w.sums.fine) {   // the wavefront's 4 cells
+            fs += __shfl_xor(fs, GS);
+            fs += __shfl_xor(fs, 2 * GS);
+            if ((threadIdx.x & (WAVE - 1)) == 0) w.sums.fine[c / 4] = fs;
         }
     }
     deleted = wave_sum(deleted);
@@ -1386,44 +1516,62 @@ __device__ __forceinline__ void cell_count_body(const Grid& G, int n_cells, cons
     if (!LIST) wave_stat(w.stats, 5, arrivals);
 }
 
-template <int DIM, int CAP, bool LIST = false>
+template <int DIM, int CAP>
 __global__ void __launch_bounds__(256) k_cell_count(int n_cells, const int* __restrict__ old_off,
                                                     const uint32_t* __restrict__ pid, DevParams pp, DevWork w,
                                                     int reseed) {
-    cell_count_body<DIM, CAP, LIST>(hw_grid(), n_cells, old_off, pid, pp, w, reseed);
+    __shared__ CountRows<CAP> rows;
+    cell_count_body<DIM, CAP>(rows, hw_grid(), n_cells, old_off, pid, pp, w, reseed);
 }
 
-// k_cell_big: the census of k_cell_count for the cells it listed, those of up
-// to GCAP_L candidates by a 16-lane group each, then the others by a 256-thread
-// block each, candidates staged in LDS.  Bound by the latency of a cell's chain
-// of dependent reads and barriers, so the groups' 16 cells a block matter: with
-// a block for every listed cell (and a launch of its own for the group pass on
-// lattices of more than 16 parts) the few thousand of 101,785 cells with a 4x4
-// lattice took 32 us, now 20.
+// k_cell_big: the census of k_cell_count for the cells it listed, candidates
+// staged in LDS: a 256-thread block for each while there are blocks enough,
+// and for more cells a 16-lane group for each of those with up to GCAP_L
+// candidates first.  Bound by the latency of a cell's chain of dependent reads
+// and barriers, so what counts is how many cells run at once: the few thousand
+// listed of 101,785 cells with a 4x4 lattice took 32 us with a block each and
+// take 21 with groups, the few hundred of 25,446 cells 12 with blocks and 17 with
+// groups.  One launch for both: the group pass of its own on lattices of more
+// than 16 parts cost 4 us.
 // A cell with more than BIGCAP candidates sets overflow flag 2 and keeps no
 // particle.
 constexpr int BIGCAP = 2048;
 
 template <int DIM>
 __device__ __forceinline__ void cell_big_body(const Grid& G, const int* __restrict__ old_off, const uint32_t* __restrict__ pid, const DevParams& pp, const DevWork& w, int reseed) {
-    __shared__ int s_idx[BIGCAP];
-    __shared__ __align__(16) unsigned long long s_kid[BIGCAP];
-    __shared__ __align__(16) uint32_t s_sid[BIGCAP];
+    struct BigRow {
+        __attribute__((aligned(16))) unsigned long long kid[BIGCAP];
+        __attribute__((aligned(16))) uint32_t sid[BIGCAP];
+        int idx[BIGCAP];
+    };
+    // (one after the other: 38 KB, four workgroups a CU)
+    __shared__ union {
+        CountRows<GCAP_L> rows;
+        BigRow row;
+    } lds;
+    auto &s_idx = lds.row.idx;
+    auto &s_kid = lds.row.kid;
+    auto &s_sid = lds.row.sid;
     __shared__ unsigned long long s_hit;
     __shared__ int s_nvalid, s_nsurv;
     if (state_dead(w.counters)) return;
     const int tid = threadIdx.x;
     const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
-    const int nbig = w.big[0];
+    const int nbig = w.big[0], set = w.counters[8];
+    add_fine_sums(w, set, (int)G.bid, (int)G.nblk);
     if (nbig == 0) return;
-    cell_count_body<DIM, GCAP_L, true>(G, 0, old_off, pid, pp, w, reseed);
+    const bool by_group = nbig > (int)G.nblk;
+    if (by_group) {
+        cell_count_body<DIM, GCAP_L, true>(lds.rows, G, 0, old_off, pid, pp, w, reseed);
+        __syncthreads();
+    }
     int deleted = 0;
     for (int b = G.bid; b < nbig; b += G.nblk) {
         const int c = w.big[1 + b];
         const int n_st = old_off[c + 1] - old_off[c];
         const int na = w.arr_cnt[c];
         const int k = n_st + na;
-        if (k <= GCAP_L && na <= w.aslots) continue;   // done by a group
+        if (by_group && k <= GCAP_L && na <= w.aslots) continue;   // done
         const int kin = n_st + (na < w.aslots ? na : w.aslots);   // candidates in the old segment and slots
         if (k > BIGCAP) {
             for (int j = tid; j < kin; j += blockDim.x) w.spos[candidate(w, old_off, c, n_st, j)] = -1;
@@ -1516,7 +1664,9 @@ __device__ __forceinline__ void cell_big_body(const Grid& G, const int* __restri
             const int spawns = reseed ? __popcll(all & ~hm) : 0;
             w.hitmask[c] = reseed ? hm : all;
             w.nsurv[c] = s_nsurv;
-            w.fs_cnt[c] = ((unsigned long long)(s_nsurv + spawns) << 32) | (unsigned)spawns;
+            const unsigned long long fs = ((unsigned long long)(s_nsurv + spawns) << 32) | (unsigned)spawns;
+            w.fs_cnt[c] = fs;
+            add_cell_sum(w, set, c, fs);
             deleted += s_nvalid - s_nsurv;
         }
         __syncthreads();
@@ -1588,22 +1738,38 @@ __device__ __forceinline__ void regroup_cells(RegroupCells<CB>& s, int cb, int n
     const int t = threadIdx.x;
     const int last = nc - cb < CB ? nc - cb : CB;
     bool past = false;
-    if (t < CB) {
+    if (t < WAVE) {
+        const int set = w.counters[8];
         const int c = cb + (t < last ? t : last - 1);
-        const unsigned long long fo = w.fs_off[c];
-        const int nfinal = (int)(w.fs_cnt[c] >> 32);
-        const long long out0 = (long long)(fo >> 32), b0 = __shfl(out0, 0);
+        const unsigned long long n = w.fs_cnt[c], v = t < last ? n : 0ull;
+        const int nsurv = w.nsurv[c];
+        const unsigned long long hit = w.hitmask[c];
+        const unsigned long long base = cell_offset(w, set, cb);
+        unsigned long long incl = v;   // particles and new ones up to cell t of the workgroup
+        if (w.sums.fine) {
+#pragma unroll
+            for (int h = 1; h < CB; h <<= 1) {
+                const unsigned long long o = __shfl_up(incl, h);
+                if (t >= h) incl += o;
+            }
+        } else {
+            incl = w.fs_off[c] - base + n;
+        }
         const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
-        if (t == 0) s.base = out0;
-        s.off[t] = (int)(out0 - b0) + (t < last ? 0 : nfinal);
-        if (t == CB - 1) s.off[CB] = (int)(out0 - b0) + nfinal;
-        s.nsurv[t] = w.nsurv[c];
-        s.empty[t] = all & ~w.hitmask[c];
-        s.spawn0[t] = (uint32_t)fo;
+        if (t == 0) s.base = (long long)(base >> 32);
+        if (t < CB) {
+            s.off[t] = (int)((incl - v) >> 32);
+            if (t == CB - 1) s.off[CB] = (int)(incl >> 32);
+            s.nsurv[t] = nsurv;
+            s.empty[t] = all & ~hit;
+            s.spawn0[t] = (uint32_t)(base + incl - v);
+        }
         if (t < last) {
+            const long long out0 = (long long)((base + incl - v) >> 32);
             w.new_off[c] = (int)out0;
-            past = w.nsurv[c] > w.aslots;
-            if (out0 + nfinal > cap) atomicOr(&w.counters[2], 1);
+            past = nsurv > w.aslots;
+            if (out0 + (long long)(v >> 32) > cap) atomicOr(&w.counters[2], 1);
+            clear_next_sums(w, set, c);
         }
     }
     if (__syncthreads_or(past)) {
@@ -1768,7 +1934,7 @@ __global__ void __launch_bounds__(256) k_cell_write(DevMesh<DIM> m, const int* _
     cell_write_body<DIM, GATHER, SUMS, DEG>(hw_grid(), m, old_off, A, B, pp, w, omap, partial);
 }
 
-// totals after the scans: particle count, id counter, statistics; resets the
+// totals after the census: particle count, id counter, statistics; resets the
 // queue counters for the next step (one workgroup of QSHARDS threads: k_finalize,
 // or the last workgroup of k_node in a fused step)
 __device__ __forceinline__ void finalize_block(int n_cells, const DevWork& w, int* queue_count,
@@ -1786,10 +1952,12 @@ __device__ __forceinline__ void finalize_block(int n_cells, const DevWork& w, in
     const int a = (int)w.stats[(size_t)t * NSTAT + 5];
     w.stats[(size_t)t * NSTAT + 5] = 0;
     if (a) atomicAdd(&s_arr, a);
+    const int set = w.counters[8];
+    const unsigned long long fo = cell_total(w, set, n_cells);
     __syncthreads();
     if (t != 0) return;
     w.counters[1] = s_arr;
-    const unsigned long long fo = w.fs_off[n_cells];
+    w.counters[8] = (set & 1) ^ 1;
     // a dead state publishes no particles (its total may exceed the capacity)
     const bool dead = state_dead(w.counters);
     const int total = dead ? 0 : (int)(fo >> 32);
@@ -1821,6 +1989,45 @@ __global__ void __launch_bounds__(QSHARDS) k_finalize(int n_cells, DevWork w, in
 // and the re-sort's regroup write is never done.  Any other use of the
 // particles first settles the layout (k_settle + a regroup without reseed).
 // (The census marks the survivors when DevWork::pend_mark is set.)
+
+// slots and segment end of a pending layout (the first wavefront of the grid)
+__device__ __forceinline__ void pend_slots(const DevWork& w, int nc, int seg_end, long long cap) {
+    if (blockIdx.x != 0 || threadIdx.x >= WAVE) return;
+    const unsigned long long tot = cell_total(w, w.counters[8], nc);
+    if (threadIdx.x != 0) return;
+    const long long slots = (long long)seg_end + (uint32_t)tot;
+    if (slots > cap) atomicOr(&w.counters[2], 1);
+    w.counters[6] = slots > cap ? 0 : (int)slots;
+    w.counters[7] = seg_end;
+}
+
+// offsets (particles << 32 | new particles) of the cell c0 + threadIdx.x of a
+// workgroup of 256 threads (all call; c0 a multiple of 256); clears its next sums
+__device__ __forceinline__ unsigned long long pend_offset(const DevWork& w, int c0, int nc) {
+    __shared__ unsigned long long s_base, s_w[256 / WAVE];
+    const int t = threadIdx.x, lane = t & (WAVE - 1), wv = t / WAVE, c = c0 + t;
+    if (!w.sums.fine) return c < nc ? w.fs_off[c] : 0ull;
+    const int set = w.counters[8];
+    const unsigned long long v = c < nc ? w.fs_cnt[c] : 0ull;
+    if (c < nc) clear_next_sums(w, set, c);
+    if (wv == 0) {
+        const unsigned long long b = cell_offset(w, set, c0);
+        if (lane == 0) s_base = b;
+    }
+    unsigned long long incl = v;
+#pragma unroll
+    for (int h = 1; h < WAVE; h <<= 1) {
+        const unsigned long long o = __shfl_up(incl, h);
+        if (lane >= h) incl += o;
+    }
+    if (lane == WAVE - 1) s_w[wv] = incl;
+    __syncthreads();
+    unsigned long long fo = s_base + incl - v;
+    for (int q = 0; q < wv; ++q) fo += s_w[q];
+    __syncthreads();
+    return fo;
+}
+
 template <int DIM, bool GATHER, int DEG = 1>
 __global__ void __launch_bounds__(256) k_cell_pend(DevMesh<DIM> m, const int* __restrict__ old_off, DevParticles A,
                                                    DevParams pp, DevWork w) {
@@ -1829,18 +2036,14 @@ __global__ void __launch_bounds__(256) k_cell_pend(DevMesh<DIM> m, const int* __
     if (state_dead(w.counters)) return;
     const int nc = m.n_cells;
     const int seg_end = old_off[nc];
-    const unsigned long long ftot = w.fs_off[nc];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const long long slots = (long long)seg_end + (uint32_t)ftot;
-        if (slots > A.cap) atomicOr(&w.counters[2], 1);
-        w.counters[6] = slots > A.cap ? 0 : (int)slots;
-        w.counters[7] = seg_end;
-    }
+    pend_slots(w, nc, seg_end, A.cap);
     // one cell per thread: new particles are few, and most cells only get
     // their resets
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += gridDim.x * blockDim.x) {
+    for (int c0 = blockIdx.x * 256; c0 < nc; c0 += gridDim.x * 256) {
+        const int c = c0 + threadIdx.x;
+        const unsigned long long fo = pend_offset(w, c0, nc);
+        if (c >= nc) continue;
         if ((uint32_t)w.fs_cnt[c] != 0u) {   // spawns, in lattice order
-            const unsigned long long fo = w.fs_off[c];
             const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
             const unsigned long long empty = all & ~w.hitmask[c];
             double P[NV][DIM], Vc[ND][DIM];

@@ -40,9 +40,9 @@ int fail(int code, const std::string& msg) {
     } while (0)
 
 // Timing ids of pf2_kernel_times / pf2_kernel_name.  The ids of kernels that
-// no longer exist (K_GROUP, K_QPREFIX, K_CELL_MAP, K_CELL_GATHER,
-// K_CELL_GATHER32) stay reserved, so that a caller's
-// numbering does not shift; they report no launches.
+// no longer exist (K_GROUP, K_QPREFIX, K_SEARCH_R1 to K_SEARCH32_R2,
+// K_CELL_MAP, K_CELL_GATHER, K_CELL_GATHER32) stay reserved, so that a
+// caller's numbering does not shift; they report no launches.
 enum KernelId {
     K_MOVE = 0, K_GROUP, K_CELL_COUNT, K_CELL_WRITE, K_SCAN, K_FINALIZE, K_PARTIALS, K_NODE, K_WALL,
     K_SEED, K_MISC, K_MOVE32, K_CELL_WRITE32, K_PARTIALS32, K_SEARCH, K_SEARCH32, K_QPREFIX,
@@ -150,6 +150,7 @@ struct pf2_handle_s {
     int2* ovf = nullptr;
     int aslots = 0;
     unsigned long long *fs_cnt = nullptr, *fs_off = nullptr;
+    pf2::CellSums sums{};   // meshes of up to SUMS_CELLS cells
     unsigned long long* hitmask = nullptr;
     int* nsurv = nullptr;
     double* partial = nullptr;
@@ -337,6 +338,7 @@ DevWork dev_work(pf2_handle_s* h) {
     w.ovf_head = h->ovf_head;
     w.fs_cnt = h->fs_cnt;
     w.fs_off = h->fs_off;
+    w.sums = h->sums;
     w.new_off = h->off[1 - h->cur_off];
     w.hitmask = h->hitmask;
     w.nsurv = h->nsurv;
@@ -496,10 +498,11 @@ int regroup(pf2_handle_s* h, int reseed, bool fuse_sums = false, bool defer_fina
     }
     {
         Timed t(h, K_CELL_BIG);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_big<DIM>), dim3(512), dim3(256), 0, h->stream, old_off,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_big<DIM>), dim3(1024), dim3(256), 0, h->stream, old_off,
                            h->buf[h->cur].id, pp, w, reseed);
     }
-    if (int r = scan(h, h->fs_cnt, h->fs_off, nc + 1)) return r;
+    if (!h->sums.fine)
+        if (int r = scan(h, h->fs_cnt, h->fs_off, nc + 1)) return r;
     if (pend) {
         // survivors marked and new particles placed in the current buffer;
         // the next move or a settle regroups them (FP64 handles)
@@ -873,9 +876,10 @@ size_t estimate_bytes(int dim, long long nc, long long nvt, long long nd, long l
     if (p->precision != PF2_FP32_MIXED) b += ndc * dim * 8 * 2;                          // FP64 cell V / dV copies
     b += nd * dim * 8 * 3;                                                              // V, V_old, staging
     b += (nc + 1) * 4 * 9 + nc * 4 * (1 + arrival_slots(dim, p));                     // per-cell work, arrival slots
-    b += nc * 8 + nc * 4 + ndc * (dim + 1) * 8 + 32;                                     // census, partials, counters
+    b += nc * 8 + nc * 4 + ndc * (dim + 1) * 8 + 64;                                     // census, partials, counters
     b += (size_t)NQROUNDS * (QSHARDS + 1) * QSTRIDE * 4 + (size_t)NQROUNDS * (QSHARDS + 2) * 4;
     b += 4 + (size_t)STAT_SHARDS * NSTAT * 8 + ((nc + 1 + SCAN_TILE - 1) / SCAN_TILE) * 8;
+    if (nc <= SUMS_CELLS) b += (fine_sums((int)nc) + 2 * (size_t)tile_sums((int)nc)) * 8;
     b += ndc * dim * 4 * 2 + nc * geo32_floats(dim) * 4;                                 // FP32 fields, geometry
     long long per = 4 + 4 + 3 * dim * 8;
     if (p->keep_velocity_ext) {
@@ -1022,7 +1026,7 @@ void batch_fill(pf2_handle_s* h, const double* field, BatchSim<DIM>& S, int* gri
     S.qcount = h->qcount;
     S.tiles = h->scan_tiles;
     const int nc = h->n_cells;
-    S.ntiles = (nc + 1 + SCAN_TILE - 1) / SCAN_TILE;
+    S.ntiles = h->sums.fine ? 0 : (nc + 1 + SCAN_TILE - 1) / SCAN_TILE;
     // each kernel's grid as the simulation's own step would launch it
     const int qgrid = grid_for(h->n_est / 2 + 1, 256, SEARCH_GRID);
     grid[BK_REFRESH] = grid_for(std::max((long long)nc * h->nd, (long long)h->n_dofs), 256, 4096);
@@ -1080,9 +1084,11 @@ int batch_step(pf2_batch_s* b, int n, const pf2_handle* hs, const double* const*
     if (tot[BK_COUNT_L])
         hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_count<DIM, GCAP_L>), dim3(tot[BK_COUNT_L]), dim3(256), 0, st, bv);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_big<DIM>), dim3(tot[BK_BIG]), dim3(256), 0, st, bv);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_scan_tiles<DIM>), dim3(tot[BK_TILES]), dim3(256), 0, st, bv);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_scan_tops<DIM>), dim3(n), dim3(256), 0, st, bv);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_scan_apply<DIM>), dim3(tot[BK_TILES]), dim3(256), 0, st, bv);
+    if (tot[BK_TILES]) {   // simulations past SUMS_CELLS
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_scan_tiles<DIM>), dim3(tot[BK_TILES]), dim3(256), 0, st, bv);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_scan_tops<DIM>), dim3(n), dim3(256), 0, st, bv);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_scan_apply<DIM>), dim3(tot[BK_TILES]), dim3(256), 0, st, bv);
+    }
     if (mx) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_write32<DIM>), dim3(tot[BK_WRITE]), dim3(256), 0, st, bv);
     else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_write<DIM>), dim3(tot[BK_WRITE]), dim3(256), 0, st, bv);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_finalize<DIM>), dim3(n), dim3(QSHARDS), 0, st, bv);
@@ -1285,6 +1291,8 @@ int pf2_create_in(const pf2_mesh* mesh, const pf2_params* params, long long capa
     } else if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(PF2_E_HIP, "hipStreamCreate failed"));
     const int nc = h->n_cells, nvt = h->n_vertices, nd = h->n_dofs, dim = h->dim;
+    h->sums.nfine = fine_sums(nc);
+    h->sums.ntile = tile_sums(nc);
     if (dalloc(&h->dX, (size_t)nvt * dim) || dalloc(&h->dcv, nck) || dalloc(&h->dcd, ndc) ||
         dalloc(&h->dstar_off, nvt + 1) || dalloc(&h->dstar_cell, h->star_cell.size()) ||
         dalloc(&h->dstar_dir, h->star_dir.size()) || dalloc(&h->ddof_off, nd + 1) ||
@@ -1295,8 +1303,10 @@ int pf2_create_in(const pf2_mesh* mesh, const pf2_params* params, long long capa
         dalloc(&h->dV, (size_t)nd * dim) ||
         dalloc(&h->dVold, (size_t)nd * dim) || dalloc(&h->dtmp, (size_t)nd * dim) || dalloc(&h->off[0], nc + 1) ||
         dalloc(&h->off[1], nc + 1) || dalloc(&h->arr_cnt, nc + 1) ||
-        dalloc(&h->arr_slot, (size_t)nc * h->aslots) || dalloc(&h->ovf_head, nc) || dalloc(&h->fs_cnt, nc + 1) || dalloc(&h->fs_off, nc + 1) || dalloc(&h->hitmask, nc) || dalloc(&h->nsurv, nc) ||
-        dalloc(&h->partial, ndc * (dim + 1)) || dalloc(&h->counters, 8) || dalloc(&h->big, nc + 1) ||
+        dalloc(&h->arr_slot, (size_t)nc * h->aslots) || dalloc(&h->ovf_head, nc) || dalloc(&h->fs_cnt, nc + 1) || dalloc(&h->fs_off, nc + 1) ||
+        (nc <= SUMS_CELLS && (dalloc(&h->sums.fine, fine_sums(nc)) || dalloc(&h->sums.tile, 2 * (size_t)tile_sums(nc)))) ||
+        dalloc(&h->hitmask, nc) || dalloc(&h->nsurv, nc) ||
+        dalloc(&h->partial, ndc * (dim + 1)) || dalloc(&h->counters, 16) || dalloc(&h->big, nc + 1) ||
         dalloc(&h->qcount, (size_t)NQROUNDS * (QSHARDS + 1) * QSTRIDE) ||
         dalloc(&h->qprefix, (size_t)NQROUNDS * (QSHARDS + 2)) ||
         dalloc(&h->pcounter, 1) || dalloc(&h->stats, STAT_SHARDS * NSTAT) ||
@@ -1330,8 +1340,9 @@ int pf2_create_in(const pf2_mesh* mesh, const pf2_params* params, long long capa
         hipMemsetAsync(h->off[1], 0, sizeof(int) * (nc + 1), h->stream) ||
         hipMemsetAsync(h->arr_cnt, 0, sizeof(int) * (nc + 1), h->stream) ||
         hipMemsetAsync(h->ovf_head, 0xff, sizeof(int) * nc, h->stream) ||
+        (h->sums.tile && hipMemsetAsync(h->sums.tile, 0, sizeof(unsigned long long) * 2 * (size_t)h->sums.ntile, h->stream)) ||
         hipMemsetAsync(h->fs_cnt, 0, sizeof(unsigned long long) * (nc + 1), h->stream) ||
-        hipMemsetAsync(h->counters, 0, sizeof(int) * 8, h->stream) ||
+        hipMemsetAsync(h->counters, 0, sizeof(int) * 16, h->stream) ||
         hipMemsetAsync(h->big, 0, sizeof(int) * (nc + 1), h->stream) ||
         hipMemsetAsync(h->qprefix, 0, sizeof(int) * NQROUNDS * (QSHARDS + 2), h->stream) ||
         hipMemsetAsync(h->qcount, 0, sizeof(int) * NQROUNDS * (QSHARDS + 1) * QSTRIDE, h->stream) ||
@@ -1360,7 +1371,7 @@ int pf2_destroy(pf2_handle h) {
                     h->dftol, h->dcellX, h->dcell_star, h->dcell_nbr, h->dvbnd, h->dvdof, h->dcellV, h->dcellDV, h->dV, h->dVold, h->dtmp, h->dV32,
                     h->dX0, h->dW, h->dcmoved,
                     h->dVold32, h->dgeo32, h->off[0], h->off[1], h->arr_cnt, h->arr_slot, h->ovf_head, h->fs_cnt,
-                    h->fs_off, h->hitmask, h->nsurv, h->partial, h->counters, h->big, h->qcount, h->qprefix,
+                    h->fs_off, h->sums.fine, h->sums.tile, h->hitmask, h->nsurv, h->partial, h->counters, h->big, h->qcount, h->qprefix,
                     h->pcounter, h->stats, h->scan_tmp, h->scan_tiles};
     if (!h->in_block)
         for (void* p : ptrs)

@@ -1232,17 +1232,13 @@ __global__ void __launch_bounds__(256) k_cell_pend32(int n_cells, const int* __r
     if (state_dead(w.counters)) return;
     const int nc = n_cells;
     const int seg_end = old_off[nc];
-    const unsigned long long ftot = w.fs_off[nc];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const long long slots = (long long)seg_end + (uint32_t)ftot;
-        if (slots > cap) atomicOr(&w.counters[2], 1);
-        w.counters[6] = slots > cap ? 0 : (int)slots;
-        w.counters[7] = seg_end;
-    }
+    pend_slots(w, nc, seg_end, cap);
     // one cell per thread, as in k_cell_pend
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += gridDim.x * blockDim.x) {
+    for (int c0 = blockIdx.x * 256; c0 < nc; c0 += gridDim.x * 256) {
+        const int c = c0 + threadIdx.x;
+        const unsigned long long fo = pend_offset(w, c0, nc);
+        if (c >= nc) continue;
         if ((uint32_t)w.fs_cnt[c] != 0u) {   // spawns, in lattice order
-            const unsigned long long fo = w.fs_off[c];
             const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
             const unsigned long long empty = all & ~w.hitmask[c];
             double Vc[ND][DIM];
