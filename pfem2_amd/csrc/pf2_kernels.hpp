@@ -357,6 +357,25 @@ __device__ __forceinline__ void interp(const double (*Fc)[DIM], const double* xi
         for (int d = 0; d < DIM; ++d) u[d] += N[k] * Fc[k][d];
 }
 
+// the same with one node at a time (at(k): the velocity of node k), for a rare
+// point: the nodes of a degree-2 cell held at once take the registers of a
+// whole kernel (k_cell_write on degree-2 hexahedra: 408 -> 248,
+// 151 -> 130 us per step on 68,992)
+template <int DIM, int DEG, class F>
+__device__ __forceinline__ void interp_each(const double* xi, double* u, F at) {
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) u[d] = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < QF<DIM, DEG>::ND; ++k) {
+        ShapeOne<DIM, DEG> N;
+        N.init(k);
+        const double nk = N(xi);
+        const auto* f = at(k);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) u[d] += nk * (double)f[d];
+    }
+}
+
 template <int DIM>
 __device__ __forceinline__ int part_key(const DevParams& pp, const double* xi) {
     // bits 0-15: part index with the phantom value q_d (the grouping key);
@@ -1826,15 +1845,29 @@ __device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM
     constexpr int ND = QF<DIM, DEG>::ND;
     constexpr int CH = 256;   // positions per pass
     __shared__ RegroupCells<S::CB> s;
-    __shared__ double s_xi[SUMS ? DIM : 1][SUMS ? CH : 1];
+    // degree-2 hexahedra: each particle's 1-D factors in LDS, from which a lane
+    // multiplies its 7 nodes' shape values; the nodes' coefficients instead took
+    // 168 registers a lane, 2 wavefronts per SIMD (130 -> 98 us per step on
+    // 68,992)
+    constexpr bool TAB = SUMS && DIM == 3 && DEG == 2;
+    static_assert(!TAB || S::LPC % (DIM + 1) == 0, "a lane's sums are of one component");
+    __shared__ double s_xi[SUMS && !TAB ? DIM : 1][SUMS && !TAB ? CH : 1];
+    __shared__ double s_l[TAB ? CH : 1][3 * DIM];
     __shared__ double s_v[SUMS ? DIM : 1][SUMS ? CH : 1];
     if (state_dead(w.counters)) return;
     const int tid = threadIdx.x, g = tid / S::LPC, gl = tid % S::LPC;
     // the lane's sums: vertex a / (DIM + 1), component a % (DIM + 1) (the last
     // one the weight) for a = gl, gl + LPC, ...
-    ShapeOne<DIM, DEG> sh[S::NA];
-    int comp[S::NA];
-    if constexpr (SUMS)
+    ShapeOne<DIM, DEG> sh[TAB ? 1 : S::NA];
+    int comp[S::NA], fac[TAB ? S::NA : 1][DIM];
+    if constexpr (TAB)
+#pragma unroll
+        for (int u = 0; u < S::NA; ++u) {
+            const int a = gl + u * S::LPC;
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) fac[u][d] = 3 * d + q2_axis(DIM, (a < S::NACC ? a : 0) / (DIM + 1), d);
+        }
+    else if constexpr (SUMS)
 #pragma unroll
         for (int u = 0; u < S::NA; ++u) {
             const int a = gl + u * S::LPC;
@@ -1870,12 +1903,22 @@ __device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM
                 // a new particle: most wavefronts hold one or two, so its
                 // loads go out behind the records' and before any wait
                 if (src < 0) {
-                    double P[NV][DIM], Vc[ND][DIM];
-                    load_cell<DIM, GATHER, DEG>(m, c, P, Vc);
+                    double P[NV][DIM];
                     id = *w.particle_counter + s.spawn0[k] + (uint32_t)(p - s.off[k] - s.nsurv[k]) + 1u;
                     lattice_point<DIM>(pp, -1 - src, xi);
-                    forward<DIM>(P, xi, x);
-                    interp<DIM, DEG>(Vc, xi, v);
+                    if constexpr (DEG == 1) {
+                        double Vc[ND][DIM];
+                        load_cell<DIM, GATHER, DEG>(m, c, P, Vc);
+                        forward<DIM>(P, xi, x);
+                        interp<DIM, DEG>(Vc, xi, v);
+                    } else {
+                        load_vertices<DIM>(m, c, P);
+                        forward<DIM>(P, xi, x);
+                        interp_each<DIM, DEG>(xi, v, [&](int n) {
+                            return GATHER ? m.Vn + (size_t)m.cd[(size_t)c * ND + n] * DIM
+                                          : m.cellV + ((size_t)c * ND + n) * DIM;
+                        });
+                    }
 #pragma unroll
                     for (int d = 0; d < DIM; ++d) e[d] = 0.0;
                 }
@@ -1888,10 +1931,11 @@ __device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM
                     B.xi[(size_t)d * B.cap + o] = xi[d];
                     B.v[(size_t)d * B.cap + o] = v[d];
                     if (pp.keep_vext) B.vext[(size_t)d * B.cap + o] = e[d];
-                    if constexpr (SUMS) {
-                        s_xi[d][tid] = xi[d];
-                        s_v[d][tid] = v[d];
-                    }
+                    if constexpr (TAB)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) s_l[tid][3 * d + q] = lag2(q, xi[d]);
+                    else if constexpr (SUMS) s_xi[d][tid] = xi[d];
+                    if constexpr (SUMS) s_v[d][tid] = v[d];
                 }
             }
             if constexpr (SUMS) {
@@ -1899,6 +1943,15 @@ __device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM
                 const int q0 = s.off[g] > p0 ? s.off[g] - p0 : 0;
                 const int e = s.off[g + 1] < total ? s.off[g + 1] : total;
                 const int q1 = e - p0 < CH ? e - p0 : CH;
+                if constexpr (TAB) {
+                    const int cp = gl % (DIM + 1);
+                    for (int q = q0; q < q1; ++q) {
+                        const double vc = cp < DIM ? s_v[cp < DIM ? cp : 0][q] : 1.0;
+#pragma unroll
+                        for (int u = 0; u < S::NA; ++u)
+                            acc[u] += s_l[q][fac[u][0]] * s_l[q][fac[u][1]] * s_l[q][fac[u][2]] * vc;
+                    }
+                } else
                 for (int q = q0; q < q1; ++q) {
                     double xi[DIM], v[DIM];
 #pragma unroll

@@ -789,14 +789,19 @@ __device__ __forceinline__ void cell_write32_body(const Grid& G, int n_cells, co
                     for (int d = 0; d < DIM; ++d) e[d] = pp.keep_vext ? avext[(size_t)d * cap + src] : 0.0;
                 }
                 if (src < 0) {   // a new particle
-                    double xi[DIM], Vc[ND][DIM], v[DIM];
-#pragma unroll
-                    for (int n = 0; n < ND; ++n)
-#pragma unroll
-                        for (int d = 0; d < DIM; ++d) Vc[n][d] = (double)V32c[((size_t)c * ND + n) * DIM + d];
+                    double xi[DIM], v[DIM];
                     id = *w.particle_counter + s.spawn0[k] + (uint32_t)(p - s.off[k] - s.nsurv[k]) + 1u;
                     lattice_point<DIM>(pp, -1 - src, xi);
-                    interp<DIM, DEG>(Vc, xi, v);
+                    if constexpr (DEG == 1) {
+                        double Vc[ND][DIM];
+#pragma unroll
+                        for (int n = 0; n < ND; ++n)
+#pragma unroll
+                            for (int d = 0; d < DIM; ++d) Vc[n][d] = (double)V32c[((size_t)c * ND + n) * DIM + d];
+                        interp<DIM, DEG>(Vc, xi, v);
+                    } else {
+                        interp_each<DIM, DEG>(xi, v, [&](int n) { return V32c + ((size_t)c * ND + n) * DIM; });
+                    }
                     if constexpr (DIM == 2) {
                         a = make_float4((float)xi[0], (float)xi[1], (float)v[0], (float)v[1]);
                     } else {
