@@ -2625,6 +2625,16 @@ __global__ void k_particle_rows(RowCopies r, long long n, long long cap) {
         for (int d = 0; d < DIM; ++d) o[i * DIM + d] = s[(size_t)d * cap + i];
 }
 
+// the field and the overflow flags to host memory
+template <int DIM>
+__global__ void k_field_out(const double* __restrict__ src, double* __restrict__ dst, int n,
+                            const int* __restrict__ counters, int* __restrict__ flags) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *flags = counters[2];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) dst[(size_t)d * n + i] = src[(size_t)i * DIM + d];
+}
+
 template <int DIM>
 __global__ void k_to_comp_major(const double* __restrict__ src, double* __restrict__ dst, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)

@@ -124,7 +124,11 @@ constexpr int kBatchAhead = 3;   // batched steps queued ahead (below the batch'
 constexpr int kSizeClasses = 3;
 int size_class(int n_cells) { return n_cells < 16384 ? 0 : (n_cells < 131072 ? 1 : 2); }
 
+__attribute__((visibility("hidden"))) void pf2_stage_user(bool add);   // pf2_lib.hip: staging blocks outlive the requests' handles
+
 struct pf2_server_s {
+    pf2_server_s() { pf2_stage_user(true); }
+    ~pf2_server_s() { pf2_stage_user(false); }
     pf2_server_config cfg{};
     BatchGroup groups[2][2][kSizeClasses];   // [dim - 2][precision][size class]
     char* block = nullptr;
