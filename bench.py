@@ -161,13 +161,12 @@ def kernel_bytes(name, info, m, dim=2, vext=False):
         # the relocations of the re-sort (q[2]): entry, record and vertices
         # in; x, xi, destination and part key out
         return int(q[2] * (8 + 4 + 3 * dim * 8 + nv * dim * 8 + 2 * dim * 8 + 8))
-    if name.startswith("k_search_resume"):
-        # one launch per relocation round; round r handles q[r] particles
-        mm = re.match(r"(k_search_resume(?:32)?)(?:_r(\d))?$", name)
-        base, r = mm.group(1), int(mm.group(2) or 0)
-        wx = 8 if base == "k_search_resume" else 4
-        per = 8 + 4 + 4 + dim * wx * (2 if base == "k_search_resume" else 1) + 8 * dim + 8 + dim * wx
-        return int(q[r] * per) if r < len(q) else None
+    if name in ("k_search_resume", "k_search_resume32"):
+        # per queued particle: entry, parked record; reference point,
+        # destination and part key out
+        wx = 8 if name == "k_search_resume" else 4
+        per = 8 + 4 + 4 + dim * wx * (2 if name == "k_search_resume" else 1) + 8 * dim + 8 + dim * wx
+        return int(q[0] * per)
     if name == "k_cell_count":
         return (n0 + arr) * 12 + arr * 4 + n0 * 4 + nc * (8 + 4 + 4 + 20)
     if name in ("k_cell_write", "k_cell_write32"):
@@ -486,8 +485,7 @@ def roofline(res, m, profile=None):
     per_step = res["kernels_ms_per_step"]
     fam = {}
     for key, v in per_step.items():
-        f = re.sub(r"_r\d$", "", key) if key.startswith("k_search_resume_r") else key
-        fam.setdefault(f, []).append(key)
+        fam.setdefault(key, []).append(key)
     dom = max(fam, key=lambda f: sum(per_step[k] for k in fam[f]))
     members = fam[dom]
     vext = res.get("keep_vext", False)
