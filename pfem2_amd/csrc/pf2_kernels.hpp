@@ -206,7 +206,7 @@ struct DevWork {
     int* new_off;       // n_cells + 1: particle offsets, written by the cell writes
     unsigned long long* hitmask;   // per cell: in-range parts that hold a particle
     int* nsurv;         // per cell: survivors
-    double* partial;    // per cell: NV * (DIM + 1) projection sums
+    double* partial;    // projection sums, DIM + 1 per cell and DoF of it (partial_at)
     int* counters;      // [0] n_particles, [1] arrivals of the last regroup, [2] overflow flags,
                         // [3] count before the last regroup, [4] overflow entries in use,
                         // [5] id counter at the last advection (ids up to it hold an inverse-mapped xi),
@@ -374,6 +374,23 @@ __device__ __forceinline__ void interp_each(const double* xi, double* u, F at) {
 #pragma unroll
         for (int d = 0; d < DIM; ++d) u[d] += nk * (double)f[d];
     }
+}
+
+// Position of sum a (DoF a / (DIM + 1), component a % (DIM + 1)) of cell c
+// among the cells' projection sums.  Degree-1 hexahedra: DoF by DoF, then cell
+// by cell, so that k_node's neighbouring nodes, which read the same DoF of
+// neighbouring cells, share 128-byte lines; with a cell's sums together each line
+// was fetched by several XCDs for a quarter of it (k_node 31 -> 16 us per step on
+// 202,240, the write the same).  Elsewhere a cell's sums lie together: the
+// scattered stores cost the write more than k_node gains (68,992 degree-2
+// hexahedra: 97 -> 129 and 36 -> 23 us; 407,140 quads: 507 -> 520 and 25 -> 20).
+template <int DIM, int DEG>
+__device__ __forceinline__ size_t partial_at(int n_cells, int c, int a) {
+    if constexpr (DIM == 3 && DEG == 1) {
+        const int k = a / (DIM + 1);
+        return ((size_t)k * n_cells + c) * (DIM + 1) + (a - k * (DIM + 1));
+    }
+    return (size_t)c * (QF<DIM, DEG>::ND * (DIM + 1)) + a;
 }
 
 template <int DIM>
@@ -1975,7 +1992,7 @@ __device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM
             if (cb + g < m.n_cells)
 #pragma unroll
                 for (int u = 0; u < S::NA; ++u)
-                    if (gl + u * S::LPC < S::NACC) partial[(size_t)(cb + g) * S::NACC + gl + u * S::LPC] = acc[u];
+                    if (gl + u * S::LPC < S::NACC) partial[partial_at<DIM, DEG>(m.n_cells, cb + g, gl + u * S::LPC)] = acc[u];
         __syncthreads();   // s is refilled
     }
 }
@@ -2241,7 +2258,7 @@ __device__ __forceinline__ void partials_body(const Grid& G, int n_cells, const 
         if (cv)
 #pragma unroll
             for (int u = 0; u < NA; ++u)
-                if (gl + u * PGS < NACC) partial[(size_t)c * NACC + gl + u * PGS] = acc[u];
+                if (gl + u * PGS < NACC) partial[partial_at<DIM, DEG>(n_cells, c, gl + u * PGS)] = acc[u];
     }
 }
 
@@ -2258,7 +2275,6 @@ template <int DIM, bool FIN, int DEG = 1>
 __device__ __forceinline__ void node_body(const Grid& G, const DevMesh<DIM>& m, const double* __restrict__ partial, double* __restrict__ V, double* __restrict__ Vold, unsigned long long* stats, const DevWork& w, int* queue_count) {
     constexpr int NV = Q1<DIM>::NV;   // cells per chunk
     constexpr int ND = QF<DIM, DEG>::ND;
-    constexpr int NACC = ND * (DIM + 1);
     // FIN (a step whose regroup left its bookkeeping for later): the last
     // workgroup runs it; it depends on the cell write only, as the node sums do
     if (FIN && G.bid == G.nblk - 1) {
@@ -2283,7 +2299,7 @@ __device__ __forceinline__ void node_body(const Grid& G, const DevMesh<DIM>& m, 
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
                 const int c = ck[q] >= 0 ? ck[q] / ND : 0, k = ck[q] >= 0 ? ck[q] - c * ND : 0;
-                const double* p = partial + (size_t)c * NACC + k * (DIM + 1);
+                const double* p = partial + partial_at<DIM, DEG>(m.n_cells, c, k * (DIM + 1));
 #pragma unroll
                 for (int d = 0; d <= DIM; ++d) pv[q][d] = ck[q] >= 0 ? p[d] : 0.0;
             }

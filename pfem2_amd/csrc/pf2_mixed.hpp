@@ -866,7 +866,8 @@ __device__ __forceinline__ void cell_write32_body(const Grid& G, int n_cells, co
 #pragma unroll
                 for (int u = 0; u < S::NA; ++u)
                     if (gl + u * S::LPC < S::NACC)
-                        partial[(size_t)(cb + g) * S::NACC + gl + u * S::LPC] = (double)sum[u] - (double)cmp[u];
+                        partial[partial_at<DIM, DEG>(n_cells, cb + g, gl + u * S::LPC)] =
+                            (double)sum[u] - (double)cmp[u];
         __syncthreads();   // s is refilled
     }
 }
@@ -951,7 +952,7 @@ __device__ __forceinline__ void partials32_body(const Grid& G, int n_cells, cons
         }
 #pragma unroll
         for (int u = 0; u < NA; ++u)
-            if (cv && gl + u * PGS < NACC) partial[(size_t)c * NACC + gl + u * PGS] = (double)sum[u] - (double)cmp[u];
+            if (cv && gl + u * PGS < NACC) partial[partial_at<DIM, DEG>(n_cells, c, gl + u * PGS)] = (double)sum[u] - (double)cmp[u];
     }
 }
 
