@@ -1760,13 +1760,20 @@ struct RegroupCells {
     int nsurv[CB];
     unsigned long long empty[CB];    // parts to reseed
     uint32_t spawn0[CB];             // new particles of earlier cells
+    int dead;                        // the state was dead: nothing to write
 };
 
-// Fills s for the cells cb, cb + 1, ... (all threads call; a barrier at the
-// end): offsets, overflow flag, and for cells whose survivors outnumber the
-// slot row (rare) their sources in omap.
+// Fills s for the cells cb, cb + 1, ... (all threads call; barriers inside,
+// none after the resets at the end): offsets, overflow flag, and for cells
+// whose survivors outnumber the slot row (rare) their sources in omap.
+// False: the state is dead.  Other workgroups of the same launch raise that
+// flag, so the first wavefront reads it once and decides for the workgroup:
+// were each wavefront to read it, the first could leave while the others,
+// their barrier no longer waiting for it, took the cells from LDS that it
+// never wrote.  (The cells' counts are read either way: they are in range in
+// a dead state too.)
 template <int CB>
-__device__ __forceinline__ void regroup_cells(RegroupCells<CB>& s, int cb, int nc, const int* __restrict__ old_off,
+__device__ __forceinline__ bool regroup_cells(RegroupCells<CB>& s, int cb, int nc, const int* __restrict__ old_off,
                                               long long cap, const DevParams& pp, const DevWork& w,
                                               int* __restrict__ omap) {
     constexpr int LPC = 256 / CB;
@@ -1775,6 +1782,7 @@ __device__ __forceinline__ void regroup_cells(RegroupCells<CB>& s, int cb, int n
     const int last = nc - cb < CB ? nc - cb : CB;
     bool past = false;
     if (t < WAVE) {
+        const bool dead = (__builtin_amdgcn_readfirstlane(load_agent(&w.counters[2])) & DEAD_FLAGS) != 0;
         const int set = w.counters[8];
         const int c = cb + (t < last ? t : last - 1);
         const unsigned long long n = w.fs_cnt[c], v = t < last ? n : 0ull;
@@ -1792,7 +1800,10 @@ __device__ __forceinline__ void regroup_cells(RegroupCells<CB>& s, int cb, int n
             incl = w.fs_off[c] - base + n;
         }
         const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
-        if (t == 0) s.base = (long long)(base >> 32);
+        if (t == 0) {
+            s.base = (long long)(base >> 32);
+            s.dead = dead;
+        }
         if (t < CB) {
             s.off[t] = (int)((incl - v) >> 32);
             if (t == CB - 1) s.off[CB] = (int)(incl >> 32);
@@ -1800,7 +1811,7 @@ __device__ __forceinline__ void regroup_cells(RegroupCells<CB>& s, int cb, int n
             s.empty[t] = all & ~hit;
             s.spawn0[t] = (uint32_t)(base + incl - v);
         }
-        if (t < last) {
+        if (t < last && !dead) {
             const long long out0 = (long long)((base + incl - v) >> 32);
             w.new_off[c] = (int)out0;
             past = nsurv > w.aslots;
@@ -1808,7 +1819,9 @@ __device__ __forceinline__ void regroup_cells(RegroupCells<CB>& s, int cb, int n
             clear_next_sums(w, set, c);
         }
     }
-    if (__syncthreads_or(past)) {
+    const bool any_past = __syncthreads_or(past);
+    if (s.dead) return false;
+    if (any_past) {
         const int g = t / LPC, gl = t % LPC, c = cb + g;
         if (g < last && s.nsurv[g] > w.aslots) {
             const int n_st = old_off[c + 1] - old_off[c], na = w.arr_cnt[c];
@@ -1832,6 +1845,7 @@ __device__ __forceinline__ void regroup_cells(RegroupCells<CB>& s, int cb, int n
         w.arr_cnt[cb + t] = 0;
         w.ovf_head[cb + t] = -1;
     }
+    return true;
 }
 
 // source of the output position p after s.base: a particle, or for a new one
@@ -1871,7 +1885,6 @@ __device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM
     __shared__ double s_xi[SUMS && !TAB ? DIM : 1][SUMS && !TAB ? CH : 1];
     __shared__ double s_l[TAB ? CH : 1][3 * DIM];
     __shared__ double s_v[SUMS ? DIM : 1][SUMS ? CH : 1];
-    if (state_dead(w.counters)) return;
     const int tid = threadIdx.x, g = tid / S::LPC, gl = tid % S::LPC;
     // the lane's sums: vertex a / (DIM + 1), component a % (DIM + 1) (the last
     // one the weight) for a = gl, gl + LPC, ...
@@ -1893,7 +1906,7 @@ __device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM
             sh[u].init(kk);
         }
     for (int cb = G.bid * S::CB; cb < m.n_cells; cb += G.nblk * S::CB) {
-        regroup_cells<S::CB>(s, cb, m.n_cells, old_off, A.cap, pp, w, omap);
+        if (!regroup_cells<S::CB>(s, cb, m.n_cells, old_off, A.cap, pp, w, omap)) return;
         const long long base = s.base;
         const int total = base + s.off[S::CB] <= B.cap ? s.off[S::CB] : (int)(B.cap > base ? B.cap - base : 0);
         double acc[S::NA];

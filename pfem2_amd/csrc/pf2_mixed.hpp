@@ -752,7 +752,6 @@ __device__ __forceinline__ void cell_write32_body(const Grid& G, int n_cells, co
     __shared__ RegroupCells<S::CB> s;
     __shared__ float4 s_a[SUMS ? CH : 1];
     __shared__ float2 s_b[SUMS && DIM == 3 ? CH : 1];
-    if (state_dead(w.counters)) return;
     const int tid = threadIdx.x, g = tid / S::LPC, gl = tid % S::LPC;
     ShapeOne32<DIM, DEG> sh[S::NA];
     int comp[S::NA];
@@ -765,7 +764,7 @@ __device__ __forceinline__ void cell_write32_body(const Grid& G, int n_cells, co
             sh[u].init(kk);
         }
     for (int cb = G.bid * S::CB; cb < n_cells; cb += G.nblk * S::CB) {
-        regroup_cells<S::CB>(s, cb, n_cells, old_off, cap, pp, w, omap);
+        if (!regroup_cells<S::CB>(s, cb, n_cells, old_off, cap, pp, w, omap)) return;
         const long long base = s.base;
         const int total = base + s.off[S::CB] <= cap ? s.off[S::CB] : (int)(cap > base ? cap - base : 0);
         float sum[S::NA], cmp[S::NA];

@@ -1,0 +1,127 @@
+"""A regroup that needs more particles than the capacity on meshes of many
+write workgroups (RegroupShape::CB = 16 cells, 32 degree-1 hexahedra): the
+range is cut in the middle of a workgroup, the workgroups behind it start past
+the capacity, and some start after the flag is raised.  Every wavefront of a
+workgroup has to take the same decision on that flag.  The capacity error is
+reported, and the particles and fields of another handle, of another member of
+the same batch, stay those of a run without the overflow."""
+import numpy as np
+import pytest
+
+from parity_util import bitwise_equal
+from pfem2_amd import FP32_MIXED, FP64, Batch, ParticleStage, Pf2Error
+from pfem2_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+
+def _one_cell(m, q, n=64):
+    """n particles in cell 0: the reseed fills all other cells."""
+    rng = np.random.default_rng(41)
+    return np.zeros(n, dtype=np.int32), rng.uniform(0.05, 0.95, size=(n, m.dim))
+
+
+def _every_third(m, q):
+    """Every third cell crowded past its slot row, the others empty."""
+    cell, xi = M.jittered_lattice(m, q, 0.0, 1)
+    keep = cell % 3 == 0
+    return np.repeat(cell[keep], 4), np.repeat(xi[keep], 4, axis=0)
+
+
+CASES = {   # mesh, lattice, MAX, inserted particles, capacity as a share of the lattice points
+    "800 quads": (lambda: M.quad_2d(40, 20, (0.0, 0.0), (2.0, 1.0), jitter=0.1, seed=3), [2, 2], 3, _one_cell, 0.53),
+    "34,000 quads": (lambda: M.quad_2d(200, 170, (0.0, 0.0), (2.0, 1.7)), [2, 2], 3, _one_cell, 0.53),
+    "99 quads past the slots": (lambda: M.quad_2d(11, 9, (0.0, 0.0), (1.1, 0.9)), [8, 8], 3, _every_third, 1.34),
+    "800 quads q2": (lambda: M.q2(M.quad_2d(40, 20, (0.0, 0.0), (2.0, 1.0))), [2, 2], 3, _one_cell, 0.47),
+    "768 hexes": (lambda: M.box_3d(12, 8, 8, (0.0, 0.0, 0.0), (1.2, 0.8, 0.8), jitter=0.1, seed=3), [2, 2, 2], 3,
+                  _one_cell, 0.53),
+    "768 hexes q2": (lambda: M.q2(M.box_3d(12, 8, 8, (0.0, 0.0, 0.0), (1.2, 0.8, 0.8))), [2, 2, 2], 3, _one_cell, 0.47),
+}
+
+
+def _overflowing(case, precision):
+    """A handle whose first step overflows, and its field."""
+    mesh, q, mx, insert, share = CASES[case]
+    m = mesh()
+    points = m.n_cells * int(np.prod(q))
+    cap = int(share * points)
+    cell, xi = insert(m, q)
+    # what the census leaves: up to MAX of each occupied part, one in every other
+    part = cell.astype(np.int64) * np.prod(q) + np.minimum((xi * q).astype(int), np.array(q) - 1) @ \
+        np.cumprod([1] + list(q))[:m.dim]
+    n = np.bincount(part, minlength=points)
+    assert len(cell) <= cap < np.minimum(np.maximum(n, 1), mx).sum()
+    V = M.uniform_field(m, [0.0] * m.dim)
+    g = ParticleStage(m, 0.01, 2, mx, q, precision, capacity=cap)
+    g.upload_fields(V, V)
+    g.insert_particles(cell, xi)
+    return g, V
+
+
+def _bystander(dim, precision, seed):
+    m = M.quad_2d(30, 12, (0.0, 0.0), (1.5, 0.6), jitter=0.1, seed=seed) if dim == 2 else \
+        M.box_3d(8, 6, 6, (0.0, 0.0, 0.0), (0.8, 0.6, 0.6), jitter=0.1, seed=seed)
+    V = M.uniform_field(m, [0.4, 0.2, 0.1][:dim])
+    s = ParticleStage(m, 0.02, 4, 2, [3, 3, 2][:dim], precision)
+    s.upload_fields(V, V)
+    s.seed_particles()
+    return s, V
+
+
+def _assert_same(a, b):
+    pa, pb = a.particles(), b.particles()
+    for key in ("cell", "id", "x", "xi", "v"):
+        assert np.array_equal(pa[key], pb[key]), key
+    assert bitwise_equal(a.download_field(), b.download_field())
+    assert a.stats() == b.stats()
+
+
+@pytest.mark.parametrize("separate", [False, True])
+@pytest.mark.parametrize("precision", [FP64, FP32_MIXED])
+@pytest.mark.parametrize("case", list(CASES))
+def test_overflow_over_many_workgroups(case, precision, separate):
+    dim = 3 if "hex" in case else 2
+    a, _ = _bystander(dim, precision, 5)
+    b, _ = _bystander(dim, precision, 5)
+    g, _ = _overflowing(case, precision)
+    a.step()
+    for _ in range(3):   # the later ones start in a dead state
+        if separate:
+            g.correct_particles_velocities()
+            g.move_particles()
+            g.distribute_particle_velocities_to_grid(download=False)
+        else:
+            g.step()
+    a.step()
+    for call in (g.n_global_particles, g.cell_counts, g.particles, lambda: g.step(download=True)):
+        with pytest.raises(Pf2Error, match="capacity"):
+            call()
+    g.close()
+    b.step()
+    b.step()
+    _assert_same(a, b)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("precision", [FP64, FP32_MIXED])
+@pytest.mark.parametrize("case", ["800 quads", "34,000 quads", "768 hexes"])
+def test_overflow_of_a_batch_member(case, precision):
+    import torch
+    dim = 3 if "hex" in case else 2
+    solo, bat = ([_bystander(dim, precision, 5 + k) for k in range(2)] for _ in range(2))
+    g, Vg = _overflowing(case, precision)
+    members = [bat[0][0], g, bat[1][0]]
+    fields = [torch.from_numpy(np.ascontiguousarray(V)).to("cuda") for V in (bat[0][1], Vg, bat[1][1])]
+    torch.cuda.synchronize()
+    b = Batch(3)
+    for _ in range(3):
+        b.step(members, [f.data_ptr() for f in fields])
+        for (s, _), f in zip(solo, (fields[0], fields[2])):
+            s.step_with_field(f.data_ptr())
+    with pytest.raises(Pf2Error, match="capacity"):
+        g.n_global_particles()
+    for (s, _), (t, _) in zip(solo, bat):
+        _assert_same(s, t)
+    b.close()
+    g.close()
