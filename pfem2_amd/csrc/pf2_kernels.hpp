@@ -227,6 +227,16 @@ struct DevWork {
 constexpr int DEAD_FLAGS = 3;
 __device__ __forceinline__ bool state_dead(const int* counters) { return (counters[2] & DEAD_FLAGS) != 0; }
 
+// The same for the workgroups of a kernel that raises a flag itself and shares
+// LDS between wavefronts: one thread reads it for all (all threads call), so
+// that no wavefront leaves the others to LDS that it was to fill.
+__device__ __forceinline__ bool workgroup_dead(const int* counters) {
+    __shared__ int s_dead;
+    if (threadIdx.x == 0) s_dead = state_dead(counters);
+    __syncthreads();
+    return s_dead != 0;
+}
+
 // vertex coordinates and nodal velocities of cell c, from the packed per-cell
 // copies, or (GATHER: FP32-mixed handles, which keep no FP64 velocity copy)
 // with the velocities gathered from V through the cell's DoF map (the same
@@ -1343,7 +1353,8 @@ __device__ __forceinline__ void cell_count_body(CountRows<CAP>& rows, const Grid
     auto &s_sid = rows.sid;
     auto &s_cnt = rows.cnt;
     auto &s_mask = rows.mask;
-    if (state_dead(w.counters)) return;
+    // (LIST: cell_big_body has decided for the workgroup)
+    if (!LIST && state_dead(w.counters)) return;
     const int g = threadIdx.x / GS, gl = threadIdx.x % GS;
     const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
     int nk = 1;
@@ -1590,10 +1601,10 @@ __device__ __forceinline__ void cell_big_body(const Grid& G, const int* __restri
     auto &s_sid = lds.row.sid;
     __shared__ unsigned long long s_hit;
     __shared__ int s_nvalid, s_nsurv;
-    if (state_dead(w.counters)) return;
+    const int nbig = w.big[0], set = w.counters[8];   // (read along with the flag)
+    if (workgroup_dead(w.counters)) return;           // (raised below by other workgroups)
     const int tid = threadIdx.x;
     const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
-    const int nbig = w.big[0], set = w.counters[8];
     add_fine_sums(w, set, (int)G.bid, (int)G.nblk);
     if (nbig == 0) return;
     const bool by_group = nbig > (int)G.nblk;

@@ -1,10 +1,11 @@
 """A regroup that needs more particles than the capacity on meshes of many
 write workgroups (RegroupShape::CB = 16 cells, 32 degree-1 hexahedra): the
 range is cut in the middle of a workgroup, the workgroups behind it start past
-the capacity, and some start after the flag is raised.  Every wavefront of a
-workgroup has to take the same decision on that flag.  The capacity error is
-reported, and the particles and fields of another handle, of another member of
-the same batch, stay those of a run without the overflow."""
+the capacity, and some start after the flag is raised.  Likewise cells past the
+census limit among many that k_cell_big counts.  Every wavefront of a
+workgroup has to take the same decision on the flag that its launch raises.  The
+capacity error is reported, and the particles and fields of another handle, of
+another member of the same batch, stay those of a run without the overflow."""
 import numpy as np
 import pytest
 
@@ -125,3 +126,45 @@ def test_overflow_of_a_batch_member(case, precision):
         _assert_same(s, t)
     b.close()
     g.close()
+
+
+def _crowded(shape, precision):
+    """Cells of more than 2048 particles among cells that the census lists for
+    k_cell_big: fewer of them than its workgroups, or more."""
+    nx, ny = {"few": (33, 3), "many": (300, 8)}[shape]
+    m = M.quad_2d(nx, ny, (0.0, 0.0), (0.1 * nx, 0.1 * ny), jitter=0.1, seed=8)
+    rng = np.random.default_rng(43)
+    per = np.array([66, 100, 130, 300, 128, 20])[np.arange(m.n_cells) % 6]
+    per[[5, m.n_cells // 2, m.n_cells - 3]] = 2100
+    cell = np.repeat(np.arange(m.n_cells, dtype=np.int32), per)
+    V = M.uniform_field(m, [0.6, 0.1])
+    g = ParticleStage(m, 0.05, 3, 20, [4, 4], precision, capacity=2 * len(cell))
+    g.upload_fields(V, V)
+    g.insert_particles(cell, rng.uniform(0.02, 0.98, size=(len(cell), 2)))
+    return g, V
+
+
+@pytest.mark.parametrize("batch", [False, True])
+@pytest.mark.parametrize("precision", [FP64, FP32_MIXED])
+@pytest.mark.parametrize("shape", ["few", "many"])
+def test_crowded_cells_among_listed_ones(shape, precision, batch):
+    import torch
+    a, V = _bystander(2, precision, 5)
+    b, _ = _bystander(2, precision, 5)
+    g, Vg = _crowded(shape, precision)
+    fields = [torch.from_numpy(np.ascontiguousarray(f)).to("cuda") for f in (Vg, V)]
+    torch.cuda.synchronize()
+    bt = Batch(2)
+    for _ in range(3):
+        if batch:
+            bt.step([g, a], [f.data_ptr() for f in fields])
+        else:
+            g.step_with_field(fields[0].data_ptr())
+            a.step_with_field(fields[1].data_ptr())
+        b.step_with_field(fields[1].data_ptr())
+    with pytest.raises(Pf2Error, match="2048"):
+        g.n_global_particles()
+    _assert_same(a, b)
+    bt.close()
+    for s in (a, b, g):
+        s.close()
