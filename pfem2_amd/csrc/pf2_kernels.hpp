@@ -2127,9 +2127,9 @@ __global__ void __launch_bounds__(256) k_cell_pend(DevMesh<DIM> m, const int* __
                                                    DevParams pp, DevWork w) {
     constexpr int NV = Q1<DIM>::NV;
     constexpr int ND = QF<DIM, DEG>::ND;
-    if (state_dead(w.counters)) return;
     const int nc = m.n_cells;
     const int seg_end = old_off[nc];
+    if (workgroup_dead(w.counters)) return;   // (pend_slots raises the flag)
     pend_slots(w, nc, seg_end, A.cap);
     // one cell per thread: new particles are few, and most cells only get
     // their resets

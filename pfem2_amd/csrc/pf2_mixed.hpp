@@ -1234,9 +1234,9 @@ __global__ void __launch_bounds__(256) k_cell_pend32(int n_cells, const int* __r
                                                      const float* __restrict__ V32, long long cap, DevParams pp,
                                                      DevWork w) {
     constexpr int ND = QF<DIM, DEG>::ND;
-    if (state_dead(w.counters)) return;
     const int nc = n_cells;
     const int seg_end = old_off[nc];
+    if (workgroup_dead(w.counters)) return;   // (pend_slots raises the flag)
     pend_slots(w, nc, seg_end, cap);
     // one cell per thread, as in k_cell_pend
     for (int c0 = blockIdx.x * 256; c0 < nc; c0 += gridDim.x * 256) {

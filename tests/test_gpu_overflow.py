@@ -168,3 +168,39 @@ def test_crowded_cells_among_listed_ones(shape, precision, batch):
     bt.close()
     for s in (a, b, g):
         s.close()
+
+
+@pytest.mark.parametrize("precision", [FP64, FP32_MIXED])
+@pytest.mark.parametrize("case", ["800 quads", "34,000 quads", "768 hexes"])
+def test_overflow_of_a_pending_layout(case, precision):
+    """The new particles of a mesh move exceed the capacity: the host's estimate
+    (the 64 inserted) leaves room for a full reseed, but the step before has
+    reseeded the whole mesh, and the stretched mesh needs more at its rim."""
+    mesh, q, mx, insert, _ = CASES[case]
+    m = mesh()
+    cell, xi = insert(m, q)
+    V = M.uniform_field(m, [0.02, 0.01, 0.01][:m.dim])
+    mid = 0.5 * (m.vertices.min(axis=0) + m.vertices.max(axis=0))
+    X = mid + (m.vertices - mid) * (1.0 + 0.6 / max(round(m.n_cells ** (1.0 / m.dim)), 12))
+    cap = len(cell) + m.n_cells * int(np.prod(q))
+    a, _ = _bystander(m.dim, precision, 5)
+    b, _ = _bystander(m.dim, precision, 5)
+    full, g = (ParticleStage(m, 0.01, 2, mx, q, precision, keep_velocity_ext=True, capacity=c) for c in (4 * cap, cap))
+    for s in (full, g):
+        s.upload_fields(V, V)
+        s.insert_particles(cell, xi)
+        s.set_profiling()
+        s.step()
+        s.move_mesh(X)
+        assert s.kernel_times()["k_cell_pend"][1] == 1
+    assert full.n_global_particles() > cap
+    a.step()
+    g.step()
+    g.move_mesh(m.vertices)
+    g.step()
+    with pytest.raises(Pf2Error, match="capacity"):
+        g.n_global_particles()
+    b.step()
+    _assert_same(a, b)
+    for s in (a, b, full, g):
+        s.close()
