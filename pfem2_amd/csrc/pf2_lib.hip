@@ -837,8 +837,11 @@ int download_field(pf2_handle_s* h, double* V) {
         else
             hipLaunchKernelGGL(HIP_KERNEL_NAME(k_field_out<3>), g, dim3(256), 0, h->stream, h->dV, (double*)st.p, n,
                                h->counters, f);
-        HIPC(hipGetLastError());
+        // (the error may be an earlier call's: the kernel uses the block until
+        // the stream has run, whatever is returned)
+        const hipError_t launched = hipGetLastError();
         HIPC(hipStreamSynchronize(h->stream));
+        HIPC(launched);
         std::memcpy(V, st.p, bytes);
         return flag_error(*f);
     }
@@ -873,9 +876,11 @@ int upload_field(pf2_handle_s* h, const double* src, double* dst, hipMemcpyKind 
     else
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_to_node_major<3>), dim3(grid_for(n, 256)), dim3(256), 0, h->stream, from,
                            dst, n);
-    HIPC(hipGetLastError());
-    // the host source buffer may be reused by the caller after return
+    const hipError_t launched = hipGetLastError();
+    // the host source buffer may be reused by the caller after return, the
+    // block by another call
     if (kind == hipMemcpyHostToDevice) HIPC(hipStreamSynchronize(h->stream));
+    HIPC(launched);
     return 0;
 }
 
