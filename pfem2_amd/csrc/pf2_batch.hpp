@@ -83,7 +83,7 @@ template <int DIM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 5 : 2))) kb_move(BatchView<DIM> bv) {
     Grid G;
     const BatchSim<DIM>& S = bv.at(BK_MOVE, G);
-    move_body<DIM>(G, S.m, S.V, S.Vold, S.A, S.pp, S.w, S.qu, 1, 1);
+    move_body<DIM>(G, S.m, S.A, S.pp, S.w, S.qu, 1, 1);
 }
 
 template <int DIM>
@@ -97,7 +97,7 @@ template <int DIM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 3 : 2))) kb_search(BatchView<DIM> bv) {
     Grid G;
     const BatchSim<DIM>& S = bv.at(BK_SEARCH, G);
-    search_body<DIM>(G, S.m, S.V, S.A, S.pp, S.w, S.qu, 0);
+    search_body<DIM>(G, S.m, S.A, S.pp, S.w, S.qu, 0);
 }
 
 template <int DIM>

@@ -391,7 +391,7 @@ __device__ __forceinline__ int closed_form(const double (*P)[2], const QuadCell&
     out[0] = xi;
     out[1] = eta;
     if (!ok) return 2;
-    return (xi >= 0.0) & (xi <= 1.0) & (eta >= 0.0) & (eta <= 1.0) ? 0 : 1;
+    return ((xi >= 0.0) & (xi <= 1.0) & (eta >= 0.0) & (eta <= 1.0)) ? 0 : 1;
 }
 
 // least-squares affine fit of a cell, inverted: A[:, j] = sum_k P_k

@@ -58,25 +58,6 @@ __device__ __forceinline__ void stat_add(unsigned long long* stats, int k, unsig
     atomicAdd(&stats[wave_shard() * NSTAT + k], v);
 }
 
-// atomicAdd(&cnt[key], 1) for the lanes with pred set, one atomic per distinct
-// key in the wavefront; returns the previous value for this lane (all lanes call)
-__device__ __forceinline__ int wave_inc_by_key(int* cnt, bool pred, int key) {
-    int result = 0;
-    unsigned long long todo = __ballot(pred);
-    const int lane = threadIdx.x & (WAVE - 1);
-    while (todo) {
-        const int leader = __ffsll((long long)todo) - 1;
-        const int k = __shfl(key, leader);
-        const unsigned long long same = __ballot(pred && key == k) & todo;
-        int base = 0;
-        if (lane == leader) base = atomicAdd(&cnt[k], __popcll(same));
-        base = __shfl(base, leader);
-        if ((same >> lane) & 1) result = base + __popcll(same & ((1ull << lane) - 1));
-        todo &= ~same;
-    }
-    return result;
-}
-
 // flush per-lane statistics with one sharded atomic per wavefront (all lanes must call)
 __device__ __forceinline__ void wave_stat(unsigned long long* stats, int k, int v) {
     const int t = wave_sum(v);
@@ -588,10 +569,8 @@ __device__ __forceinline__ bool inside_margin(const double* r) {
     return in;
 }
 
-// inverse_map and the unit-cell test of a candidate cell.  CLOSED (2-D): the
-// closed form first, the clearly-outside test only where it does not decide
-// (both orders give the same answer).
-template <int DIM, bool CLOSED>
+// inverse_map and the unit-cell test of a candidate cell
+template <int DIM>
 __device__ __forceinline__ bool contains(const DevMesh<DIM>& m, int c, const double (*Q)[DIM], const double* x,
                                          double* r) {
     if constexpr (DIM == 3) {
@@ -599,12 +578,6 @@ __device__ __forceinline__ bool contains(const DevMesh<DIM>& m, int c, const dou
         H.load(m.ftol + (size_t)c * HEX_N);
         return hex_map(Q, H, x, r) && inside_unit<DIM>(r);
     } else {
-        if constexpr (CLOSED) {
-            QuadCell qc;
-            qc.init(Q);
-            const int st = closed_form(Q, qc, x, r);
-            if (st != 2) return st == 0;
-        }
         return inverse_map<DIM>(Q, x, r, m.ftol[c], true) && inside_unit<DIM>(r);
     }
 }
@@ -738,7 +711,7 @@ __device__ __forceinline__ int relocate(const DevMesh<DIM>& m, int c, const doub
         }
         double r[DIM];
         load_vertices<DIM>(m, cc, Q);
-        if (contains<DIM, !SHORTCUT>(m, cc, Q, x, r)) {
+        if (contains<DIM>(m, cc, Q, x, r)) {
 #pragma unroll
             for (int d = 0; d < DIM; ++d) xi_out[d] = r[d];
             return cc;
@@ -1029,9 +1002,8 @@ __device__ __forceinline__ void park_particle(const DevParticles& A, const DevWo
 // k_move: [correction] + substeps until done or the first failed own-cell test.
 //   correct_particles_velocities  TurekBenchmark/pfem2particle.cpp:792-811
 template <int DIM, int DEG = 1>
-__device__ __forceinline__ void move_body(const Grid& G, const DevMesh<DIM>& m, const double* __restrict__ V,
-                                          const double* __restrict__ Vold, const DevParticles& A, const DevParams& pp,
-                                          const DevWork& w, const DevQueues& qu, int do_correct, int do_move) {
+__device__ __forceinline__ void move_body(const Grid& G, const DevMesh<DIM>& m, const DevParticles& A,
+                                          const DevParams& pp, const DevWork& w, const DevQueues& qu, int do_correct, int do_move) {
     constexpr int NV = Q1<DIM>::NV;
     constexpr int ND = QF<DIM, DEG>::ND;
     // a pending layout (k_cell_pend): its slots, the current cell of a kept
@@ -1090,10 +1062,9 @@ __device__ __forceinline__ void move_body(const Grid& G, const DevMesh<DIM>& m, 
 }
 
 template <int DIM, int DEG = 1>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? (DEG == 1 ? 5 : 3) : 2))) k_move(DevMesh<DIM> m, const double* __restrict__ V,
-                                              const double* __restrict__ Vold, DevParticles A, DevParams pp,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? (DEG == 1 ? 5 : 3) : 2))) k_move(DevMesh<DIM> m, DevParticles A, DevParams pp,
                                               DevWork w, DevQueues qu, int do_correct, int do_move) {
-    move_body<DIM, DEG>(hw_grid(), m, V, Vold, A, pp, w, qu, do_correct, do_move);
+    move_body<DIM, DEG>(hw_grid(), m, A, pp, w, qu, do_correct, do_move);
 }
 
 // Queue entries for the lanes of a search wavefront that hold no particle.
@@ -1147,9 +1118,9 @@ struct Refill {
 // consumes a substep, so each lane ends, and a wavefront leaves when its
 // segment is drained and none of its lanes holds a particle.
 template <int DIM, int DEG = 1, bool RESORT = false>
-__device__ __forceinline__ void search_body(const Grid& G, const DevMesh<DIM>& m, const double* __restrict__ V,
-                                            const DevParticles& A, const DevParams& pp, const DevWork& w,
-                                            const DevQueues& qu, int round) {
+__device__ __forceinline__ void search_body(const Grid& G, const DevMesh<DIM>& m, const DevParticles& A,
+                                            const DevParams& pp, const DevWork& w, const DevQueues& qu,
+                                            int round) {
     constexpr int NV = Q1<DIM>::NV;
     __shared__ int s_pref[QSHARDS + 2];
     const int n = queue_prefix(qu, round, s_pref, G);
@@ -1224,16 +1195,15 @@ __device__ __forceinline__ void search_body(const Grid& G, const DevMesh<DIM>& m
 }
 
 template <int DIM, int DEG = 1>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 3 : 2))) k_search_resume(DevMesh<DIM> m, const double* __restrict__ V,
-                                                       DevParticles A, DevParams pp, DevWork w, DevQueues qu,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 3 : 2))) k_search_resume(DevMesh<DIM> m, DevParticles A, DevParams pp, DevWork w, DevQueues qu,
                                                        int round) {
-    search_body<DIM, DEG>(hw_grid(), m, V, A, pp, w, qu, round);
+    search_body<DIM, DEG>(hw_grid(), m, A, pp, w, qu, round);
 }
 
 // the relocations of the re-sort after a mesh move (queue RESORT_QUEUE)
 template <int DIM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM == 2 ? 3 : 2))) k_resort_search(DevMesh<DIM> m, DevParticles A, DevParams pp, DevWork w, DevQueues qu) {
-    search_body<DIM, 1, true>(hw_grid(), m, nullptr, A, pp, w, qu, RESORT_QUEUE);
+    search_body<DIM, 1, true>(hw_grid(), m, A, pp, w, qu, RESORT_QUEUE);
 }
 
 // candidate j of cell c: stayers of the old segment first, then the
@@ -2541,7 +2511,7 @@ __global__ void __launch_bounds__(256) k_resort(DevMesh<DIM> m, DevParticles A, 
                     qc.init(P);
                     st = closed_form(P, qc, x, r);
                 } else {
-                    st = contains<DIM, false>(m, c, P, x, r) ? 0 : 1;
+                    st = contains<DIM>(m, c, P, x, r) ? 0 : 1;
                 }
                 if (st == 0) {
 #pragma unroll
@@ -2640,11 +2610,6 @@ __global__ void k_pack_fields(DevMesh<DIM> m, const double* __restrict__ V, cons
             if (cellDV) cellDV[(size_t)t * DIM + d] = a - b;
         }
     }
-}
-
-__global__ void k_fill_int(int* p, int val, long long n) {
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        p[i] = val;
 }
 
 // nodal field layout conversion: component-major <-> node-major

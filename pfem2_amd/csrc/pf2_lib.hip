@@ -703,21 +703,19 @@ int run_move(pf2_handle_s* h, int do_correct, int do_move, bool fuse_sums = fals
             Timed t(h, K_MOVE);
             if (h->deg == 2)
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_move<DIM, 2>), dim3(grid), dim3(256), 0, h->stream,
-                                   dev_mesh<DIM>(h), h->dV, h->dVold, dev_particles(h, h->cur), pp, w, qu, do_correct,
-                                   do_move);
+                                   dev_mesh<DIM>(h), dev_particles(h, h->cur), pp, w, qu, do_correct, do_move);
             else
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_move<DIM>), dim3(grid), dim3(256), 0, h->stream,
-                                   dev_mesh<DIM>(h), h->dV, h->dVold, dev_particles(h, h->cur), pp, w, qu, do_correct,
-                                   do_move);
+                                   dev_mesh<DIM>(h), dev_particles(h, h->cur), pp, w, qu, do_correct, do_move);
         }
         if (do_move) {
             Timed t(h, K_SEARCH);
             if (h->deg == 2)
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume<DIM, 2>), dim3(qgrid), dim3(256), 0, h->stream,
-                                   dev_mesh<DIM>(h), h->dV, dev_particles(h, h->cur), pp, w, qu, 0);
+                                   dev_mesh<DIM>(h), dev_particles(h, h->cur), pp, w, qu, 0);
             else
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_search_resume<DIM>), dim3(qgrid), dim3(256), 0, h->stream,
-                                   dev_mesh<DIM>(h), h->dV, dev_particles(h, h->cur), pp, w, qu, 0);
+                                   dev_mesh<DIM>(h), dev_particles(h, h->cur), pp, w, qu, 0);
         }
     }
     HIPC(hipGetLastError());

@@ -92,12 +92,6 @@ __device__ __forceinline__ void rec_store_v(const Rec32& r, long long i, const f
     }
 }
 
-template <int DIM>
-__device__ __forceinline__ void rec_copy(const Rec32& src, long long i, const Rec32& dst, long long o) {
-    dst.a[o] = src.a[i];
-    if constexpr (DIM == 3) dst.b[o] = src.b[i];
-}
-
 // multilinear coefficients of F_K relative to vertex 0, in FP32
 //   2-D: F = x0 + a xi0 + b xi1 + c xi0 xi1
 //   3-D: F = x0 + a xi0 + b xi1 + c xi2 + d xi0 xi1 + e xi0 xi2 + f xi1 xi2 + g xi0 xi1 xi2
@@ -177,27 +171,6 @@ __device__ __forceinline__ void shape32(const float* xi, float* N) {
         for (int d = 0; d < DIM; ++d) val *= ((k >> d) & 1) ? xi[d] : (1.0f - xi[d]);
         N[k] = val;
     }
-}
-
-// N_k alone, for a lane with a fixed vertex k: factor d is t_d xi_d + s_d
-// (xi_d, or 1 - xi_d with one rounding), multiplied in shape32's order, so
-// the value is shape32's N[k]
-template <int DIM>
-__device__ __forceinline__ void shape_one32_coeffs(int k, float* t, float* s) {
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-        const bool one = (k >> d) & 1;
-        t[d] = one ? 1.0f : -1.0f;
-        s[d] = one ? 0.0f : 1.0f;
-    }
-}
-
-template <int DIM>
-__device__ __forceinline__ float shape_one32(const float* t, const float* s, const float* xi) {
-    float val = __fmaf_rn(t[0], xi[0], s[0]);
-#pragma unroll
-    for (int d = 1; d < DIM; ++d) val *= __fmaf_rn(t[d], xi[d], s[d]);
-    return val;
 }
 
 // The local difference of F_K splits into the Jacobian J(xi) at the current
@@ -438,9 +411,10 @@ struct Field32 {
 };
 
 // N_k of one node k of a degree-DEG cell in FP32 (a lane's node in the
-// projection sums): DEG 1 as shape_one32; DEG 2 the product over the
-// directions of the 1-D Lagrange factor (c0 t + c1)(c2 t + c3) of the node's
-// axis index (lag2_coeffs)
+// projection sums), a product over the directions.  DEG 1: the factor c0 t + c1
+// (t, or 1 - t with one rounding) in shape32's order, so the value is shape32's
+// N[k]; DEG 2: the 1-D Lagrange factor (c0 t + c1)(c2 t + c3) of the node's axis
+// index (lag2_coeffs)
 template <int DIM, int DEG>
 struct ShapeOne32 {
     float c[DIM][4];
@@ -1151,7 +1125,7 @@ __global__ void __launch_bounds__(256) k_resort32(DevMesh<DIM> m, const int* __r
                     qc.init(P);
                     st = closed_form(P, qc, x, r);
                 } else {
-                    st = contains<DIM, false>(m, c, P, x, r) ? 0 : 1;
+                    st = contains<DIM>(m, c, P, x, r) ? 0 : 1;
                 }
                 if (st == 0) {
 #pragma unroll
