@@ -1763,8 +1763,7 @@ __device__ __forceinline__ bool regroup_cells(RegroupCells<CB>& s, int cb, int n
     const int last = nc - cb < CB ? nc - cb : CB;
     bool past = false;
     if (t < WAVE) {
-        const bool dead = (__builtin_amdgcn_readfirstlane(load_agent(&w.counters[2])) & DEAD_FLAGS) != 0;
-        const int set = w.counters[8];
+        const int flags = w.counters[2], set = w.counters[8];
         const int c = cb + (t < last ? t : last - 1);
         const unsigned long long n = w.fs_cnt[c], v = t < last ? n : 0ull;
         const int nsurv = w.nsurv[c];
@@ -1781,6 +1780,7 @@ __device__ __forceinline__ bool regroup_cells(RegroupCells<CB>& s, int cb, int n
             incl = w.fs_off[c] - base + n;
         }
         const unsigned long long all = pp.nparts_in >= 64 ? ~0ull : ((1ull << pp.nparts_in) - 1);
+        const bool dead = (__builtin_amdgcn_readfirstlane(flags) & DEAD_FLAGS) != 0;
         if (t == 0) {
             s.base = (long long)(base >> 32);
             s.dead = dead;
