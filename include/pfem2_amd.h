@@ -92,7 +92,10 @@ int pf2_create(const pf2_mesh* mesh, const pf2_params* params, long long capacit
 int pf2_create_in(const pf2_mesh* mesh, const pf2_params* params, long long capacity, void* block,
                   unsigned long long block_bytes, void* stream, pf2_handle* out);
 /* Device bytes pf2_create takes for this mesh / params / capacity (upper
- * bound), and the bytes a handle holds. */
+ * bound), and the bytes a handle holds: those of its creation and the scratch
+ * that pf2_reinterpolate_fields and pf2_calculate_loads keep until
+ * pf2_destroy (the size of a few nodal fields; the estimate leaves it out, and
+ * a handle in a caller's block takes it outside of that). */
 int pf2_estimate_bytes(const pf2_mesh* mesh, const pf2_params* params, long long capacity,
                        unsigned long long* bytes);
 int pf2_memory_bytes(pf2_handle h, unsigned long long* bytes);

@@ -1835,7 +1835,7 @@ int pf2_set_graphs(pf2_handle h, int on) {
 
 int pf2_memory_bytes(pf2_handle h, unsigned long long* bytes) {
     if (!h || !bytes) return fail(PF2_E_ARG, "handle/bytes is NULL");
-    *bytes = h->bytes;
+    *bytes = h->bytes + h->scratch_len * sizeof(double);
     return 0;
 }
 

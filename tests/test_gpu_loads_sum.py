@@ -27,3 +27,20 @@ def test_face_counts():
         assert bitwise_equal(a, _oracle_loads(o, V, P, faces, *args)), n
         g.reinterpolate_fields(np.zeros((m.n_vertices, 2)), P)   # another user of the scratch in between
     g.close()
+
+
+def test_kept_scratch_is_counted():
+    """memory_bytes includes the scratch that the nodal routines keep: the
+    displacements, the new velocities, and each extra field twice; a smaller
+    call afterwards takes no more."""
+    m = M.cylinder_channel(0.2, seed=67)
+    g = ParticleStage(m, 0.01, 2, 3, [2, 2], FP64)
+    g.upload_fields(np.zeros((2, m.n_dofs)), np.zeros((2, m.n_dofs)))
+    own = g.memory_bytes()
+    P = np.zeros(m.n_dofs)
+    g.reinterpolate_fields(np.zeros((m.n_vertices, 2)), P)
+    kept = 8 * (2 * m.n_vertices + 2 * m.n_dofs + 2 * m.n_dofs)
+    assert g.memory_bytes() == own + kept
+    g.reinterpolate_fields(np.zeros((m.n_vertices, 2)))
+    assert g.memory_bytes() == own + kept
+    g.close()
