@@ -342,9 +342,9 @@ struct QuadCell {
 // its answer.  Straight-line but for the choice of the root's quotient: a
 // value out of range or NaN fails a comparison at the end.  About 105 instead
 // of 150 instructions per point (one reciprocal per cell for the two roots,
-// no scaling steps): k_move, bound by them, 134 -> 118 us per step on 101,785
-// cells with 2.4M particles, 759 -> 670 us on 407,140 with 11M; early exits
-// instead of the straight line took most of that back (707 us).
+// no scaling steps): k_move, bound by them, 153 -> 136 us on 101,785 quads,
+// 808 -> 721 on 407,140; early exits instead of the straight line took 40% of
+// the gain back.
 __device__ __forceinline__ int closed_form(const double (*P)[2], const QuadCell& q, const double* p, double* out) {
     const double x = p[0], y = p[1];
     const double x0 = P[0][0], x1 = P[1][0], x2 = P[2][0], x3 = P[3][0];
@@ -578,8 +578,8 @@ PF2_HD bool inverse_map(const double (*P)[DIM], const double* p, double* out, do
 // inverse_map's bits; computed in the particle kernels they took about 350
 // instructions per containment test, or the registers to keep them.  With the
 // norms compared by their squares, and degree-2 fields read per substep:
-// 505 -> 332 us (k_move) and 260 -> 165 us (search) per step on 68,992
-// degree-2 hexahedra, 309 -> 287 and 393 -> 336 on 50,000 of degree 1.
+// 546 -> 358 us (k_move) and 290 -> 197 (search) on 68,992 degree-2 hexahedra,
+// 293 -> 282 and 259 -> 225 on 202,240 of degree 1 (FP64).
 constexpr int HEX_N = 20;   // doubles per cell (19 used)
 
 struct HexCell {

@@ -27,6 +27,11 @@
 // No floating-point atomics anywhere.  Integer atomics only build lists whose
 // order is erased again by the id ordering; counters that many wavefronts
 // update are sharded over separate cache lines.
+//
+// Times in these sources are kernel times of one MI355X per step or launch on
+// the timed workloads (perf/cases.py: 101,785 quads with 2.4M particles,
+// 407,140 with 11M on a moving mesh, 202,240 hexahedra, 68,992 of degree 2),
+// unless they say otherwise.
 #pragma once
 
 #include "pf2_geom.hpp"
@@ -157,8 +162,15 @@ struct DevParams {
 //            counts itself (which fine leaves out).  Two sets: a census adds to
 //            one and the write after it clears the other for the next
 //            (counters[8] says which).
-// Two launches less are 3% of a step on 2,000 cells; from about 100,000 on the
-// sums cost more than the scan (per step on 407,140: census +14 us, write +17).
+// Two launches less are 3% of a step on 2,000 cells.  Whole steps of a fixed
+// cylinder mesh with sums and with the scan, FP64 and FP32-mixed: 182 and 185,
+// 176 and 179 us on 25,446 cells; 236 and 240, 203 and 208 on 40,000; 318 and
+// 322, 238 and 242 on 60,000; 409 and 413, 287 and 289 on 80,000; the same on
+// 101,785; 918 and 908, 599 and 593 on 200,000.  So they cross near 100,000
+// cells, past which a workgroup's loads of the tiles before its own cost more
+// than the launches (on 407,140 the census takes 14 us more and the write 17).
+// The line lies below that, where a wavefront reads all tiles with two loads a
+// lane; it gives away 1-2% of a step from there to 80,000 cells.
 // Tiles added by the census itself, an atomic per wavefront, cost it 40 us on
 // 101,785 cells: atomics on neighbouring sums serialise.
 constexpr int TILE = 256;
@@ -350,8 +362,7 @@ __device__ __forceinline__ void interp(const double (*Fc)[DIM], const double* xi
 
 // the same with one node at a time (at(k): the velocity of node k), for a rare
 // point: the nodes of a degree-2 cell held at once take the registers of a
-// whole kernel (k_cell_write on degree-2 hexahedra: 408 -> 248,
-// 151 -> 130 us per step on 68,992)
+// whole kernel (k_cell_write on degree-2 hexahedra: 408 -> 248)
 template <int DIM, int DEG, class F>
 __device__ __forceinline__ void interp_each(const double* xi, double* u, F at) {
 #pragma unroll
@@ -371,8 +382,9 @@ __device__ __forceinline__ void interp_each(const double* xi, double* u, F at) {
 // among the cells' projection sums.  Degree-1 hexahedra: DoF by DoF, then cell
 // by cell, so that k_node's neighbouring nodes, which read the same DoF of
 // neighbouring cells, share 128-byte lines; with a cell's sums together each line
-// was fetched by several XCDs for a quarter of it (k_node 31 -> 16 us per step on
-// 202,240, the write the same).  Elsewhere a cell's sums lie together: the
+// was fetched by several XCDs for a quarter of it (202,240 hexahedra: k_node
+// 32 -> 16 us and the write 79 either way in FP32-mixed, 35 -> 18 and 143 -> 146
+// in FP64).  Elsewhere a cell's sums lie together: the
 // scattered stores cost the write more than k_node gains (68,992 degree-2
 // hexahedra: 97 -> 129 and 36 -> 23 us; 407,140 quads: 507 -> 520 and 25 -> 20).
 template <int DIM, int DEG>
@@ -423,14 +435,6 @@ __device__ __forceinline__ void lattice_point(const DevParams& pp, int ordinal, 
     }
 }
 
-// Relocation of a particle whose position left cell c
-// (pfem2ParticleHandler::sort_particles_into_subdomains_and_cells, the part
-// after the own-cell test, cylinder2D/pfem2particle.cpp:278-386).  The
-// reference sorts the star of the selected vertex by decreasing alignment
-// (stable for equal keys) and takes the first cell that contains the point;
-// that is the containing cell with the largest key, earliest star position on
-// ties, which is what the loop below selects.  Returns -1 if no star cell
-// contains the point.
 // Face through which the step from xold to x most likely left the cell: the
 // linearised reference displacement J(xi_old)^-1 (x - xold) added to xi_old,
 // the component furthest outside [0, 1] (face 2a + s is xi_a = s), -1 if
@@ -582,10 +586,18 @@ __device__ __forceinline__ bool contains(const DevMesh<DIM>& m, int c, const dou
     }
 }
 
+// Relocation of a particle whose position left cell c
+// (pfem2ParticleHandler::sort_particles_into_subdomains_and_cells, the part
+// after the own-cell test, cylinder2D/pfem2particle.cpp:278-386).  The
+// reference sorts the star of the selected vertex by decreasing alignment
+// (stable for equal keys) and takes the first cell that contains the point;
+// that is the containing cell with the largest key, earliest star position on
+// ties, which is what the loop below selects.  Returns -1 if no star cell
+// contains the point.
+//
 // `Q` returns the vertices of the cell found.  (A caller's other data of the
 // cell, loaded with each candidate's vertices to overlap the two loads, cost
-// more in registers than it saved: FP64 search 167 -> 147 us, FP32 round 0
-// 77 -> 71 us per step on 101,785 cells without it.)
+// more in registers than it saved: without it the searches took 8-12% less.)
 //
 // OWN and own (2-D): the own-cell test's clearly-outside test said no and the
 // rest of it is pending; only that test runs: c is returned if it places x in
@@ -1072,10 +1084,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIM ==
 // grid has wavefronts, up to RSEGS, so every segment has a wavefront), chunk k
 // to segment k mod nseg: the particles with long crossing chains lie together
 // (around the obstacle), and with one contiguous range a segment its few
-// wavefronts were still searching when the others had left (FP64 search 197 ->
-// 159 us per step on 101,785 cells with 2.4M particles).  The segment's cursor
-// advances by one returning atomic once REFILL_MIN lanes are idle or all are
-// (8 or 32: the same).
+// wavefronts were still searching when the others had left (101,785 quads: FP64
+// search 208 -> 163 us, FP32-mixed 215 -> 153; 202,240 hexahedra, FP32-mixed
+// 145 -> 140).  Where the long chains are few it costs the neighbourhood that
+// consecutive chunks share: 407,140 quads 479 -> 490 in FP64 (FP32-mixed the
+// same), 68,992 degree-2 hexahedra 198 -> 207.  The segment's cursor advances
+// by one returning atomic once REFILL_MIN lanes are idle or all are (8 or 32: the
+// same).
 struct Refill {
     int* cursor;
     int n, seg, nseg;
@@ -1114,8 +1129,9 @@ struct Refill {
 // returning atomic per wavefront and refill, taken once REFILL_MIN lanes are
 // idle or all are), so a wavefront does not wait for its longest crossing
 // chain before it takes new particles, and no particle is parked twice.
-// Every iteration (one search, then the substeps up to the next exit)
-// consumes a substep, so each lane ends, and a wavefront leaves when its
+// Every iteration settles a pending own-cell test or makes one search, then the
+// substeps up to the next exit; a test that says no comes back as a search, and
+// every other iteration consumes a substep, so each lane ends, and a wavefront leaves when its
 // segment is drained and none of its lanes holds a particle.
 template <int DIM, int DEG = 1, bool RESORT = false>
 __device__ __forceinline__ void search_body(const Grid& G, const DevMesh<DIM>& m, const DevParticles& A,
@@ -1160,8 +1176,10 @@ __device__ __forceinline__ void search_body(const Grid& G, const DevMesh<DIM>& m
             // of the test first
             const bool own = DIM == 2 && newton && !clearly_outside<DIM>(P, x, m.ftol[c]);
             newton = false;
-            // (3-D: the face-neighbour shortcut's registers push this kernel
-            // into heavy spilling)
+            // (3-D moves go without the face-neighbour shortcut: it made this
+            // kernel spill heavily before the cells' tables (HexCell).  With
+            // them the two are close: 207 us without, 200 with on 68,992
+            // degree-2 hexahedra, 242 and 238 on 202,240 of degree 1.)
             double Q[NV][DIM], r[DIM];
             const int cn =
                 relocate<DIM, DIM == 2 || RESORT, DIM == 2>(m, c, P, xi, vext, x, r, Q, searches, own);
@@ -1236,10 +1254,9 @@ constexpr int GCAP_L = 128;          // the same for larger lattices
 // the census row of a lattice: GCAP for up to 16 parts, or when the
 // survivors of a full cell (MAX per part) leave 8 of GCAP's entries for
 // arrivals; else GCAP_L.  A cell whose candidates do not fit goes to
-// k_cell_big either way; on the 5x5
-// lattice with MAX 2 of the moving-mesh workload the smaller rows (LDS for 8
-// workgroups per CU instead of 4) take the census from 0.62 to 0.40 ms per
-// step, the listed cells adding ~0.04 ms.
+// k_cell_big either way; on the 5x5 lattice with MAX 2 of 407,140 quads the
+// smaller rows (LDS for 7 workgroups per CU instead of 4, parts as bit masks)
+// take 145 instead of 279 us a census, and their listed cells 15 instead of 5.
 constexpr int SMALL_ROW_SURVIVORS = GCAP - 8;
 __host__ __device__ inline bool census_small_row(int nparts, int max_per_part) {
     return nparts <= 16 || (long long)max_per_part * nparts <= SMALL_ROW_SURVIVORS;
@@ -1712,13 +1729,14 @@ __global__ void __launch_bounds__(256) k_cell_big(const int* __restrict__ old_of
 // through LDS on the way, where LPC lanes per cell add the projection sums in
 // ascending id order (accumulators in registers across the passes, so any
 // number of particles per cell), and no other pass reads them again.
-// Bound by HBM: 64 (80 with velocity_ext) bytes in and out per 2-D FP64
-// particle, 80-90% of a large copy's rate.  It takes the place of a map of the
-// positions, a gather by it, a pass of sums and its own bookkeeping launch:
-// per step 114 -> 86 us (FP64) and 76 -> 47 us (FP32) on 101,785 cells with
-// 2.4M particles, 576 -> 480 and 360 -> 274 on 407,140 with 11M.  One position
-// per thread and pass: two or four, for more loads in flight, cost registers
-// (98-124 us).
+// Bound by HBM: it moves bytes at a large copy's rate.  A 2-D FP64 particle is
+// 64 bytes in and out (80 with velocity_ext); the counters show about half as
+// much again read, for lines of scattered arrivals and slot rows that are used
+// in part.  It takes the place of a map of the positions, a gather by it, a
+// pass of sums and its own bookkeeping launch: 125 -> 92 us (FP64) and 83 -> 50
+// (FP32-mixed) on 101,785 quads, 625 -> 521 and 396 -> 307 on 407,140.  One
+// position per thread and pass: two or four, for more loads in flight, cost
+// registers (14-44% slower).
 //
 // New particles: reference point at the part centre, location mapped,
 // velocity interpolated from V (cylinder2D/pfem2particle.cpp:533-549), ids
@@ -1727,7 +1745,8 @@ template <int DIM, int DEG>
 struct RegroupShape {
     static constexpr int NACC = QF<DIM, DEG>::ND * (DIM + 1);   // sums per cell
     // cells per workgroup: 16 (8 and 32 were 5-10% slower in 2-D), 32 of the
-    // few particles of a hexahedron (78 -> 68 us per FP32 step on 202,240)
+    // few particles of a hexahedron (16: 87 instead of 79 us in FP32-mixed, 161
+    // instead of 146 in FP64 on 202,240)
     static constexpr int CB = DIM == 3 && DEG == 1 ? 32 : 16;
     static constexpr int LPC = 256 / CB;                        // lanes per cell in the sums
     static constexpr int NA = (NACC + LPC - 1) / LPC;           // sums per lane
@@ -1859,8 +1878,8 @@ __device__ __forceinline__ void cell_write_body(const Grid& G, const DevMesh<DIM
     __shared__ RegroupCells<S::CB> s;
     // degree-2 hexahedra: each particle's 1-D factors in LDS, from which a lane
     // multiplies its 7 nodes' shape values; the nodes' coefficients instead took
-    // 168 registers a lane, 2 wavefronts per SIMD (130 -> 98 us per step on
-    // 68,992)
+    // 168 registers a lane, 2 wavefronts per SIMD (with interp_each 151 -> 104 us
+    // on 68,992)
     constexpr bool TAB = SUMS && DIM == 3 && DEG == 2;
     static_assert(!TAB || S::LPC % (DIM + 1) == 0, "a lane's sums are of one component");
     __shared__ double s_xi[SUMS && !TAB ? DIM : 1][SUMS && !TAB ? CH : 1];
@@ -2548,9 +2567,6 @@ __global__ void k_keys(DevParticles A, DevParams pp, DevWork w) {
     }
 }
 
-// per-cell copies of V and V - V_old at the cell's DoFs (one load level in
-// the particle kernels); V - V_old is the same per-node difference the
-// correction forms (TurekBenchmark/pfem2particle.cpp:806-807)
 // prescribed mesh motion: X = X0 + a W
 __global__ void k_displace(const double* __restrict__ X0, const double* __restrict__ W, double a,
                            double* __restrict__ X, long long n) {
@@ -2597,6 +2613,9 @@ __global__ void k_refresh(DevMesh<DIM> m, const double* __restrict__ Vcm, double
     refresh_body<DIM>(hw_grid(), m, Vcm, V, Vold, cellV, cellDV, V32, DV32);
 }
 
+// per-cell copies of V and V - V_old at the cell's DoFs (one load level in
+// the particle kernels); V - V_old is the same per-node difference the
+// correction forms (TurekBenchmark/pfem2particle.cpp:806-807)
 template <int DIM>
 __global__ void k_pack_fields(DevMesh<DIM> m, const double* __restrict__ V, const double* __restrict__ Vold,
                               double* __restrict__ cellV, double* __restrict__ cellDV) {

@@ -92,11 +92,17 @@ int dalloc(T** p, size_t n) {
 // the device end reads or writes the block itself, so a transfer is one launch,
 // one wait and a copy in host memory.  A copy from or to pageable memory costs
 // the runtime's own staging, launch and wait, and a field's download had two
-// (a host-driven step on 4,000 cells 200 -> 149 us, a moving-body step on 25,446
-// 564 -> 510, a batch of 12 with their downloads 2,477 -> 2,046).  A call takes a block and gives it back before it returns (the
-// mutex covers any number of threads; with none free, or past STAGE_BYTES, the
-// pageable copy is made); the blocks, at most STAGE_BLOCKS, are freed with the
-// last handle or server.
+// (a host-driven step on 4,000 cells 188 -> 143 us, a batch of 12 with their
+// downloads 2,460 -> 1,980).  A call takes a block and gives it back before it
+// returns, once its kernel has run (the mutex covers any number of threads; with
+// none free, or past STAGE_BYTES, the pageable copy is made); the blocks, at most
+// STAGE_BLOCKS, are freed with the last handle or server.
+// STAGE_BYTES: up and down through a block and pageable, us, 2-D fields of
+// 4,096 DoFs 19 / 16 and 33 / 44, of 16,384 24 / 24 and 38 / 52, of 65,536 (1 MiB)
+// 62 / 72 and 71 / 101, of 130,321 104 / 117 and 101 / 151, of 1,002,001 598 / 867
+// and 498 / 937: past a MiB an upload no longer gains (the kernel's reads of host
+// memory are slower than the copy engine), and a download gains 7-23%, for which
+// all blocks would have to grow to the largest field's size.
 constexpr size_t STAGE_BYTES = 1 << 20;
 constexpr int STAGE_BLOCKS = 8;
 struct StagePool {
@@ -680,9 +686,12 @@ int run_move(pf2_handle_s* h, int do_correct, int do_move, bool fuse_sums = fals
     DevQueues qu = dev_queues(h);
     // the move: up to 8192 workgroups, about one wavefront-sized chunk per
     // wavefront on the cylinder workload (a smaller grid looping over
-    // several chunks was 1% slower); the search: up to 1024, all the
-    // chip holds at 4 wavefronts per SIMD, whose lanes refill (2048 the same,
-    // 512 20% slower)
+    // several chunks was 1% slower).  The search: up to 1024, all the chip
+    // holds at 4 wavefronts per SIMD (FP32-mixed quads; FP64 quads and FP32-mixed
+    // hexahedra have 3, FP64 hexahedra 2), since lanes refill.  512, 768, 1024,
+    // 2048: 194, 165, 152, 153 us on 101,785 quads FP32-mixed, 195, 166, 163, 167
+    // FP64, 596, 491, 490, 489 on 407,140 FP64, 164, 138, 140, 141 on 202,240
+    // hexahedra FP32-mixed; 68,992 of degree 2 208-210 with any.
     const int grid = grid_for(h->n_est, 256, 8192);
     const int qgrid = grid_for(h->n_est / 2 + 1, 256, SEARCH_GRID);
     if (mixed(h)) {
@@ -1580,8 +1589,8 @@ int pf2_download_particles(pf2_handle h, int* cell, uint32_t* id, double* x, dou
     if (id) HIPC(hipMemcpyAsync(id, b.id, n * 4, hipMemcpyDeviceToHost, h->stream));
     // The rows are formed on the device, in the buffer that the next regroup
     // fills, and copied straight to the caller: the host's own transposition
-    // through a temporary took over half of an output step (11.9 -> 4.3 ms with
-    // 400,000 particles).
+    // through a temporary took over half of an output step (with 400,000
+    // particles it was 2.4 times as long).
     const PBufs& o = h->buf[1 - h->cur];
     double* const srcs[3] = {b.x, b.xi, b.v};
     double* const rows[3] = {o.x, o.xi, o.v};
@@ -2073,7 +2082,7 @@ int pf2_move_mesh_scaled(pf2_handle h, double a) {
 // n doubles of device scratch, kept with the handle from one call to the next
 // (its size is that of a few nodal fields; the calls below end with a
 // synchronisation, so none still uses it).  The allocations and frees of each
-// call, which wait for the device, cost about 70 of the 650 us of a moving-body step on
+// call, which wait for the device, cost about a tenth of a moving-body step on
 // 25,446 cells.
 static double* scratch_for(pf2_handle_s* h, size_t n) {
     if (n > h->scratch_len) {

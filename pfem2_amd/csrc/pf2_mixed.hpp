@@ -593,9 +593,9 @@ __global__ void __launch_bounds__(256) k_move32(DevMesh<DIM> m, const float* __r
 // (pf2_kernels.hpp).  Bound by the latency of its dependent reads and the
 // relocations' FP64 instructions.  It takes the place of a round that parked
 // a particle again and a round that looped the rest to the end, whose
-// wavefronts waited for their longest chain: per step 165 -> 153 us on 101,785
-// quads with 2.4M particles, 459 -> 378 on 407,140 with 11M, 192 -> 138 on
-// 202,240 hexahedra, 35 -> 19 on a channel of 2,000 (one launch less).  4
+// wavefronts waited for their longest chain: 164 -> 153 us on 101,785 quads,
+// 457 -> 383 on 407,140, 190 -> 140 on 202,240 hexahedra, 35 -> 19 on a channel
+// of 2,000 quads (one launch less).  4
 // wavefronts per SIMD in 2-D (3: the same, 5: spills, 5% slower), 3 in 3-D
 // (spills; 2 without: 4% slower).  The face-neighbour shortcut misses more
 // often on later crossings, and without it 101,785 quads take 148 us, but
