@@ -1269,10 +1269,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ int load_agent(const int* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // sum / OR over a 16-lane group, all of whose lanes are active: a row of the
 // data-parallel primitives, rotated by 8, 4, 2, 1 (no LDS permutes)
 template <int N>
